@@ -15,15 +15,19 @@ static hipError_t scenes_ok(const SceneSet* ss, hipStream_t s) {
   }
   return touch(s);
 }
-hipError_t table_clear(const TableView&, Workspace&, hipStream_t s, uint32_t*, int64_t) { return touch(s); }
-hipError_t table_activate(const TableView&, Workspace&, const float*, int64_t, float, int, int, float, hipStream_t s, bool, const SceneSet* ss) { return scenes_ok(ss, s); }
+hipError_t table_clear(const TableView&, Workspace&, hipStream_t s) { return touch(s); }
+hipError_t table_activate(const TableView&, Workspace&, const float*, int64_t, float, int, int, float, hipStream_t s) { return touch(s); }
+hipError_t build_clear(const TableView&, Workspace&, int64_t, hipStream_t s) { return touch(s); }
+hipError_t build_activate(const TableView&, Workspace&, const float*, int64_t, float, hipStream_t s, const SceneSet* ss) { return scenes_ok(ss, s); }
+hipError_t build_enlarge(const TableView&, Workspace&, int64_t, const SortView&, hipStream_t s) { return touch(s); }
+hipError_t build_place(const TableView&, Workspace&, int64_t, const SortView&, hipStream_t s) { return touch(s); }
+size_t rank_scratch_words(uint64_t orders) { return orders / 512 + 64; }
 hipError_t table_enlarge(const TableView&, Workspace&, const int32_t*, const int32_t*, int32_t, hipStream_t s) { return touch(s); }
 hipError_t table_query(const TableView&, const int32_t*, int64_t, int32_t*, hipStream_t s) { return touch(s); }
 hipError_t bucket_sort(const TableView&, Workspace&, const float*, int64_t, float, int, int, float, const SortView&, hipStream_t s) { return touch(s); }
-hipError_t bucket_sort_slots(Workspace&, int64_t, const SortView&, hipStream_t s, bool) { return touch(s); }
 hipError_t block_neighbours(const TableView&, Workspace&, hipStream_t s) { return touch(s); }
 hipError_t check_launch_limits(int) { return hipSuccess; }
-hipError_t grid_clear(float*, const int32_t*, int32_t, hipStream_t s, uint32_t*) { return touch(s); }
+hipError_t grid_clear(float*, const int32_t*, int32_t, hipStream_t s) { return touch(s); }
 hipError_t stress(const Model&, const ParticlesView&, Workspace&, hipStream_t s, const ClosureView* cl, float*, bool, const SceneSet* ss) { return ss && ss->n > 0 && cl ? hipErrorNotSupported : scenes_ok(ss, s); }
 hipError_t stress_closure(const Model&, const ClosureView&, const ParticlesView&, float*, Workspace&, hipStream_t s) { return touch(s); }
 hipError_t mlp_infer(const float*, const float*, int64_t, float*, hipStream_t s) { return touch(s); }

@@ -277,19 +277,14 @@ int32_t reserve(zsmpm_policy_s* p, int64_t n, int32_t T) {
   ZA(w.la_val, w.list_cap);
   ZA(w.lb_key, w.list_cap);
   ZA(w.lb_val, w.list_cap);
-  ZA(w.bkt, w.n_cap);
-  ZA(w.run_start, w.n_cap);
-  ZA(w.rk_a, w.n_cap);
-  ZA(w.rv_a, w.n_cap);
-  ZA(w.rk_b, w.n_cap);
-  ZA(w.rv_b, w.n_cap);
-  ZA(w.run_len, w.n_cap);
-  ZA(w.run_dest, w.n_cap);
-  ZA(w.tile_heads, w.n_cap / 4096 + 2);
-  ZA(w.tile_base, w.n_cap / 4096 + 2);
-  const uint32_t big = w.n_cap > w.ts_cap ? w.n_cap : w.ts_cap;
-  w.rs_words = radix_sort_scratch_words(big);
-  ZA(w.rs_scratch, w.rs_words);
+  ZA(w.seg_heads, w.n_cap / 64 + 2);
+  ZA(w.seg_in, (size_t)w.n_cap + 64);
+  ZA(w.seg_list, w.n_cap);
+  ZA(w.seg_alt, w.n_cap);
+  ZA(w.scnt, w.ts_cap);
+  ZA(w.bcnt, w.ts_cap);
+  ZA(w.bpart, w.ts_cap / 1024 + 2);
+  ZA(w.segoff, w.ts_cap);
   w.scan_words = 16384 + 64;
   ZA(w.scan_tmp, w.scan_words);
   ZA(w.counters, kCtrCount);
@@ -305,11 +300,13 @@ int32_t reserve(zsmpm_policy_s* p, int64_t n, int32_t T) {
     const uint64_t orders = (uint64_t)w.n_cap > 8ull * w.ts_cap ? (uint64_t)w.n_cap : 8ull * w.ts_cap;
     w.bm_words = (uint32_t)(orders / 32 + 2);
   }
-  ZA(w.bitmap, w.bm_words);
+  ZA(w.bitmap, (size_t)w.bm_words + 8);  // read in whole vectors
   ZA(w.bm_prefix, w.bm_words);
-  ZA(w.pslot, w.n_cap);
+  ZA(w.bitmap_b, w.ts_cap / 32 + 10);
+  ZA(w.rank_a, rank_scratch_words(w.n_cap));
+  ZA(w.rank_b, rank_scratch_words(w.ts_cap));
   ZA(w.slot_block, w.ts_cap);
-  ZA(w.dmask, w.ts_cap / 32 + 1);
+  ZA(w.dmask, 2 * (w.ts_cap / 32 + 1));
   p->own_cap_blocks = (int32_t)w.ts_cap;
   ZA(p->own_counts, (size_t)p->own_cap_blocks + 1);
   ZA(p->own_offsets, (size_t)p->own_cap_blocks + 1);
@@ -475,7 +472,7 @@ int32_t ensure_bitmap(zsmpm_policy_s* p, uint64_t orders) {
   if (words > 0xffffffffull) return ZSMPM_INVALID_ARGUMENT;
   ZS_HIP(hipStreamSynchronize(p->stream));
   uint32_t *bm = nullptr, *pre = nullptr;
-  ZS_HIP(alloc(p, &bm, (size_t)words));
+  ZS_HIP(alloc(p, &bm, (size_t)words + 8));
   ZS_HIP(alloc(p, &pre, (size_t)words));
   destroy_graph(p);  // a captured graph holds the old addresses
   ++p->ws_epoch;
@@ -553,7 +550,6 @@ int32_t run_substep(zsmpm_policy_s* pol, const zsmpm_model* model, const zsmpm_p
     CellScope(Workspace& w_, bool on) : w(w_) { w.cell = on; }
     ~CellScope() { w.cell = false; }
   } cell_scope(ws, cell);
-  const int32_t lo[3] = {0, 0, 0}, hi[3] = {2, 2, 2};
   // The stress pass reads F and logJp and writes ws.contrib; the sparsity
   // stages read x only. It runs on the side stream beside them and P2G waits
   // for both.
@@ -567,28 +563,24 @@ int32_t run_substep(zsmpm_policy_s* pol, const zsmpm_model* model, const zsmpm_p
   }
   {
     StageScope sc(pol, ZSMPM_STAGE_TABLE_CLEAR);
-    // the same launch clears the bucket counts the bucket pass adds to
-    ZS_HIP(table_clear(t, ws, s, reinterpret_cast<uint32_t*>(sv.counts), (int64_t)sv.cap_blocks + 1));
+    // also resets the P2G bucket queue and the max |v|^2 counter
+    ZS_HIP(build_clear(t, ws, ps.n, s));
   }
   {
     StageScope sc(pol, ZSMPM_STAGE_ACTIVATE);
-    ZS_HIP(table_activate(t, ws, ps.x, ps.n, dx, 4, -2, 0.5f, s, /*record_slots=*/true, ss));
+    ZS_HIP(build_activate(t, ws, ps.x, ps.n, dx, s, ss));
   }
   {
     StageScope sc(pol, ZSMPM_STAGE_ENLARGE);
-    ZS_HIP(table_enlarge(t, ws, lo, hi, t.T / 8 > 0 ? t.T / 8 : 1, s));
+    ZS_HIP(build_enlarge(t, ws, ps.n, sv, s));
   }
   {
     StageScope sc(pol, ZSMPM_STAGE_BUCKET_SORT);
-    // the activation above recorded every particle's key slot in the table it
-    // just built from empty: the bucket pass reads those instead of x
-    ZS_HIP(bucket_sort_slots(ws, ps.n, sv, s, /*counts_zeroed=*/true));
-    ZS_HIP(block_neighbours(t, ws, s));
+    ZS_HIP(build_place(t, ws, ps.n, sv, s));
   }
   {
     StageScope sc(pol, ZSMPM_STAGE_GRID_CLEAR);
-    // also resets the P2G bucket queue and the max |v|^2 counter
-    ZS_HIP(zsmpm::grid_clear(grid->data, t.cnt, grid->capacity_blocks, s, ws.counters));
+    ZS_HIP(zsmpm::grid_clear(grid->data, t.cnt, grid->capacity_blocks, s));
   }
   ZS_HIP(side.join());
   {
@@ -1352,7 +1344,7 @@ static int32_t run_g2p2g(zsmpm_policy_s* pol, const Model& m, const ParticlesVie
     pf.logJp = lj;
   }
   ZS_HIP(zsmpm::stress(m, pf, pol->ws, s));
-  ZS_HIP(grid_clear(tg, t.cnt, grid->capacity_blocks, s, nullptr));
+  ZS_HIP(grid_clear(tg, t.cnt, grid->capacity_blocks, s));
   ZS_HIP(p2g_force_scatter(ps, t, sv, tg, grid->capacity_blocks, -1.f, grid->dx, pol->ws, s));
   ZS_HIP(implicit_add_force(tg, grid->capacity_blocks, t, r, s));
   return ZSMPM_OK;

@@ -16,9 +16,15 @@
 //     (Shun & Blelloch, "Phase-Concurrent Hash Tables for Determinism",
 //     SPAA 2014), i.e. the layout zpc's seq_exec path produces.
 // The bucket sort is stable by particle index (zpc's seq semantics of
-// SpatiallyCount/SpatiallyDistribute): particles are cut into runs of equal
-// bucket, runs are radix-sorted by bucket (stable) and every particle lands at
-// its run's destination plus its offset in the run.
+// SpatiallyCount/SpatiallyDistribute): a wave cuts its 64 particles into
+// segments of equal key; every segment takes a place in its bucket's list with
+// the one atomic that also counts it, and a workgroup per bucket orders the
+// list by first particle and writes the bucket's indices. No sort over the
+// whole set: the counts give the buckets, and a list has ~8 entries when the
+// particles are in bucket order (a few hundred when they are shuffled).
+// The substep's own build (build_begin .. build_place) numbers, places and
+// enlarges from one dedup hash and one clear, with no device-wide scan: 9
+// launches where the stage-by-stage operators take about 35.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -30,8 +36,6 @@ namespace zsmpm {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kTileItems = 16;
-constexpr int kTile = kThreads * kTileItems;  // 4096 particles per bucket-sort tile
 
 inline int groups_for(int64_t n, int threads) {
   int64_t g = (n + threads - 1) / threads;
@@ -42,10 +46,9 @@ inline int groups_for(int64_t n, int threads) {
 
 // --------------------------------------------------------------- clearing
 __global__ void clear_table_kernel(TableView t, uint64_t* skey, uint32_t* sorder, uint32_t* dmask, uint32_t ts,
-                                   uint32_t* counters, uint32_t* zero, int64_t nzero) {
+                                   uint32_t* counters) {
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < (int64_t)((ts + 31u) >> 5); e += stride) dmask[e] = 0u;
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < nzero; e += stride) zero[e] = 0u;
   for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < t.T; e += stride) {
     t.keys[3 * e] = kKeySentinel;
     t.keys[3 * e + 1] = kKeySentinel;
@@ -64,15 +67,13 @@ __global__ void clear_table_kernel(TableView t, uint64_t* skey, uint32_t* sorder
 }
 
 __global__ void clear_scratch_kernel(uint64_t* skey, uint32_t* sorder, uint32_t* dmask, uint32_t ts,
-                                     const int32_t* cnt, uint32_t* counters, int32_t* slot_block,
-                                     uint32_t* bitmap, int64_t bm_n) {
+                                     const int32_t* cnt, uint32_t* counters, uint32_t* bitmap, int64_t bm_n) {
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < (int64_t)((ts + 31u) >> 5); e += stride) dmask[e] = 0u;
   for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < bm_n; e += stride) bitmap[e] = 0u;
   for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < ts; e += stride) {
     skey[e] = kEmpty64;
     sorder[e] = 0xffffffffu;
-    if (slot_block) slot_block[e] = -1;
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     counters[kCtrList] = 0;
@@ -96,52 +97,78 @@ struct Dedup {
 
 __device__ __forceinline__ uint32_t dedup_home(uint64_t pk, uint32_t ts) { return (uint32_t)mix64(pk) & (ts - 1u); }
 
-// Finishes an insert whose probe at slot s returned prev: probes on until the
-// slot is free or holds pk (ts probes in all), then lowers the slot's order;
-// the insert that claims a free slot marks it. Returns the slot holding pk, or
-// ~0u when the scratch table is full.
-__device__ __forceinline__ uint32_t dedup_finish(uint64_t pk, uint32_t order, uint32_t s, uint64_t prev,
-                                                 const Dedup& d) {
-  for (uint32_t probe = 1; prev != kEmpty64 && prev != pk; ++probe) {
+// Finishes an insert whose look at slot s showed cur: probes on until the slot
+// is free or holds pk (ts probes in all), then lowers the slot's order; the
+// insert that claims a free slot marks it in `mask`. Returns the slot holding
+// pk, or ~0u when the scratch table is full. Plain loads come before the
+// atomics: keys are only ever added and orders only lowered, so a stale value
+// costs an atomic that was not needed and nothing else.
+__device__ __forceinline__ uint32_t dedup_finish(uint64_t pk, uint32_t order, uint32_t s, uint64_t cur,
+                                                 const Dedup& d, uint32_t* mask) {
+  for (uint32_t probe = 1;; ++probe) {
+    if (cur == pk) break;
+    if (cur == kEmpty64) {
+      cur = atomicCAS((unsigned long long*)&d.skey[s], (unsigned long long)kEmpty64, (unsigned long long)pk);
+      if (cur == kEmpty64) {
+        atomicOr(&mask[s >> 5], 1u << (s & 31u));
+        break;
+      }
+      if (cur == pk) break;
+    }
     if (probe >= d.ts) {
       atomicOr(d.err, kErrTableFull);
       return ~0u;
     }
     s = (s + 1u) & (d.ts - 1u);
-    prev = atomicCAS((unsigned long long*)&d.skey[s], (unsigned long long)kEmpty64, (unsigned long long)pk);
+    cur = d.skey[s];
   }
-  atomicMin(&d.sorder[s], order);
-  if (prev == kEmpty64) atomicOr(&d.dmask[s >> 5], 1u << (s & 31u));
+  if (d.sorder[s] > order) atomicMin(&d.sorder[s], order);
   return s;
 }
 
 __device__ __forceinline__ uint32_t dedup_insert(uint64_t pk, uint32_t order, const Dedup& d) {
   const uint32_t s = dedup_home(pk, d.ts);
-  const uint64_t prev =
-      atomicCAS((unsigned long long*)&d.skey[s], (unsigned long long)kEmpty64, (unsigned long long)pk);
-  return dedup_finish(pk, order, s, prev, d);
+  return dedup_finish(pk, order, s, d.skey[s], d, d.dmask);
 }
 
-constexpr int kActItems = 4;  // 64-particle groups per wave, their loads and first probes issued together
+// The segments of a 64-particle group: bit l of heads is set where particle l
+// starts a segment (another key than particle l - 1's, or l = 0). Length of
+// the segment that starts at `lane`, cw particles in the group.
+__device__ __forceinline__ int segment_length(uint64_t heads, int lane, int cw) {
+  const uint64_t above = lane == 63 ? 0ull : heads >> (lane + 1);
+  const int next = above ? lane + __ffsll((long long)above) : cw;
+  return next - lane;
+}
 
-// ComputeSparsity candidates: one per particle, order = particle index. Each
-// distinct key of a 64-particle group is inserted once, by its lowest lane
-// (the smallest particle index holding it), so hot keys see one atomic per
-// group. A wave takes kActItems groups and issues their x loads, then their
-// first probes, together: the kernel is bound by those round trips, not by
-// bytes. The dedup hash keeps the minimum order per key, so the result does
-// not depend on the order of the inserts. With pslot, every particle's
-// scratch slot (the identity of its key) is recorded for the bucket sort.
+// Per group, its heads; per segment (the j-th of group g at 64 g + j), the
+// bucket it belongs to (a dedup slot or a block) and its place in that
+// bucket's list, from the atomic that counted it: `place` holds segments << 32
+// | particles per bucket.
+struct Segments {
+  uint64_t* heads = nullptr;  // [groups]
+  uint2* in = nullptr;        // [64 groups]
+  uint64_t* place = nullptr;
+};
+
+// ComputeSparsity candidates: one per segment of a 64-particle group, by its
+// first particle (order = particle index). A wave takes kItems groups and
+// issues their x loads, then their first probes, together: the kernel is bound
+// by those round trips, not by bytes (one group per wave below 2^22 particles,
+// where waves are scarce). The dedup hash keeps the minimum order per key, so
+// the result does not depend on the order of the inserts. Inserting one lane
+// per segment, not per distinct key of the group, needs no loop over the
+// group's keys: 1M shuffled particles 143 -> 33 us, 16M in bucket order (where
+// the two are the same) 88 us either way. kSegs: the segments are
+// recorded for the bucket sort.
 // kMulti (a batch, ss): particle p takes its scene's 1/dx, and its key is
 // shifted by the scene's offset (a key outside the scene's own range
 // [-512, 511) along axis 0 is a key-range error)
-template <bool kMulti>
+template <bool kMulti, bool kSegs, int kItems>
 __global__ __launch_bounds__(kThreads) void activate_kernel(const float* __restrict__ x, int64_t n,
                                                             float dxinv, int blockLen, int offset,
-                                                            float disp, Dedup dd, uint32_t* pslot,
-                                                            SceneSet ss) {
+                                                            float disp, Dedup dd, Segments sg, SceneSet ss) {
   uint32_t* err = dd.err;
-  const int64_t span = (int64_t)kThreads * kActItems;
+  const int64_t span = (int64_t)kThreads * kItems;
   const int64_t stride = (int64_t)gridDim.x * span;
   const int lane = lane_id();
   __shared__ int64_t sfirst[kMulti ? kMaxScenes + 1 : 1];
@@ -150,9 +177,9 @@ __global__ __launch_bounds__(kThreads) void activate_kernel(const float* __restr
     __syncthreads();
   }
   for (int64_t base = (int64_t)blockIdx.x * span; base < n; base += stride) {
-    float cx[kActItems], cy[kActItems], cz[kActItems];
+    float cx[kItems], cy[kItems], cz[kItems];
 #pragma unroll
-    for (int r = 0; r < kActItems; ++r) {
+    for (int r = 0; r < kItems; ++r) {
       const int64_t p = base + (int64_t)r * kThreads + threadIdx.x;
       cx[r] = cy[r] = cz[r] = 0.f;
       if (p < n) {
@@ -161,11 +188,10 @@ __global__ __launch_bounds__(kThreads) void activate_kernel(const float* __restr
         cz[r] = x[3 * p + 2];
       }
     }
-    uint64_t pk[kActItems];
-    int leader[kActItems];
-    bool head[kActItems];
+    uint64_t pk[kItems], cur[kItems], heads[kItems];
+    uint32_t slot[kItems];
 #pragma unroll
-    for (int r = 0; r < kActItems; ++r) {
+    for (int r = 0; r < kItems; ++r) {
       const int64_t p = base + (int64_t)r * kThreads + threadIdx.x;
       pk[r] = kEmpty64;
       if (p < n) {
@@ -186,44 +212,40 @@ __global__ __launch_bounds__(kThreads) void activate_kernel(const float* __restr
           atomicOr(err, kErrKeyRange);
         }
       }
-      // peel off one distinct key per iteration: the lowest pending lane leads
-      bool pending = pk[r] != kEmpty64;
-      bool h = false;
-      int my_leader = lane;
-      for (uint64_t m = ballot(pending); m != 0; m = ballot(pending)) {
-        const int ld = __ffsll((long long)m) - 1;
-        const uint64_t lk = shfl(pk[r], ld);
-        const bool same = pending && pk[r] == lk;
-        my_leader = same ? ld : my_leader;
-        h = h || lane == ld;
-        pending = pending && !same;
-      }
-      head[r] = h;
-      leader[r] = my_leader;
-    }
-    uint32_t slot[kActItems];
-    uint64_t prev[kActItems];
-#pragma unroll
-    for (int r = 0; r < kActItems; ++r) {
+      const uint64_t left = __shfl_up(pk[r], 1, kWave);
+      const bool head = p < n && (lane == 0 || left != pk[r]);
+      heads[r] = ballot(head);
       slot[r] = ~0u;
-      prev[r] = kEmpty64;
-      if (head[r]) {
+      cur[r] = kEmpty64;
+      if (head && pk[r] != kEmpty64) {
         slot[r] = dedup_home(pk[r], dd.ts);
-        prev[r] = atomicCAS((unsigned long long*)&dd.skey[slot[r]], (unsigned long long)kEmpty64,
-                            (unsigned long long)pk[r]);
+        cur[r] = dd.skey[slot[r]];
       }
     }
 #pragma unroll
-    for (int r = 0; r < kActItems; ++r) {
+    for (int r = 0; r < kItems; ++r) {
       const int64_t p = base + (int64_t)r * kThreads + threadIdx.x;
-      if (head[r]) slot[r] = dedup_finish(pk[r], (uint32_t)p, slot[r], prev[r], dd);
+      if (slot[r] != ~0u) slot[r] = dedup_finish(pk[r], (uint32_t)p, slot[r], cur[r], dd, dd.dmask);
     }
-    if (pslot) {
+    if constexpr (kSegs) {
+      uint32_t local[kItems];
 #pragma unroll
-      for (int r = 0; r < kActItems; ++r) {
-        const int64_t p = base + (int64_t)r * kThreads + threadIdx.x;
-        const uint32_t ls = (uint32_t)__shfl((int)slot[r], leader[r], kWave);
-        if (p < n) pslot[p] = pk[r] != kEmpty64 ? ls : ~0u;
+      for (int r = 0; r < kItems; ++r) {
+        const int64_t g64 = base + (int64_t)r * kThreads + threadIdx.x - lane;  // the group's first particle
+        const int cw = (int)min((int64_t)kWave, n - g64);
+        local[r] = 0;
+        if (slot[r] != ~0u)
+          local[r] = (uint32_t)(atomicAdd((unsigned long long*)&sg.place[slot[r]],
+                                          (1ull << 32) | (unsigned long long)segment_length(heads[r], lane, cw)) >>
+                                32);
+      }
+#pragma unroll
+      for (int r = 0; r < kItems; ++r) {
+        const int64_t g64 = base + (int64_t)r * kThreads + threadIdx.x - lane;
+        if (g64 >= n) continue;
+        if (lane == 0) sg.heads[g64 >> 6] = heads[r];
+        if ((heads[r] >> lane) & 1ull)
+          sg.in[g64 + __popcll(heads[r] & lanemask_lt())] = make_uint2(slot[r], local[r]);
       }
     }
   }
@@ -338,6 +360,31 @@ __global__ __launch_bounds__(kThreads) void collect_new_kernel(const uint64_t* _
     list_put(gbase + i, bkey[i], bval[i], lkey, lval, list_cap, err);
 }
 
+// block `rank` with the key k into zpc's table by priority linear probing on
+// indices[] (the lower block number wins a slot)
+__device__ __forceinline__ void place_block(const TableView& t, uint32_t rank, int32_t k0, int32_t k1, int32_t k2,
+                                            uint32_t* err) {
+  t.active[3 * (int64_t)rank] = k0;
+  t.active[3 * (int64_t)rank + 1] = k1;
+  t.active[3 * (int64_t)rank + 2] = k2;
+  // carried element: starts as this key; a displaced lower-priority entry
+  // continues from the slot after the one it lost
+  uint32_t cur = rank;
+  int32_t s = zpc_home(k0, k1, k2, t.T);
+  int64_t steps = 0;
+  const int64_t limit = 2ll * t.T + 64;
+  while (true) {
+    const uint32_t old = atomicMin((uint32_t*)&t.indices[s], cur);
+    if (old == 0xffffffffu) break;
+    if (old > cur) cur = old;
+    s = probe_next(s, t.T);
+    if (++steps > limit) {
+      atomicOr(err, kErrTableFull);
+      break;
+    }
+  }
+}
+
 // Number the new keys cnt0 + rank, record _activeKeys and place them by
 // priority linear probing on indices[] (lower block number wins a slot).
 __global__ __launch_bounds__(kThreads) void assign_kernel(const uint32_t* __restrict__ lorder,
@@ -346,7 +393,7 @@ __global__ __launch_bounds__(kThreads) void assign_kernel(const uint32_t* __rest
                                                           const uint32_t* __restrict__ bm_prefix, uint32_t bm_words,
                                                           const uint64_t* __restrict__ skey,
                                                           TableView t, const uint32_t* counters,
-                                                          uint32_t list_cap, uint32_t* err, int32_t* slot_block) {
+                                                          uint32_t list_cap, uint32_t* err) {
   const uint32_t nl = min(counters[kCtrList], list_cap);
   const uint32_t cnt0 = counters[kCtrCnt0];
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -367,26 +414,7 @@ __global__ __launch_bounds__(kThreads) void assign_kernel(const uint32_t* __rest
       atomicOr(err, kErrTableFull);
       continue;
     }
-    if (slot_block) slot_block[sl] = (int32_t)rank;  // the block number of the key in scratch slot sl
-    t.active[3 * (int64_t)rank] = k0;
-    t.active[3 * (int64_t)rank + 1] = k1;
-    t.active[3 * (int64_t)rank + 2] = k2;
-    // carried element: starts as this key; a displaced lower-priority entry
-    // continues from the slot after the one it lost
-    uint32_t cur = rank;
-    int32_t s = zpc_home(k0, k1, k2, t.T);
-    int64_t steps = 0;
-    const int64_t limit = 2ll * t.T + 64;
-    while (true) {
-      const uint32_t old = atomicMin((uint32_t*)&t.indices[s], cur);
-      if (old == 0xffffffffu) break;
-      if (old > cur) cur = old;
-      s = probe_next(s, t.T);
-      if (++steps > limit) {
-        atomicOr(err, kErrTableFull);
-        break;
-      }
-    }
+    place_block(t, rank, k0, k1, k2, err);
   }
 }
 
@@ -428,275 +456,565 @@ __global__ void query_kernel(TableView t, const int32_t* __restrict__ keys, int6
     out[i] = table_find(t, keys[3 * i], keys[3 * i + 1], keys[3 * i + 2]);
 }
 
+// ------------------------------------------------------- the substep's build
+// Ranks among set bits of a bitmap of orders without a scan: counts of the set
+// bits per 2^10, 2^17 and 2^24 orders (c1, c2, c3), added to as the bits are
+// set. rank(o) = c3 before o's 2^24 group + c2 before its 2^17 group in that +
+// c1 before its 2^10 group in that + the bits before it there: at most 32
+// words and 3 x 128 counts, read by 8 lanes per key.
+struct Ranks {
+  uint32_t* bitmap = nullptr;
+  uint32_t* c1 = nullptr;
+  uint32_t* c2 = nullptr;
+  uint32_t* c3 = nullptr;
+  uint32_t words = 0;  // of the bitmap
+};
+constexpr int kR1 = 10, kR2 = 17, kR3 = 24;
+// entries of a count level, a whole number of vectors past the last one
+inline uint64_t rank_pad(uint64_t last) { return (last + 1 + 7) & ~(uint64_t)3; }
+
+// h3: the workgroup's own counts per 2^24 orders (a few addresses for the whole
+// launch: 36K atomics on one took 0.4 ms)
+__device__ __forceinline__ void rank_mark(const Ranks& r, uint32_t o, uint32_t* h3) {
+  if ((o >> 5) >= r.words) return;  // reported where the rank is taken
+  atomicOr(&r.bitmap[o >> 5], 1u << (o & 31u));
+  atomicAdd(&r.c1[o >> kR1], 1u);
+  atomicAdd(&r.c2[o >> kR2], 1u);
+  if (r.words > (1u << (kR3 - 5)) + 1u) atomicAdd(&h3[o >> kR3], 1u);
+}
+
+__device__ __forceinline__ uint32_t sum_range(const uint32_t* __restrict__ a, uint32_t lo, uint32_t hi, int j) {
+  // this lane's share (every 8th group of 4) of a[lo, hi), lo a multiple of 4
+  uint32_t s = 0;
+  for (uint32_t i = lo + 4 * j; i < hi; i += 32) {
+    const uint4 q = *reinterpret_cast<const uint4*>(a + i);  // the arrays are padded to whole vectors
+    s += q.x + (i + 1 < hi ? q.y : 0u) + (i + 2 < hi ? q.z : 0u) + (i + 3 < hi ? q.w : 0u);
+  }
+  return s;
+}
+
+// set bits before order o; called by the 8 lanes of a key's group (j = lane & 7)
+__device__ __forceinline__ uint32_t rank_below(const Ranks& r, uint32_t o, int j) {
+  uint32_t s = 0;
+  const uint32_t w0 = (o >> kR1) << (kR1 - 5), w1 = o >> 5;
+  const uint32_t i = w0 + 4 * j;
+  if (i <= w1) {
+    const uint4 q = *reinterpret_cast<const uint4*>(r.bitmap + i);
+    const uint32_t v[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const uint32_t w = i + k;
+      s += (uint32_t)__popc(w < w1 ? v[k] : (w == w1 ? v[k] & ((1u << (o & 31u)) - 1u) : 0u));
+    }
+  }
+  s += sum_range(r.c1, (o >> kR2) << (kR2 - kR1), o >> kR1, j);
+  s += sum_range(r.c2, (o >> kR3) << (kR3 - kR2), o >> kR2, j);
+  s += sum_range(r.c3, 0, o >> kR3, j);
+#pragma unroll
+  for (int d = 1; d < 8; d <<= 1) s += __shfl_xor(s, d, kWave);
+  return s;
+}
+
+// Everything the build reads before it writes it, in one launch.
+struct ClearList {
+  static constexpr int kMax = 12;
+  uint32_t* p[kMax];
+  int64_t n[kMax];
+  uint32_t v[kMax];
+  int count = 0;
+};
+
+__global__ __launch_bounds__(kThreads) void build_clear_kernel(ClearList c, TableView t, uint32_t* counters) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  const int64_t i0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  for (int k = 0; k < c.count; ++k) {
+    const uint32_t v = c.v[k];
+    uint32_t* p = c.p[k];
+    const int64_t n = c.n[k];
+    const int64_t mis = min(n, (int64_t)((4 - ((uintptr_t)p >> 2)) & 3));  // words before a 16-byte boundary
+    const int64_t nv = (n - mis) / 4;
+    for (int64_t i = i0; i < nv; i += stride) reinterpret_cast<uint4*>(p + mis)[i] = make_uint4(v, v, v, v);
+    if (i0 < mis) p[i0] = v;
+    if (i0 < n - mis - 4 * nv) p[mis + 4 * nv + i0] = v;
+  }
+  if (i0 == 0) {
+    *t.cnt = 0;
+    counters[kCtrList] = 0u;
+    counters[kCtrListB] = 0u;
+    counters[kCtrQueue] = 0u;
+    counters[kCtrMaxVel] = 0u;
+  }
+}
+
+// The slots a pass claimed (set bits of mask) as a list of (order, slot), their
+// orders marked for ranking. A workgroup takes 64 mask words, lists their slots
+// in LDS and reserves room with one atomic; the list's order is irrelevant.
+__global__ __launch_bounds__(kThreads) void build_collect_kernel(const uint32_t* __restrict__ mask, uint32_t nw,
+                                                                 const uint32_t* __restrict__ sorder, Ranks rk,
+                                                                 uint32_t* count, uint32_t* __restrict__ lorder,
+                                                                 uint32_t* __restrict__ lslot) {
+  __shared__ uint32_t buf[kWave * 32];
+  __shared__ uint32_t total, base, h3[1u << (32 - kR3)];
+  for (uint32_t i = threadIdx.x; i < (1u << (32 - kR3)); i += kThreads) h3[i] = 0u;
+  const uint32_t w = blockIdx.x * kWave + threadIdx.x;
+  if (threadIdx.x < kWave) {
+    uint32_t bits = w < nw ? mask[w] : 0u;
+    const uint32_t c = (uint32_t)__popc(bits);
+    uint32_t inc = c;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const uint32_t u = __shfl_up(inc, o, kWave);
+      if (lane_id() >= o) inc += u;
+    }
+    uint32_t at = inc - c;
+    while (bits) {
+      buf[at++] = w * 32u + (uint32_t)(__ffs(bits) - 1);
+      bits &= bits - 1u;
+    }
+    if (threadIdx.x == kWave - 1) {
+      total = inc;
+      base = inc ? atomicAdd(count, inc) : 0u;
+    }
+  }
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < total; i += kThreads) {
+    const uint32_t s = buf[i], o = sorder[s];
+    rank_mark(rk, o, h3);
+    lorder[base + i] = o;
+    lslot[base + i] = s;
+  }
+  if (rk.words > (1u << (kR3 - 5)) + 1u) {
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < (1u << (32 - kR3)); i += kThreads)
+      if (h3[i]) atomicAdd(&rk.c3[i], h3[i]);
+  }
+}
+
+// Numbers the listed keys first + rank and places them, 8 lanes per key.
+// kEnlarge (the particles' keys, first = 0): lane j also inserts the key's
+// j-th neighbour key + (j>>2, j>>1&1, j&1) -- EnlargeSparsity's loop order --
+// with order 8 b + j, and records its slot in nbr[8 b + j]: the 2^3 blocks the
+// bucket's stencils cover need no table probe later. bcnt receives the
+// bucket's segment and particle counts, part their sums per 1,024 blocks.
+template <bool kEnlarge>
+__global__ __launch_bounds__(kThreads) void build_number_kernel(const uint32_t* count, const uint32_t* first_count,
+                                                                const uint32_t* __restrict__ lorder,
+                                                                const uint32_t* __restrict__ lslot, Ranks rk,
+                                                                TableView t, Dedup dd, uint32_t* mask2,
+                                                                int32_t* slot_block, const uint64_t* scnt,
+                                                                uint64_t* bcnt, uint64_t* part, int32_t* nbr) {
+  const uint32_t nl = *count;
+  const uint32_t first = kEnlarge ? 0u : *first_count;
+  const int j = lane_id() & 7;
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i8 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i8 < 8ll * nl; i8 += stride) {
+    const uint32_t o = lorder[i8 >> 3], sl = lslot[i8 >> 3];
+    if ((o >> 5) >= rk.words) {
+      if (j == 0) atomicOr(dd.err, kErrCapacity);
+      continue;
+    }
+    const uint32_t rank = first + rank_below(rk, o, j);
+    if (rank >= (uint32_t)t.T) {
+      if (j == 0) atomicOr(dd.err, kErrTableFull);
+      continue;
+    }
+    int32_t k0, k1, k2;
+    unpack_key(dd.skey[sl], k0, k1, k2);
+    if (j == 0) {
+      slot_block[sl] = (int32_t)rank;
+      if (kEnlarge) {
+        const uint64_t c = scnt[sl];
+        bcnt[rank] = c;
+        atomicAdd((unsigned long long*)&part[rank >> 10], (unsigned long long)c);
+        nbr[8 * (int64_t)rank] = (int32_t)sl;
+      }
+      place_block(t, rank, k0, k1, k2, dd.err);
+    } else if (kEnlarge) {
+      k0 += (j >> 2) & 1;
+      k1 += (j >> 1) & 1;
+      k2 += j & 1;
+      int32_t r = -1;
+      if (!key_packable(k0, k1, k2)) {
+        atomicOr(dd.err, kErrKeyRange);
+      } else {
+        const uint64_t pk = pack_key(k0, k1, k2);
+        const uint32_t s = dedup_home(pk, dd.ts);
+        r = (int32_t)dedup_finish(pk, 8u * rank + (uint32_t)j, s, dd.skey[s], dd, mask2);
+      }
+      nbr[8 * (int64_t)rank + j] = r;
+    }
+  }
+}
+
+// Bucket counts and offsets of every block (zero past the particles' blocks)
+// and the start of each bucket's segment list, from the counts per block and
+// their sums per 1,024: a workgroup adds up the sums before its blocks and
+// scans its own. bcnt, part: segments << 32 | particles.
+__device__ __forceinline__ void counts_scan(const uint64_t* __restrict__ bcnt, const uint64_t* __restrict__ part,
+                                            int32_t nb, const SortView& sv, uint32_t* __restrict__ segoff,
+                                            uint32_t* counters, uint64_t* lds) {
+  const int lane = lane_id(), wave = threadIdx.x / kWave;
+  const int64_t nchunk = ((int64_t)sv.cap_blocks + 1 + 1023) / 1024;
+  const int32_t nparts = (nb + 1023) / 1024;
+  for (int64_t c = blockIdx.x; c < nchunk; c += gridDim.x) {
+    uint64_t before = 0;
+    for (int32_t i = threadIdx.x; i < nparts && i < c; i += kThreads) before += part[i];
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) before += __shfl_xor(before, o, kWave);
+    uint64_t v[4], mine = 0;
+    const int64_t b0 = c * 1024 + (int64_t)threadIdx.x * 4;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      v[k] = b0 + k < nb ? bcnt[b0 + k] : 0ull;
+      mine += v[k];
+    }
+    uint64_t inc = mine;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const uint64_t u = __shfl_up(inc, o, kWave);
+      if (lane >= o) inc += u;
+    }
+    if (lane == kWave - 1) lds[wave] = inc;
+    if (lane == 0) lds[kThreads / kWave + wave] = before;
+    __syncthreads();
+    uint64_t run = inc - mine;
+#pragma unroll
+    for (int w = 0; w < kThreads / kWave; ++w) {
+      run += w < wave ? lds[w] : 0ull;
+      run += lds[kThreads / kWave + w];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (b0 + k <= sv.cap_blocks) {
+        // the last entry past the buckets counts nothing
+        sv.counts[b0 + k] = b0 + k < sv.cap_blocks ? (int32_t)(uint32_t)v[k] : 0;
+        sv.offsets[b0 + k] = (int32_t)(uint32_t)run;
+        if (b0 + k < nb) segoff[b0 + k] = (uint32_t)(run >> 32);
+        if (b0 + k == sv.cap_blocks) counters[kCtrRuns] = (uint32_t)(run >> 32);
+      }
+      run += v[k];
+    }
+    __syncthreads();
+  }
+}
+
+// The last of the build's bookkeeping: the keys[] of every placed block (block
+// r probes from its home until it finds the slot holding r), the block count,
+// the neighbours' block numbers in place of their slots, the bucket offsets.
+__global__ __launch_bounds__(kThreads) void build_finish_kernel(TableView t, uint32_t* counters, uint32_t* err,
+                                                                const int32_t* __restrict__ slot_block, uint32_t ts,
+                                                                int32_t* nbr, const uint64_t* __restrict__ bcnt,
+                                                                const uint64_t* __restrict__ part, SortView sv,
+                                                                uint32_t* segoff) {
+  __shared__ uint64_t lds[2 * (kThreads / kWave)];
+  const int64_t na = min((int64_t)counters[kCtrList], (int64_t)t.T);
+  const int64_t nb = min((int64_t)counters[kCtrList] + counters[kCtrListB], (int64_t)t.T);
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  const int64_t i0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i0 == 0) {  // nothing in this kernel reads the count
+    *t.cnt = (int32_t)nb;
+    if (na > sv.cap_blocks) atomicOr(err, kErrCapacity);
+  }
+  for (int64_t r = i0; r < nb; r += stride) {
+    const int32_t k0 = t.active[3 * r], k1 = t.active[3 * r + 1], k2 = t.active[3 * r + 2];
+    int32_t s = zpc_home(k0, k1, k2, t.T);
+    int32_t probe = 0;
+    for (; probe < t.T; ++probe) {
+      if (t.indices[s] == (int32_t)r) break;
+      s = probe_next(s, t.T);
+    }
+    if (probe == t.T) {
+      atomicOr(err, kErrTableFull);
+      continue;
+    }
+    t.keys[3 * (int64_t)s] = k0;
+    t.keys[3 * (int64_t)s + 1] = k1;
+    t.keys[3 * (int64_t)s + 2] = k2;
+  }
+  for (int64_t i = i0; i < 8 * na; i += stride) {
+    const uint32_t sl = (uint32_t)nbr[i];
+    nbr[i] = sl < ts ? slot_block[sl] : -1;
+  }
+  counts_scan(bcnt, part, (int32_t)min(na, (int64_t)sv.cap_blocks), sv, segoff, counters, lds);
+}
+
 // ------------------------------------------------------------ bucket sort
 __global__ void zero_u32_kernel(uint32_t* p, int64_t n) {
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += stride) p[i] = 0u;
 }
 
-constexpr uint32_t kHeadBit = 0x80000000u;  // bkt[p] bit 31: p starts a run
-
-// Bucket of every particle (the block number its key maps to), per-bucket
-// counts, run heads and the number of run heads per tile. A run head is a
-// particle whose key differs from the previous particle's; bkt[p] carries the
-// head flag in bit 31 so every later pass sees the same runs. Lanes query the
-// table only at run heads (and lane 0), the rest take the head's bucket.
-// Particles of a tile are visited in order: round r, thread t -> tile*kTile +
-// r*kThreads + t.
+// The stand-alone bucket sort's segments: the block each one's key maps to,
+// from one table query per segment, counted per block.
 __global__ __launch_bounds__(kThreads) void bucket_kernel(const float* __restrict__ x, int64_t n, float dxinv,
                                                           int blockLen, int offset, float disp, TableView t,
-                                                          uint32_t* __restrict__ bkt, uint32_t* counts,
-                                                          int32_t cap_blocks, uint32_t* __restrict__ tile_heads,
-                                                          uint32_t* err) {
-  __shared__ uint32_t wsum[kThreads / kWave];
-  const int64_t ntiles = (n + kTile - 1) / kTile;
+                                                          Segments sg, int32_t cap_blocks, uint32_t* err) {
   const int lane = lane_id();
-  for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    uint32_t heads = 0;
-    for (int r = 0; r < kTileItems; ++r) {
-      const int64_t p = tile * kTile + (int64_t)r * kThreads + threadIdx.x;
-      const bool valid = p < n;
-      int32_t k0 = 0, k1 = 0, k2 = 0;
-      if (valid) block_key(x[3 * p], x[3 * p + 1], x[3 * p + 2], dxinv, blockLen, offset, disp, k0, k1, k2);
-      int32_t q0 = __shfl_up(k0, 1, kWave), q1 = __shfl_up(k1, 1, kWave), q2 = __shfl_up(k2, 1, kWave);
-      if (lane == 0 && valid && p > 0)
-        block_key(x[3 * (p - 1)], x[3 * (p - 1) + 1], x[3 * (p - 1) + 2], dxinv, blockLen, offset, disp, q0,
-                  q1, q2);
-      const bool head = valid && (p == 0 || q0 != k0 || q1 != k1 || q2 != k2);
-      const bool lookup = valid && (head || lane == 0);
-      int32_t b = -1;
-      if (lookup) {
-        b = table_find(t, k0, k1, k2);
-        if (b < 0) atomicOr(err, kErrMissingBlock);
-        if (b >= cap_blocks) {
-          atomicOr(err, kErrCapacity);
-          b = -1;
-        }
-      }
-      const uint64_t lm = ballot(lookup);
-      const uint64_t le = lanemask_lt() | (1ull << lane);
-      const int src = 63 - __clzll(lm & le);
-      b = shfl(b, src < 0 ? 0 : src);
-      if (valid) bkt[p] = (uint32_t)(b < 0 ? 0 : b) | (head ? kHeadBit : 0u);
-      heads += head ? 1u : 0u;
-      // per-bucket counts: one atomic per (lookup segment) in the wave
-      const uint64_t vm = ballot(valid);
-      if (lookup && b >= 0) {
-        const uint64_t above = lm & ~le;
-        const int next = above ? (__ffsll((long long)above) - 1) : 64;
-        const uint64_t seg = (next >= 64 ? ~0ull : ((1ull << next) - 1ull)) & ~((1ull << lane) - 1ull);
-        atomicAdd(&counts[b], (uint32_t)__popcll(seg & vm));
-      }
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < n; base += stride) {
+    const int64_t p = base + threadIdx.x;
+    const bool valid = p < n;
+    int32_t k0 = 0, k1 = 0, k2 = 0;
+    if (valid) block_key(x[3 * p], x[3 * p + 1], x[3 * p + 2], dxinv, blockLen, offset, disp, k0, k1, k2);
+    const int32_t q0 = __shfl_up(k0, 1, kWave), q1 = __shfl_up(k1, 1, kWave), q2 = __shfl_up(k2, 1, kWave);
+    const bool head = valid && (lane == 0 || q0 != k0 || q1 != k1 || q2 != k2);
+    const uint64_t heads = ballot(head);
+    const int64_t g64 = p - lane;
+    if (lane == 0 && valid) sg.heads[g64 >> 6] = heads;
+    if (!head) continue;
+    const int cw = (int)min((int64_t)kWave, n - g64);
+    int32_t b = table_find(t, k0, k1, k2);
+    if (b < 0) atomicOr(err, kErrMissingBlock);
+    if (b >= cap_blocks) {
+      atomicOr(err, kErrCapacity);
+      b = -1;
     }
+    uint32_t local = 0;
+    if (b >= 0)
+      local = (uint32_t)(atomicAdd((unsigned long long*)&sg.place[b],
+                                   (1ull << 32) | (unsigned long long)segment_length(heads, lane, cw)) >>
+                         32);
+    sg.in[g64 + __popcll(heads & lanemask_lt())] = make_uint2((uint32_t)b, local);
+  }
+}
+
+// sums of the counts per 1,024 blocks
+__global__ __launch_bounds__(kThreads) void counts_part_kernel(const uint64_t* __restrict__ bcnt, const int32_t* nblocks,
+                                                               int32_t cap, uint64_t* part) {
+  __shared__ uint64_t lds[kThreads / kWave];
+  const int32_t nb = min(*nblocks, cap);
+  const int32_t nparts = (nb + 1023) / 1024;
+  for (int32_t c = blockIdx.x; c < nparts; c += gridDim.x) {
+    uint64_t s = 0;
+    for (int32_t b = c * 1024 + threadIdx.x; b < min(nb, (c + 1) * 1024); b += kThreads) s += bcnt[b];
 #pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) heads += __shfl_xor(heads, o, kWave);
-    if (lane == 0) wsum[threadIdx.x / kWave] = heads;
+    for (int o = kWave / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, kWave);
+    if (lane_id() == 0) lds[threadIdx.x / kWave] = s;
     __syncthreads();
     if (threadIdx.x == 0) {
-      uint32_t tot = 0;
-      for (int i = 0; i < kThreads / kWave; ++i) tot += wsum[i];
-      tile_heads[tile] = tot;
+      uint64_t g = 0;
+      for (int w = 0; w < kThreads / kWave; ++w) g += lds[w];
+      part[c] = g;
     }
     __syncthreads();
   }
 }
 
-// The same outputs as bucket_kernel from the scratch slots recorded by the
-// activation that built this table (activate_kernel with pslot): a particle's
-// slot identifies its key, and slot_block maps it to the block number, so
-// neither x nor the table is read again.
-__global__ __launch_bounds__(kThreads) void bucket_slots_kernel(const uint32_t* __restrict__ pslot, int64_t n,
+__global__ __launch_bounds__(kThreads) void counts_scan_kernel(const uint64_t* __restrict__ bcnt,
+                                                               const uint64_t* __restrict__ part,
+                                                               const int32_t* nblocks, int32_t cap, SortView sv,
+                                                               uint32_t* segoff, uint32_t* counters) {
+  __shared__ uint64_t lds[2 * (kThreads / kWave)];
+  counts_scan(bcnt, part, min(min(*nblocks, cap), sv.cap_blocks), sv, segoff, counters, lds);
+}
+
+// Every segment into its bucket's list: first particle | length << 32. A wave
+// takes 8 groups, their loads in flight together (three dependent round trips).
+// slot_block: the segments name dedup slots; null: blocks.
+constexpr int kEmitGroups = 8;
+__global__ __launch_bounds__(kThreads) void segment_emit_kernel(Segments sg, int64_t n,
                                                                 const int32_t* __restrict__ slot_block, uint32_t ts,
-                                                                uint32_t* __restrict__ bkt, uint32_t* counts,
-                                                                int32_t cap_blocks, uint32_t* __restrict__ tile_heads,
-                                                                uint32_t* err) {
-  __shared__ uint32_t wsum[kThreads / kWave];
-  const int64_t ntiles = (n + kTile - 1) / kTile;
+                                                                const uint32_t* __restrict__ segoff,
+                                                                const int32_t* nblocks, int32_t cap,
+                                                                uint64_t* __restrict__ list, uint32_t* err) {
   const int lane = lane_id();
-  for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    uint32_t heads = 0;
-    // all rounds' slots (and, for lane 0, the slot before the wave) load
-    // together, then all run heads' block lookups: two memory round trips per
-    // tile instead of two per round
-    uint32_t sl[kTileItems], pv[kTileItems];
-    int32_t bl[kTileItems];
+  const int64_t ngroups = (n + kWave - 1) / kWave;
+  const int32_t nb = min(*nblocks, cap);
+  const int64_t nwaves = (int64_t)gridDim.x * (kThreads / kWave);
+  for (int64_t g0 = ((int64_t)blockIdx.x * (kThreads / kWave) + threadIdx.x / kWave) * kEmitGroups; g0 < ngroups;
+       g0 += nwaves * kEmitGroups) {
+    uint64_t heads[kEmitGroups];
+    uint2 e[kEmitGroups];
+    int32_t b[kEmitGroups];
 #pragma unroll
-    for (int r = 0; r < kTileItems; ++r) {
-      const int64_t p = tile * kTile + (int64_t)r * kThreads + threadIdx.x;
-      sl[r] = p < n ? pslot[p] : ~0u;
-      pv[r] = (lane == 0 && p < n && p > 0) ? pslot[p - 1] : ~0u;
-    }
-    uint32_t headm = 0;
+    for (int k = 0; k < kEmitGroups; ++k) heads[k] = g0 + k < ngroups ? sg.heads[g0 + k] : 0ull;
 #pragma unroll
-    for (int r = 0; r < kTileItems; ++r) {
-      const int64_t p = tile * kTile + (int64_t)r * kThreads + threadIdx.x;
-      const bool valid = p < n;
-      uint32_t prev = __shfl_up(sl[r], 1, kWave);
-      if (lane == 0) prev = pv[r];
-      const bool head = valid && (p == 0 || sl[r] != prev);
-      headm |= head ? (1u << r) : 0u;
-      const bool lookup = valid && (head || lane == 0);
-      bl[r] = lookup ? (sl[r] < ts ? slot_block[sl[r]] : -1) : -1;
+    for (int k = 0; k < kEmitGroups; ++k) {
+      e[k] = make_uint2(~0u, 0u);
+      if ((heads[k] >> lane) & 1ull) e[k] = sg.in[(g0 + k) * kWave + __popcll(heads[k] & lanemask_lt())];
     }
 #pragma unroll
-    for (int r = 0; r < kTileItems; ++r) {
-      const int64_t p = tile * kTile + (int64_t)r * kThreads + threadIdx.x;
-      const bool valid = p < n;
-      const bool head = (headm >> r) & 1u;
-      const bool lookup = valid && (head || lane == 0);
-      int32_t b = -1;
-      if (lookup) {
-        b = bl[r];
-        if (b < 0) atomicOr(err, kErrMissingBlock);
-        if (b >= cap_blocks) {
-          atomicOr(err, kErrCapacity);
-          b = -1;
-        }
-      }
-      const uint64_t lm = ballot(lookup);
-      const uint64_t le = lanemask_lt() | (1ull << lane);
-      const int src = 63 - __clzll(lm & le);
-      b = shfl(b, src < 0 ? 0 : src);
-      if (valid) bkt[p] = (uint32_t)(b < 0 ? 0 : b) | (head ? kHeadBit : 0u);
-      heads += head ? 1u : 0u;
-      const uint64_t vm = ballot(valid);
-      if (lookup && b >= 0) {
-        const uint64_t above = lm & ~le;
-        const int next = above ? (__ffsll((long long)above) - 1) : 64;
-        const uint64_t seg = (next >= 64 ? ~0ull : ((1ull << next) - 1ull)) & ~((1ull << lane) - 1ull);
-        atomicAdd(&counts[b], (uint32_t)__popcll(seg & vm));
-      }
+    for (int k = 0; k < kEmitGroups; ++k) {
+      b[k] = (int32_t)e[k].x;
+      if (slot_block) b[k] = e[k].x < ts ? slot_block[e[k].x] : -1;
+    }
+    uint32_t at[kEmitGroups];
+#pragma unroll
+    for (int k = 0; k < kEmitGroups; ++k) {
+      const bool ok = b[k] >= 0 && b[k] < nb;
+      at[k] = ok ? segoff[b[k]] + e[k].y : ~0u;
+      if (slot_block && !ok && ((heads[k] >> lane) & 1ull)) atomicOr(err, b[k] < 0 ? kErrMissingBlock : kErrCapacity);
     }
 #pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) heads += __shfl_xor(heads, o, kWave);
-    if (lane == 0) wsum[threadIdx.x / kWave] = heads;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      uint32_t tot = 0;
-      for (int i = 0; i < kThreads / kWave; ++i) tot += wsum[i];
-      tile_heads[tile] = tot;
+    for (int k = 0; k < kEmitGroups; ++k) {
+      if (at[k] == ~0u || (int64_t)at[k] >= n) continue;
+      const int64_t g64 = (g0 + k) * kWave;
+      const int cw = (int)min((int64_t)kWave, n - g64);
+      list[at[k]] = (uint64_t)(uint32_t)(g64 + lane) | ((uint64_t)segment_length(heads[k], lane, cw) << 32);
     }
-    __syncthreads();
   }
 }
 
-// Run ids of one round of a tile (round r, thread t -> particle tile*kTile +
-// r*kThreads + t): `carry` holds the heads before the round; returns the id of
-// the run containing this thread's particle (the number of heads at or before
-// it, minus one) and adds the round's heads to carry. Workgroup-uniform call.
-__device__ __forceinline__ uint32_t round_run_id(bool head, uint32_t& carry, uint32_t* lds) {
+// A bucket's particle indices in particle order, one workgroup per bucket: its
+// segments ordered by first particle (they are disjoint), each written as a run.
+// Up to 64 segments (particles in or near bucket order): a wave compares every
+// segment with every other and needs only the summed lengths before each. Up to
+// kPlaceLds: a bitonic sort in LDS and a scan of the lengths. Beyond (thousands
+// of particles per bucket, interleaved): a radix sort of the list in global
+// memory, 8 bits of the first particle at a time, `alt` the other buffer.
+constexpr int kPlaceLds = 4096;
+
+__device__ __forceinline__ void write_segment(int32_t* __restrict__ indices, int64_t n, int64_t at, uint32_t start,
+                                              uint32_t len, int lane) {
+  if ((uint32_t)lane < len && at + lane < n) indices[at + lane] = (int32_t)(start + lane);
+}
+
+// exclusive scan of one value per thread across the workgroup
+__device__ __forceinline__ uint32_t group_scan(uint32_t v, uint32_t* lds, uint32_t& total) {
   const int lane = lane_id(), wave = threadIdx.x / kWave;
-  const uint64_t hm = ballot(head);
-  if (lane == 0) lds[wave] = (uint32_t)__popcll(hm);
+  uint32_t inc = v;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const uint32_t u = __shfl_up(inc, o, kWave);
+    if (lane >= o) inc += u;
+  }
+  if (lane == kWave - 1) lds[wave] = inc;
   __syncthreads();
-  uint32_t before = 0, total = 0;
+  uint32_t before = 0;
+  total = 0;
 #pragma unroll
   for (int w = 0; w < kThreads / kWave; ++w) {
-    const uint32_t c = lds[w];
-    before += w < wave ? c : 0u;
-    total += c;
+    before += w < wave ? lds[w] : 0u;
+    total += lds[w];
   }
   __syncthreads();
-  const uint64_t le = lanemask_lt() | (1ull << lane);
-  const uint32_t rid = carry + before + (uint32_t)__popcll(hm & le) - 1u;
-  carry += total;
-  return rid;
+  return before + inc - v;
 }
 
-__global__ __launch_bounds__(kThreads) void run_emit_kernel(const uint32_t* __restrict__ bkt, int64_t n,
-                                                            const uint32_t* __restrict__ tile_base,
-                                                            uint32_t* run_start, uint32_t* rkey, uint32_t* rval) {
-  __shared__ uint32_t lds[kThreads / kWave];
-  const int64_t ntiles = (n + kTile - 1) / kTile;
-  for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    uint32_t carry = tile_base[tile];
-    uint32_t v[kTileItems];  // all rounds load before the first barrier
-#pragma unroll
-    for (int r = 0; r < kTileItems; ++r) {
-      const int64_t p = tile * kTile + (int64_t)r * kThreads + threadIdx.x;
-      v[r] = p < n ? bkt[p] : 0u;
-    }
-#pragma unroll
-    for (int r = 0; r < kTileItems; ++r) {
-      const int64_t p = tile * kTile + (int64_t)r * kThreads + threadIdx.x;
-      const bool head = p < n && (v[r] & kHeadBit);
-      const uint32_t rid = round_run_id(head, carry, lds);
-      if (head && rid < (uint32_t)n) {
-        run_start[rid] = (uint32_t)p;
-        rkey[rid] = v[r] & ~kHeadBit;
-        rval[rid] = rid;
+__global__ __launch_bounds__(kThreads) void segment_place_kernel(const uint64_t* __restrict__ bcnt,
+                                                                 const uint32_t* __restrict__ segoff,
+                                                                 const int32_t* nblocks, int32_t cap, SortView sv,
+                                                                 int64_t n, int32_t bits, uint64_t* list,
+                                                                 uint64_t* alt) {
+  __shared__ uint64_t seg[kPlaceLds];
+  __shared__ uint32_t hist[256], lds[kThreads / kWave];
+  const int lane = lane_id(), wave = threadIdx.x / kWave;
+  const int32_t nb = min(min(*nblocks, cap), sv.cap_blocks);
+  for (int32_t b = blockIdx.x; b < nb; b += gridDim.x) {
+    const uint32_t R = (uint32_t)(bcnt[b] >> 32);
+    const int64_t off = sv.offsets[b];
+    const uint32_t s0 = segoff[b];
+    if (R == 0 || (int64_t)s0 + R > n) continue;
+    if (R <= (uint32_t)kWave) {
+      // every wave orders the list for itself and writes every fourth segment
+      const uint64_t me = (uint32_t)lane < R ? list[s0 + lane] : ~0ull;
+      const uint32_t start = (uint32_t)me, len = (uint32_t)lane < R ? (uint32_t)(me >> 32) : 0u;
+      uint32_t before = 0;
+      for (uint32_t k = 0; k < R; ++k) {
+        const uint32_t ks = (uint32_t)__builtin_amdgcn_readlane((int)start, (int)k);
+        const uint32_t kl = (uint32_t)__builtin_amdgcn_readlane((int)len, (int)k);
+        before += ks < start ? kl : 0u;
       }
-    }
-  }
-}
-
-// Lengths of the runs in sorted order.
-__global__ void run_len_kernel(const uint32_t* __restrict__ sorted_ids, const uint32_t* __restrict__ run_start,
-                               const uint32_t* counters, int64_t n, uint32_t* run_len) {
-  const uint32_t R = min(counters[kCtrRuns], (uint32_t)n);
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < R; i += stride) {
-    const uint32_t id = sorted_ids[i];
-    if (id >= R) {  // cannot happen when the run passes agree; never index with it
-      run_len[i] = 0;
+      for (uint32_t k = wave; k < R; k += kThreads / kWave) {
+        const uint32_t ks = (uint32_t)__builtin_amdgcn_readlane((int)start, (int)k);
+        const uint32_t kl = (uint32_t)__builtin_amdgcn_readlane((int)len, (int)k);
+        const uint32_t kb = (uint32_t)__builtin_amdgcn_readlane((int)before, (int)k);
+        write_segment(sv.indices, n, off + kb, ks, kl, lane);
+      }
       continue;
     }
-    const uint32_t end = (id + 1 < R) ? run_start[id + 1] : (uint32_t)n;
-    const uint32_t st = run_start[id];
-    run_len[i] = (end >= st && end <= (uint32_t)n) ? end - st : 0u;
-  }
-}
-
-__global__ void run_dest_kernel(const uint32_t* __restrict__ sorted_ids, const uint32_t* __restrict__ dest_sorted,
-                                const uint32_t* counters, int64_t n, uint32_t* run_dest) {
-  const uint32_t R = min(counters[kCtrRuns], (uint32_t)n);
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < R; i += stride) {
-    const uint32_t id = sorted_ids[i];
-    if (id < R) run_dest[id] = dest_sorted[i];
-  }
-}
-
-__global__ __launch_bounds__(kThreads) void particle_scatter_kernel(const uint32_t* __restrict__ bkt, int64_t n,
-                                                                    const uint32_t* __restrict__ tile_base,
-                                                                    const uint32_t* __restrict__ run_start,
-                                                                    const uint32_t* __restrict__ run_dest,
-                                                                    const uint32_t* counters,
-                                                                    int32_t* __restrict__ indices) {
-  __shared__ uint32_t lds[kThreads / kWave];
-  const uint32_t R = min(counters[kCtrRuns], (uint32_t)n);
-  const int64_t ntiles = (n + kTile - 1) / kTile;
-  for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    uint32_t carry = tile_base[tile];
-    // three phases, each with its loads in flight together: the tile's
-    // bucket words, the run ids (LDS scans only), the runs' destinations
-    uint32_t w[kTileItems], rid[kTileItems];
-#pragma unroll
-    for (int r = 0; r < kTileItems; ++r) {
-      const int64_t p = tile * kTile + (int64_t)r * kThreads + threadIdx.x;
-      w[r] = p < n ? bkt[p] : 0u;
-    }
-#pragma unroll
-    for (int r = 0; r < kTileItems; ++r) {
-      const int64_t p = tile * kTile + (int64_t)r * kThreads + threadIdx.x;
-      rid[r] = round_run_id(p < n && (w[r] & kHeadBit), carry, lds);
-    }
-    uint32_t dest[kTileItems], start[kTileItems];
-#pragma unroll
-    for (int r = 0; r < kTileItems; ++r) {
-      const int64_t p = tile * kTile + (int64_t)r * kThreads + threadIdx.x;
-      const bool ok = p < n && rid[r] < R;
-      dest[r] = ok ? run_dest[rid[r]] : 0u;
-      start[r] = ok ? run_start[rid[r]] : 0u;
-    }
-#pragma unroll
-    for (int r = 0; r < kTileItems; ++r) {
-      const int64_t p = tile * kTile + (int64_t)r * kThreads + threadIdx.x;
-      if (p < n && rid[r] < R) {
-        const uint64_t dst = (uint64_t)dest[r] + ((uint32_t)p - start[r]);
-        if (dst < (uint64_t)n) indices[dst] = (int32_t)p;
+    if (R <= (uint32_t)kPlaceLds) {
+      uint32_t P = 128;
+      while (P < R) P <<= 1;
+      // keyed by the first particle in the high word
+      for (uint32_t i = threadIdx.x; i < P; i += kThreads) {
+        const uint64_t v = i < R ? list[s0 + i] : ~0ull;
+        seg[i] = (v << 32) | (v >> 32);
       }
+      __syncthreads();
+      for (uint32_t k = 2; k <= P; k <<= 1) {
+        for (uint32_t j = k >> 1; j > 0; j >>= 1) {
+          for (uint32_t i = threadIdx.x; i < P / 2; i += kThreads) {
+            const uint32_t lo = 2 * i - (i & (j - 1)), hi = lo + j;
+            const uint64_t a = seg[lo], c = seg[hi];
+            if ((a > c) == ((lo & k) == 0)) {
+              seg[lo] = c;
+              seg[hi] = a;
+            }
+          }
+          __syncthreads();
+        }
+      }
+      uint32_t carry = 0;
+      const bool runs = (uint32_t)bcnt[b] >= 8u * R;  // long segments: a wave writes each
+      for (uint32_t base = 0; base < R; base += kThreads) {  // uniform across the workgroup
+        const uint32_t i = base + threadIdx.x;
+        const uint64_t v = i < R ? seg[i] : 0ull;
+        const uint32_t start = (uint32_t)(v >> 32), len = (uint32_t)v;
+        uint32_t total;
+        const uint32_t at = carry + group_scan(len, lds, total);
+        if (runs) {
+          for (int k = 0; k < kWave; ++k) {  // len 0 past the list
+            const uint32_t kl = (uint32_t)__builtin_amdgcn_readlane((int)len, k);
+            write_segment(sv.indices, n, off + (uint32_t)__builtin_amdgcn_readlane((int)at, k),
+                          (uint32_t)__builtin_amdgcn_readlane((int)start, k), kl, lane);
+          }
+        } else {
+          for (uint32_t q = 0; q < len && off + at + q < n; ++q) sv.indices[off + at + q] = (int32_t)(start + q);
+        }
+        carry += total;
+      }
+      __syncthreads();
+      continue;
     }
+    uint64_t *from = list + s0, *to = alt + s0;
+    for (int shift = 0; shift < bits; shift += 8) {
+      for (int i = threadIdx.x; i < 256; i += kThreads) hist[i] = 0u;
+      __syncthreads();
+      for (uint32_t i = threadIdx.x; i < R; i += kThreads) atomicAdd(&hist[((uint32_t)from[i] >> shift) & 255u], 1u);
+      __syncthreads();
+      uint32_t total;
+      const uint32_t first = group_scan(hist[threadIdx.x], lds, total);
+      hist[threadIdx.x] = first;
+      __syncthreads();
+      for (uint32_t base = 0; base < R; base += kWave) {  // one wave at a time keeps the pass stable
+        if (wave == 0) {
+          const uint32_t i = base + lane;
+          const bool live = i < R;
+          const uint64_t v = live ? from[i] : 0ull;
+          const uint32_t d = ((uint32_t)v >> shift) & 255u;
+          uint64_t peers = ballot(live);
+#pragma unroll
+          for (int bit = 0; bit < 8; ++bit) {
+            const bool on = (d >> bit) & 1u;
+            const uint64_t m = ballot(on);
+            peers &= on ? m : ~m;
+          }
+          const uint32_t below = (uint32_t)__popcll(peers & lanemask_lt());
+          const uint32_t at = live ? hist[d] + below : 0u;
+          wave_lds_barrier();
+          if (live && below == 0) hist[d] += (uint32_t)__popcll(peers);
+          wave_lds_barrier();
+          if (live) to[at] = v;
+        }
+      }
+      __threadfence_block();
+      __syncthreads();
+      uint64_t* q = from;
+      from = to;
+      to = q;
+    }
+    uint32_t carry = 0;
+    for (uint32_t base = 0; base < R; base += kThreads) {
+      const uint32_t i = base + threadIdx.x;
+      const uint64_t v = i < R ? from[i] : 0ull;
+      const uint32_t start = (uint32_t)v, len = (uint32_t)(v >> 32);
+      uint32_t total;
+      const uint32_t at = carry + group_scan(len, lds, total);
+      for (uint32_t q = 0; q < len && off + at + q < n; ++q) sv.indices[off + at + q] = (int32_t)(start + q);
+      carry += total;
+    }
+    __syncthreads();
   }
 }
 
@@ -711,10 +1029,6 @@ __global__ void neighbours_kernel(TableView t, int32_t* __restrict__ nbr, uint32
     nbr[i] = table_find(t, t.active[3 * b] + ((d >> 2) & 1), t.active[3 * b + 1] + ((d >> 1) & 1),
                         t.active[3 * b + 2] + (d & 1));
   }
-}
-
-__global__ void set_counter_kernel(uint32_t* counters, int slot, const uint32_t* src) {
-  counters[slot] = *src;
 }
 
 int bits_for(uint64_t maxval) {
@@ -734,8 +1048,7 @@ uint64_t bitmap_words(const Workspace& ws, uint64_t order_bound) {
 
 // dedup entries -> ranked, placed and keyed table entries (shared tail of
 // activation and enlargement); the bitmap was cleared with the dedup scratch
-hipError_t finish_insertion(const TableView& t, Workspace& ws, uint64_t order_bound, hipStream_t s,
-                            int32_t* slot_block = nullptr) {
+hipError_t finish_insertion(const TableView& t, Workspace& ws, uint64_t order_bound, hipStream_t s) {
   const uint64_t words = bitmap_words(ws, order_bound);
   collect_new_kernel<<<kCollectGroups, kThreads, 0, s>>>(ws.skey, ws.sorder, ws.dmask, ws.ts_cap, t, ws.counters,
                                                          ws.la_key,
@@ -744,40 +1057,60 @@ hipError_t finish_insertion(const TableView& t, Workspace& ws, uint64_t order_bo
   if (e != hipSuccess) return e;
   const int gl = groups_for(ws.list_cap, kThreads);
   assign_kernel<<<gl, kThreads, 0, s>>>(ws.la_key, ws.la_val, ws.bitmap, ws.bm_prefix, (uint32_t)words, ws.skey, t,
-                                        ws.counters, ws.list_cap, ws.err, slot_block);
+                                        ws.counters, ws.list_cap, ws.err);
   fill_keys_kernel<<<gl, kThreads, 0, s>>>(t, ws.counters, ws.list_cap, ws.err);
   return hipGetLastError();
 }
 
 }  // namespace
 
-hipError_t table_clear(const TableView& t, Workspace& ws, hipStream_t s, uint32_t* zero, int64_t nzero) {
+hipError_t table_clear(const TableView& t, Workspace& ws, hipStream_t s) {
   const int64_t m = (int64_t)t.T > (int64_t)ws.ts_cap ? t.T : ws.ts_cap;
   clear_table_kernel<<<groups_for(m, kThreads), kThreads, 0, s>>>(t, ws.skey, ws.sorder, ws.dmask, ws.ts_cap,
-                                                                   ws.counters, zero, zero ? nzero : 0);
+                                                                   ws.counters);
   return hipGetLastError();
 }
 
+namespace {
+
+// the activation's insertion pass; particles per launch decide the groups per wave
+template <bool kSegs>
+void launch_activate(Workspace& ws, const float* x, int64_t n, float dx, int blockLen, int offset, float disp,
+                     const Segments& sg, hipStream_t s, const SceneSet* ss) {
+  const float dxinv = (float)1.0 / dx;
+  const bool wide = n >= (int64_t)1 << 22;
+  const int g = groups_for(n, kThreads * (wide ? 4 : 1));
+  const Dedup dd = dedup_of(ws);
+  if (ss && ss->n > 0) {
+    if (wide)
+      activate_kernel<true, kSegs, 4><<<g, kThreads, 0, s>>>(x, n, dxinv, blockLen, offset, disp, dd, sg, *ss);
+    else
+      activate_kernel<true, kSegs, 1><<<g, kThreads, 0, s>>>(x, n, dxinv, blockLen, offset, disp, dd, sg, *ss);
+  } else if (wide) {
+    activate_kernel<false, kSegs, 4><<<g, kThreads, 0, s>>>(x, n, dxinv, blockLen, offset, disp, dd, sg, SceneSet{});
+  } else {
+    activate_kernel<false, kSegs, 1><<<g, kThreads, 0, s>>>(x, n, dxinv, blockLen, offset, disp, dd, sg, SceneSet{});
+  }
+}
+
+Segments segments_of(const Workspace& ws, uint64_t* place) {
+  Segments sg;
+  sg.heads = ws.seg_heads;
+  sg.in = ws.seg_in;
+  sg.place = place;
+  return sg;
+}
+
+}  // namespace
+
 hipError_t table_activate(const TableView& t, Workspace& ws, const float* x, int64_t n, float dx,
-                          int blockLen, int offset, float disp, hipStream_t s, bool record_slots,
-                          const SceneSet* ss) {
+                          int blockLen, int offset, float disp, hipStream_t s) {
   if (blockLen <= 0) return hipErrorInvalidValue;
-  int32_t* slot_block = record_slots ? ws.slot_block : nullptr;
   const uint64_t order_bound = (uint64_t)(n > 0 ? n : 1);
   clear_scratch_kernel<<<groups_for(ws.ts_cap, kThreads), kThreads, 0, s>>>(
-      ws.skey, ws.sorder, ws.dmask, ws.ts_cap, t.cnt, ws.counters, slot_block, ws.bitmap,
-      (int64_t)bitmap_words(ws, order_bound));
-  const float dxinv = (float)1.0 / dx;
-  if (n > 0) {
-    const int g = groups_for(n, kThreads * kActItems);
-    uint32_t* ps = record_slots ? ws.pslot : nullptr;
-    if (ss && ss->n > 0)
-      activate_kernel<true><<<g, kThreads, 0, s>>>(x, n, dxinv, blockLen, offset, disp, dedup_of(ws), ps, *ss);
-    else
-      activate_kernel<false><<<g, kThreads, 0, s>>>(x, n, dxinv, blockLen, offset, disp, dedup_of(ws), ps,
-                                                    SceneSet{});
-  }
-  return finish_insertion(t, ws, order_bound, s, slot_block);
+      ws.skey, ws.sorder, ws.dmask, ws.ts_cap, t.cnt, ws.counters, ws.bitmap, (int64_t)bitmap_words(ws, order_bound));
+  if (n > 0) launch_activate<false>(ws, x, n, dx, blockLen, offset, disp, Segments{}, s, nullptr);
+  return finish_insertion(t, ws, order_bound, s);
 }
 
 hipError_t table_enlarge(const TableView& t, Workspace& ws, const int32_t lo[3], const int32_t hi[3],
@@ -787,8 +1120,7 @@ hipError_t table_enlarge(const TableView& t, Workspace& ws, const int32_t lo[3],
   const int64_t total_cap = (int64_t)n0_cap * e0 * e1 * e2;
   const uint64_t order_bound = (uint64_t)(total_cap > 0 ? total_cap : 1);
   clear_scratch_kernel<<<groups_for(ws.ts_cap, kThreads), kThreads, 0, s>>>(
-      ws.skey, ws.sorder, ws.dmask, ws.ts_cap, t.cnt, ws.counters, nullptr, ws.bitmap,
-      (int64_t)bitmap_words(ws, order_bound));
+      ws.skey, ws.sorder, ws.dmask, ws.ts_cap, t.cnt, ws.counters, ws.bitmap, (int64_t)bitmap_words(ws, order_bound));
   enlarge_kernel<<<groups_for(total_cap, kThreads), kThreads, 0, s>>>(t.active, ws.counters, lo[0], lo[1], lo[2],
                                                                        e0, e1, e2, dedup_of(ws));
   return finish_insertion(t, ws, order_bound, s);
@@ -808,30 +1140,17 @@ hipError_t table_query(const TableView& t, const int32_t* keys, int64_t n, int32
 
 namespace {
 
-// after the bucket pass (bkt with run heads, counts, tile_heads): stable
-// placement of the particles through the runs
-hipError_t place_runs(Workspace& ws, int64_t n, const SortView& out, int64_t ntiles, int gt, hipStream_t s) {
-  const int64_t nb1 = (int64_t)out.cap_blocks + 1;
-  uint32_t* counts = (uint32_t*)out.counts;
-  hipError_t e = exclusive_scan_u32(ws.tile_heads, ws.tile_base, nullptr, (uint32_t)ntiles, ws.scan_tmp,
-                                    ws.counters + kCtrRuns, s);
-  if (e != hipSuccess) return e;
-  run_emit_kernel<<<gt, kThreads, 0, s>>>(ws.bkt, n, ws.tile_base, ws.run_start, ws.rk_a, ws.rv_a);
-  bool alt = false;
-  e = radix_sort_pairs(ws.rk_a, ws.rv_a, ws.rk_b, ws.rv_b, ws.counters + kCtrRuns, (uint32_t)n,
-                       bits_for((uint64_t)out.cap_blocks - 1), ws.rs_scratch, s, &alt);
-  if (e != hipSuccess) return e;
-  const uint32_t* sorted_ids = alt ? ws.rv_b : ws.rv_a;
-  uint32_t* spare = alt ? ws.rk_a : ws.rk_b;  // free buffer for the sorted dest scan
-  const int gr = groups_for(n, kThreads) < 1024 ? groups_for(n, kThreads) : 1024;  // grid-stride over R <= n runs
-  run_len_kernel<<<gr, kThreads, 0, s>>>(sorted_ids, ws.run_start, ws.counters, n, ws.run_len);
-  e = exclusive_scan_u32(ws.run_len, spare, ws.counters + kCtrRuns, (uint32_t)n, ws.scan_tmp, nullptr, s);
-  if (e != hipSuccess) return e;
-  run_dest_kernel<<<gr, kThreads, 0, s>>>(sorted_ids, spare, ws.counters, n, ws.run_dest);
-  e = exclusive_scan_u32(counts, (uint32_t*)out.offsets, nullptr, (uint32_t)nb1, ws.scan_tmp, nullptr, s);
-  if (e != hipSuccess) return e;
-  particle_scatter_kernel<<<gt, kThreads, 0, s>>>(ws.bkt, n, ws.tile_base, ws.run_start, ws.run_dest,
-                                                  ws.counters, out.indices);
+// segments counted per block (bcnt) and scanned (offsets, segoff): the lists
+// and the buckets' indices. slot_block as in segment_emit_kernel.
+hipError_t place_segments(Workspace& ws, int64_t n, const int32_t* slot_block, const int32_t* nblocks,
+                          const SortView& out, hipStream_t s) {
+  const int64_t waves = (n + (int64_t)kWave * kEmitGroups - 1) / ((int64_t)kWave * kEmitGroups);
+  const int32_t cap = out.cap_blocks < (int32_t)ws.ts_cap ? out.cap_blocks : (int32_t)ws.ts_cap;
+  segment_emit_kernel<<<groups_for(waves * kWave, kThreads), kThreads, 0, s>>>(
+      segments_of(ws, nullptr), n, slot_block, ws.ts_cap, ws.segoff, nblocks, cap, ws.seg_list, ws.err);
+  const int g = cap < 16384 ? cap : 16384;
+  segment_place_kernel<<<g, kThreads, 0, s>>>(ws.bcnt, ws.segoff, nblocks, cap, out, n, bits_for((uint64_t)n - 1),
+                                              ws.seg_list, ws.seg_alt);
   return hipGetLastError();
 }
 
@@ -840,33 +1159,117 @@ hipError_t place_runs(Workspace& ws, int64_t n, const SortView& out, int64_t nti
 hipError_t bucket_sort(const TableView& t, Workspace& ws, const float* x, int64_t n, float dx, int blockLen,
                        int offset, float disp, const SortView& out, hipStream_t s) {
   if (n > (int64_t)ws.n_cap) return hipErrorInvalidValue;
-  const int64_t nb1 = (int64_t)out.cap_blocks + 1;
-  uint32_t* counts = (uint32_t*)out.counts;
-  zero_u32_kernel<<<groups_for(nb1, kThreads), kThreads, 0, s>>>(counts, nb1);
-  if (n <= 0) {
-    return exclusive_scan_u32(counts, (uint32_t*)out.offsets, nullptr, (uint32_t)nb1, ws.scan_tmp, nullptr, s);
-  }
-  const int64_t ntiles = (n + kTile - 1) / kTile;
-  const int gt = (int)(ntiles < 65536 ? ntiles : 65536);
   const float dxinv = (float)1.0 / dx;
-  bucket_kernel<<<gt, kThreads, 0, s>>>(x, n, dxinv, blockLen, offset, disp, t, ws.bkt, counts, out.cap_blocks,
-                                        ws.tile_heads, ws.err);
-  return place_runs(ws, n, out, ntiles, gt, s);
+  zero_u32_kernel<<<groups_for(2ll * ws.ts_cap, kThreads) < 2048 ? groups_for(2ll * ws.ts_cap, kThreads) : 2048,
+                    kThreads, 0, s>>>((uint32_t*)ws.bcnt, 2ll * ws.ts_cap);
+  const int32_t cap = out.cap_blocks < (int32_t)ws.ts_cap ? out.cap_blocks : (int32_t)ws.ts_cap;
+  if (n > 0)
+    bucket_kernel<<<groups_for(n, kThreads), kThreads, 0, s>>>(x, n, dxinv, blockLen, offset, disp, t,
+                                                               segments_of(ws, ws.bcnt), cap, ws.err);
+  const int gp = (cap + 1023) / 1024;
+  counts_part_kernel<<<gp < 1024 ? gp : 1024, kThreads, 0, s>>>(ws.bcnt, t.cnt, cap, ws.bpart);
+  const int gs = (out.cap_blocks + 1024) / 1024;
+  counts_scan_kernel<<<gs < 1024 ? gs : 1024, kThreads, 0, s>>>(ws.bcnt, ws.bpart, t.cnt, cap, out, ws.segoff,
+                                                                   ws.counters);
+  if (n <= 0) return hipGetLastError();
+  return place_segments(ws, n, nullptr, t.cnt, out, s);
 }
 
-hipError_t bucket_sort_slots(Workspace& ws, int64_t n, const SortView& out, hipStream_t s, bool counts_zeroed) {
+// ------------------------------------------------------- the substep's build
+namespace {
+
+// orders of the particles' keys are particle indices, those of the enlargement
+// candidates (8 b + j) lie below T while the particles' blocks fill at most T / 8
+Ranks ranks_a(const Workspace& ws, int64_t n) {
+  Ranks r;
+  r.bitmap = ws.bitmap;
+  r.c1 = ws.rank_a;
+  r.c2 = r.c1 + rank_pad(ws.n_cap >> kR1);
+  r.c3 = r.c2 + rank_pad(ws.n_cap >> kR2);
+  r.words = (uint32_t)((uint64_t)(n > 0 ? n : 1) / 32 + 1);
+  return r;
+}
+Ranks ranks_b(const Workspace& ws, const TableView& t) {
+  Ranks r;
+  r.bitmap = ws.bitmap_b;
+  r.c1 = ws.rank_b;
+  r.c2 = r.c1 + rank_pad(ws.ts_cap >> kR1);
+  r.c3 = r.c2 + rank_pad(ws.ts_cap >> kR2);
+  const int32_t n0 = t.T / 8 > 0 ? t.T / 8 : 1;
+  r.words = (uint32_t)(8ull * (uint64_t)n0 / 32 + 1);
+  return r;
+}
+int64_t rank_words(uint64_t orders) {
+  return (int64_t)(rank_pad(orders >> kR1) + rank_pad(orders >> kR2) + rank_pad(orders >> kR3));
+}
+int few(int64_t n, int most) {
+  const int g = groups_for(n, kThreads);
+  return g < most ? g : most;
+}
+
+}  // namespace
+
+size_t rank_scratch_words(uint64_t orders) { return (size_t)rank_words(orders); }
+
+hipError_t build_clear(const TableView& t, Workspace& ws, int64_t n, hipStream_t s) {
+  ClearList c;
+  int64_t most = 0;
+  auto add = [&](void* p, int64_t words, uint32_t v) {
+    c.p[c.count] = (uint32_t*)p;
+    c.n[c.count] = words;
+    c.v[c.count++] = v;
+    most = words > most ? words : most;
+  };
+  const int64_t ts = ws.ts_cap;
+  add(t.keys, 3ll * t.T, (uint32_t)kKeySentinel);
+  add(t.indices, t.T, 0xffffffffu);
+  add(t.status, t.T, 0xffffffffu);
+  add(ws.skey, 2 * ts, 0xffffffffu);
+  add(ws.sorder, ts, 0xffffffffu);
+  add(ws.scnt, 2 * ts, 0u);
+  add(ws.dmask, 2 * (ts / 32 + 1), 0u);  // both masks
+  add(ws.bitmap, ranks_a(ws, n).words, 0u);
+  add(ws.rank_a, rank_words(ws.n_cap), 0u);
+  add(ws.bitmap_b, ranks_b(ws, t).words, 0u);
+  add(ws.rank_b, rank_words(ws.ts_cap), 0u);
+  add(ws.bpart, 2 * (ts / 1024 + 2), 0u);
+  build_clear_kernel<<<few(most / 4 + 1, 4096), kThreads, 0, s>>>(c, t, ws.counters);
+  return hipGetLastError();
+}
+
+hipError_t build_activate(const TableView& t, Workspace& ws, const float* x, int64_t n, float dx, hipStream_t s,
+                          const SceneSet* ss) {
   if (n > (int64_t)ws.n_cap) return hipErrorInvalidValue;
-  const int64_t nb1 = (int64_t)out.cap_blocks + 1;
-  uint32_t* counts = (uint32_t*)out.counts;
-  if (!counts_zeroed) zero_u32_kernel<<<groups_for(nb1, kThreads), kThreads, 0, s>>>(counts, nb1);
-  if (n <= 0) {
-    return exclusive_scan_u32(counts, (uint32_t*)out.offsets, nullptr, (uint32_t)nb1, ws.scan_tmp, nullptr, s);
-  }
-  const int64_t ntiles = (n + kTile - 1) / kTile;
-  const int gt = (int)(ntiles < 65536 ? ntiles : 65536);
-  bucket_slots_kernel<<<gt, kThreads, 0, s>>>(ws.pslot, n, ws.slot_block, ws.ts_cap, ws.bkt, counts,
-                                              out.cap_blocks, ws.tile_heads, ws.err);
-  return place_runs(ws, n, out, ntiles, gt, s);
+  if (n > 0) launch_activate<true>(ws, x, n, dx, 4, -2, 0.5f, segments_of(ws, ws.scnt), s, ss);
+  const uint32_t nw = (ws.ts_cap + 31u) / 32u;
+  build_collect_kernel<<<(int)((nw + kWave - 1) / kWave), kThreads, 0, s>>>(
+      ws.dmask, nw, ws.sorder, ranks_a(ws, n), ws.counters + kCtrList, ws.la_key, ws.la_val);
+  return hipGetLastError();
+}
+
+hipError_t build_enlarge(const TableView& t, Workspace& ws, int64_t n, const SortView& sv, hipStream_t s) {
+  uint32_t* mask2 = ws.dmask + (ws.ts_cap / 32 + 1);
+  const int g = few(8ll * ws.ts_cap, 1024);
+  build_number_kernel<true><<<g, kThreads, 0, s>>>(ws.counters + kCtrList, nullptr, ws.la_key, ws.la_val,
+                                                   ranks_a(ws, n), t, dedup_of(ws), mask2, ws.slot_block, ws.scnt,
+                                                   ws.bcnt, ws.bpart, ws.nbr);
+  const uint32_t nw = (ws.ts_cap + 31u) / 32u;
+  build_collect_kernel<<<(int)((nw + kWave - 1) / kWave), kThreads, 0, s>>>(
+      mask2, nw, ws.sorder, ranks_b(ws, t), ws.counters + kCtrListB, ws.lb_key, ws.lb_val);
+  build_number_kernel<false><<<g, kThreads, 0, s>>>(ws.counters + kCtrListB, ws.counters + kCtrList, ws.lb_key,
+                                                    ws.lb_val, ranks_b(ws, t), t, dedup_of(ws), mask2, ws.slot_block,
+                                                    ws.scnt, ws.bcnt, ws.bpart, ws.nbr);
+  const int64_t chunks = ((int64_t)sv.cap_blocks + 1024) / 1024;
+  int gf = few(ws.ts_cap, 1024);
+  if (gf < chunks) gf = (int)(chunks < 1024 ? chunks : 1024);
+  build_finish_kernel<<<gf, kThreads, 0, s>>>(t, ws.counters, ws.err, ws.slot_block, ws.ts_cap, ws.nbr, ws.bcnt,
+                                              ws.bpart, sv, ws.segoff);
+  return hipGetLastError();
+}
+
+hipError_t build_place(const TableView& t, Workspace& ws, int64_t n, const SortView& out, hipStream_t s) {
+  if (n <= 0) return hipSuccess;
+  return place_segments(ws, n, ws.slot_block, reinterpret_cast<const int32_t*>(ws.counters + kCtrList), out, s);
 }
 
 }  // namespace zsmpm

@@ -82,11 +82,7 @@ __device__ __forceinline__ void node_home(int r0, int r1, int r2, int& nb, int& 
   cell = ((r0 & 3) << 4) | ((r1 & 3) << 2) | (r2 & 3);
 }
 
-__global__ void grid_clear_kernel(float* grid, const int32_t* nblocks, int32_t cap, uint32_t* counters) {
-  if (counters && blockIdx.x == 0 && threadIdx.x == 0) {
-    counters[kCtrQueue] = 0u;
-    counters[kCtrMaxVel] = 0u;
-  }
+__global__ void grid_clear_kernel(float* grid, const int32_t* nblocks, int32_t cap) {
   const int32_t nb = min(*nblocks, cap);
   const int64_t total = (int64_t)nb * kChannels * kBlockCells / 4;
   float4* g4 = reinterpret_cast<float4*>(grid);
@@ -1447,10 +1443,9 @@ hipError_t check_launch_limits(int device) {
   return closure_launch_limits();
 }
 
-hipError_t grid_clear(float* grid, const int32_t* nblocks_dev, int32_t cap_blocks, hipStream_t s,
-                      uint32_t* counters) {
+hipError_t grid_clear(float* grid, const int32_t* nblocks_dev, int32_t cap_blocks, hipStream_t s) {
   const int64_t total = (int64_t)cap_blocks * kChannels * kBlockCells / 4;
-  grid_clear_kernel<<<groups_for(total, kThreads), kThreads, 0, s>>>(grid, nblocks_dev, cap_blocks, counters);
+  grid_clear_kernel<<<groups_for(total, kThreads), kThreads, 0, s>>>(grid, nblocks_dev, cap_blocks);
   return hipGetLastError();
 }
 

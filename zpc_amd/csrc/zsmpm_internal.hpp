@@ -119,7 +119,7 @@ __device__ __forceinline__ int32_t scene_of_particle(const int64_t* first, int32
 enum : int {
   kCtrList = 0,     // unique new keys found by a dedup pass
   kCtrCnt0 = 1,     // table size before the current insertion pass
-  kCtrRuns = 2,     // particle runs in the bucket sort
+  kCtrRuns = 2,     // segments of equal bucket in the last bucket sort
   kCtrFp64 = 3,     // particles that took the FP64 SVD path
   kCtrFallback = 4, // particles that took the SVD fallback of the learned closure
   kCtrMaxVel = 5,   // max |v|^2 as float bits
@@ -127,6 +127,7 @@ enum : int {
   kCtrFbQueue = 7,  // length of the closure's SVD fallback queue (per pass)
   kCtrNetQueue = 8, // waves the closure's network pass took (per pass)
   kCtrNetWaves = 9, // waves that evaluated the closure's network (all passes)
+  kCtrListB = 11,   // unique keys the substep's enlargement adds
   kCtrBhtRounds = 10, // placement rounds of the last bht insertion (host-side, filled by the counters call)
   kCtrCount = 16
 };
@@ -157,18 +158,16 @@ struct Workspace {
   uint32_t* lb_key = nullptr;
   uint32_t* lb_val = nullptr;
   uint32_t list_cap = 0;
-  uint32_t* bkt = nullptr;      // [n_cap] bucket of each particle
-  uint32_t* run_start = nullptr;  // [n_cap]
-  uint32_t* rk_a = nullptr;     // [n_cap] run sort keys/vals (ping-pong)
-  uint32_t* rv_a = nullptr;
-  uint32_t* rk_b = nullptr;
-  uint32_t* rv_b = nullptr;
-  uint32_t* run_len = nullptr;  // [n_cap]
-  uint32_t* run_dest = nullptr; // [n_cap]
-  uint32_t* tile_heads = nullptr;  // [n_cap / 4096 + 1]
-  uint32_t* tile_base = nullptr;
-  uint32_t* rs_scratch = nullptr;
-  size_t rs_words = 0;
+  // bucket sort: per 64-particle group the heads of its segments, per segment
+  // its bucket and place, and the buckets' segment lists (two, to order in)
+  uint64_t* seg_heads = nullptr;  // [n_cap / 64 + 2]
+  uint2* seg_in = nullptr;        // [n_cap + 64]
+  uint64_t* seg_list = nullptr;   // [n_cap]
+  uint64_t* seg_alt = nullptr;    // [n_cap]
+  uint64_t* scnt = nullptr;       // [ts_cap] per dedup slot: segments << 32 | particles
+  uint64_t* bcnt = nullptr;       // [ts_cap] the same per block
+  uint64_t* bpart = nullptr;      // [ts_cap / 1024 + 2] and summed per 1,024 blocks
+  uint32_t* segoff = nullptr;     // [ts_cap] start of each block's segment list
   uint32_t* scan_tmp = nullptr;  // tile sums for scans
   size_t scan_words = 0;
   uint32_t* counters = nullptr;  // [kCtrCount]
@@ -186,9 +185,11 @@ struct Workspace {
   uint32_t* bitmap = nullptr;    // [bm_words] one bit per insertion order: the orders of new keys
   uint32_t* bm_prefix = nullptr; // [bm_words] exclusive prefix of the bit counts
   uint32_t bm_words = 0;
-  uint32_t* pslot = nullptr;     // [n_cap] scratch slot of each particle's key (recording activation)
+  uint32_t* bitmap_b = nullptr;  // [ts_cap / 32 + 10] the same of the substep's enlargement orders
+  uint32_t* rank_a = nullptr;    // [rank_scratch_words(n_cap)] marked orders counted by size class (sparsity.hip)
+  uint32_t* rank_b = nullptr;    // [rank_scratch_words(ts_cap)]
   int32_t* slot_block = nullptr; // [ts_cap] block number of the key in each scratch slot
-  uint32_t* dmask = nullptr;     // [ts_cap / 32 + 1] one bit per dedup slot claimed by the current pass
+  uint32_t* dmask = nullptr;     // [2 (ts_cap / 32 + 1)] one bit per dedup slot claimed by a pass
 };
 
 // The next substep's constitutive part computed inside G2P from the updated
@@ -233,36 +234,35 @@ hipError_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, 
                             hipStream_t s, bool* result_in_alt);
 
 // ---------------------------------------------------------------- sparsity
-// zero[0, nzero) is cleared by the same launch (the substep's bucket counts)
-hipError_t table_clear(const TableView& t, Workspace& ws, hipStream_t s, uint32_t* zero = nullptr,
-                       int64_t nzero = 0);
-// record_slots: also fill ws.pslot / ws.slot_block for bucket_sort_slots
-// (the table must be empty: every key is then new)
-// ss (a batch): each particle's key uses its scene's dx and is shifted by the
-// scene's key offset
+hipError_t table_clear(const TableView& t, Workspace& ws, hipStream_t s);
 hipError_t table_activate(const TableView& t, Workspace& ws, const float* x, int64_t n, float dx,
-                          int blockLen, int offset, float disp, hipStream_t s, bool record_slots = false,
-                          const SceneSet* ss = nullptr);
+                          int blockLen, int offset, float disp, hipStream_t s);
 hipError_t table_enlarge(const TableView& t, Workspace& ws, const int32_t lo[3], const int32_t hi[3],
                          int32_t n0_cap, hipStream_t s);
 hipError_t table_query(const TableView& t, const int32_t* keys, int64_t n, int32_t* out, hipStream_t s);
 hipError_t bucket_sort(const TableView& t, Workspace& ws, const float* x, int64_t n, float dx,
                        int blockLen, int offset, float disp, const SortView& out, hipStream_t s);
-// bucket_sort of the particles a recording activation just inserted into an
-// emptied table (blockLen 4, offset -2, displacement 0.5 as that activation)
-// counts_zeroed: out.counts[0, cap_blocks] is already zero (table_clear did it)
-hipError_t bucket_sort_slots(Workspace& ws, int64_t n, const SortView& out, hipStream_t s,
-                             bool counts_zeroed = false);
+size_t rank_scratch_words(uint64_t orders);
+// The substep's build: clear, activation (blockLen 4, offset -2, displacement
+// 0.5), enlargement by {0,1}^3 and bucket sort in one chain. The table, the
+// buckets (counts and offsets after build_enlarge, indices after build_place)
+// and errors are those of table_clear, table_activate, table_enlarge and
+// bucket_sort; ws.nbr holds the neighbours of the blocks with particles.
+// build_clear also resets the P2G bucket queue and the max |v|^2 counter.
+// ss (a batch): each particle's key uses its scene's dx and is shifted by the
+// scene's key offset
+hipError_t build_clear(const TableView& t, Workspace& ws, int64_t n, hipStream_t s);
+hipError_t build_activate(const TableView& t, Workspace& ws, const float* x, int64_t n, float dx, hipStream_t s,
+                          const SceneSet* ss);
+hipError_t build_enlarge(const TableView& t, Workspace& ws, int64_t n, const SortView& sv, hipStream_t s);
+hipError_t build_place(const TableView& t, Workspace& ws, int64_t n, const SortView& out, hipStream_t s);
 // ws.nbr for every active block (the 2x2x2 blocks a bucket's stencils cover)
 hipError_t block_neighbours(const TableView& t, Workspace& ws, hipStream_t s);
 
 // ---------------------------------------------------------------- transfer
 // every transfer kernel's static LDS fits the device's per-workgroup limit
 hipError_t check_launch_limits(int device);
-// with counters: also resets the P2G bucket queue and the max |v|^2 counter
-// (then p2g_scatter is called with reset_queue = false)
-hipError_t grid_clear(float* grid, const int32_t* nblocks_dev, int32_t cap_blocks, hipStream_t s,
-                      uint32_t* counters = nullptr);
+hipError_t grid_clear(float* grid, const int32_t* nblocks_dev, int32_t cap_blocks, hipStream_t s);
 // P2G = stress (per particle, writes ws.contrib and logJp) + scatter (per bucket).
 // beside_sparsity: the pass runs on a second stream next to the sparsity
 // stages, and leaves room on every CU for them (at most three of its
