@@ -21,7 +21,7 @@ hipError_t build_clear(const TableView&, Workspace&, int64_t, hipStream_t s) { r
 hipError_t build_activate(const TableView&, Workspace&, const float*, int64_t, float, hipStream_t s, const SceneSet* ss) { return scenes_ok(ss, s); }
 hipError_t build_enlarge(const TableView&, Workspace&, int64_t, const SortView&, hipStream_t s) { return touch(s); }
 hipError_t build_place(const TableView&, Workspace&, int64_t, const SortView&, hipStream_t s) { return touch(s); }
-size_t rank_scratch_words(uint64_t orders) { return orders / 512 + 64; }
+size_t rank_scratch_words() { return 64; }
 hipError_t table_enlarge(const TableView&, Workspace&, const int32_t*, const int32_t*, int32_t, hipStream_t s) { return touch(s); }
 hipError_t table_query(const TableView&, const int32_t*, int64_t, int32_t*, hipStream_t s) { return touch(s); }
 hipError_t bucket_sort(const TableView&, Workspace&, const float*, int64_t, float, int, int, float, const SortView&, hipStream_t s) { return touch(s); }
@@ -35,12 +35,12 @@ hipError_t mlp_grad(const float*, const float*, const float*, int64_t, float*, f
 hipError_t mlp_reduce(float*, float*, float*, const float*, const float*, int, float, float, float, float*, float*, hipStream_t s) { return touch(s); }
 hipError_t mlp_harvest(const Model&, const float*, const float*, int64_t, float*, float*, hipStream_t s) { return touch(s); }
 hipError_t closure_launch_limits() { return hipSuccess; }
-hipError_t p2g_scatter(const ParticlesView&, const TableView&, const SortView&, float*, int32_t, float, float, bool, Workspace&, hipStream_t s, bool, const SceneSet* ss) { return scenes_ok(ss, s); }
+hipError_t p2g_scatter(const ParticlesView&, const TableView&, const SortView&, float*, int32_t, float, float, bool, Workspace&, hipStream_t s, bool, const SceneSet* ss, const StressFrom&) { return scenes_ok(ss, s); }
 hipError_t grid_update(float*, int32_t, const TableView&, float, const float*, const Colliders&, float, int, Workspace&, hipStream_t s, const SceneSet* ss, const GeneralColliders* gen) { return gen && gen->n > kMaxColliders ? hipErrorInvalidValue : scenes_ok(ss, s); }
 hipError_t g2p(const ParticlesView&, const ParticlesView*, const TableView&, const SortView&, const float*, int32_t, float, float, Workspace&, hipStream_t s, const NextStress*, const SceneSet* ss) { return scenes_ok(ss, s); }
 hipError_t grid_angular_momentum(const float*, int32_t, const TableView&, float, int, int, double*, Workspace&, hipStream_t s) { return touch(s); }
-hipError_t p2c2g_scatter(const ParticlesView&, const TableView&, const SortView&, float*, int32_t, float, float, Workspace&, hipStream_t s) { return touch(s); }
-hipError_t p2g_force_scatter(const ParticlesView&, const TableView&, const SortView&, float*, int32_t, float, float, Workspace&, hipStream_t s) { return touch(s); }
+hipError_t p2c2g_scatter(const ParticlesView&, const TableView&, const SortView&, float*, int32_t, float, float, Workspace&, hipStream_t s, const StressFrom&) { return touch(s); }
+hipError_t p2g_force_scatter(const ParticlesView&, const TableView&, const SortView&, float*, int32_t, float, float, Workspace&, hipStream_t s, const StressFrom&) { return touch(s); }
 hipError_t g2c2p(const ParticlesView&, const TableView&, const SortView&, const float*, int32_t, float, float, Workspace&, hipStream_t s) { return touch(s); }
 hipError_t reorder_particles(const ParticlesView&, const ParticlesView&, const int32_t*, Workspace&, hipStream_t s) { return touch(s); }
 hipError_t g2p2g_gather(const ParticlesView&, const TableView&, const SortView&, const float*, int32_t, float, float, float*, Workspace&, hipStream_t s) { return touch(s); }

@@ -277,13 +277,13 @@ int32_t reserve(zsmpm_policy_s* p, int64_t n, int32_t T) {
   ZA(w.la_val, w.list_cap);
   ZA(w.lb_key, w.list_cap);
   ZA(w.lb_val, w.list_cap);
-  ZA(w.seg_heads, w.n_cap / 64 + 2);
-  ZA(w.seg_in, (size_t)w.n_cap + 64);
+  ZA(w.seg_count, w.n_cap / 256 + 1);
+  ZA(w.seg_in, (size_t)w.n_cap + 1024);
+  ZA(w.seg_where, (size_t)w.n_cap + 1024);
   ZA(w.seg_list, w.n_cap);
   ZA(w.seg_alt, w.n_cap);
   ZA(w.scnt, w.ts_cap);
   ZA(w.bcnt, w.ts_cap);
-  ZA(w.bpart, w.ts_cap / 1024 + 2);
   ZA(w.segoff, w.ts_cap);
   w.scan_words = 16384 + 64;
   ZA(w.scan_tmp, w.scan_words);
@@ -303,8 +303,8 @@ int32_t reserve(zsmpm_policy_s* p, int64_t n, int32_t T) {
   ZA(w.bitmap, (size_t)w.bm_words + 8);  // read in whole vectors
   ZA(w.bm_prefix, w.bm_words);
   ZA(w.bitmap_b, w.ts_cap / 32 + 10);
-  ZA(w.rank_a, rank_scratch_words(w.n_cap));
-  ZA(w.rank_b, rank_scratch_words(w.ts_cap));
+  ZA(w.rank_a, rank_scratch_words());
+  ZA(w.rank_b, rank_scratch_words());
   ZA(w.slot_block, w.ts_cap);
   ZA(w.dmask, 2 * (w.ts_cap / 32 + 1));
   p->own_cap_blocks = (int32_t)w.ts_cap;
@@ -482,6 +482,18 @@ int32_t ensure_bitmap(zsmpm_policy_s* p, uint64_t orders) {
   return ZSMPM_OK;
 }
 
+// P2G forms the stress itself from F unless the policy's learned closure or the
+// model's FP64 SVD provides it in a pass of its own.
+StressFrom stress_from(const Model& m, const ParticlesView& ps, bool closure) {
+  StressFrom st;
+  if (closure && m.kind == ZSMPM_DRUCKER_PRAGER && m.mu != 0.f) return st;
+  if (m.fp64_gap > 0.f) return st;
+  st.F = ps.F;
+  st.store_lj = m.kind == ZSMPM_DRUCKER_PRAGER;
+  st.m = m;
+  return st;
+}
+
 int32_t run_buckets(zsmpm_policy_s* p, const TableView& t, const ParticlesView& ps, float dx, SortView& sv) {
   return from_hip(bucket_sort(t, p->ws, ps.x, ps.n, dx, 4, -2, 0.5f, sv, p->stream));
 }
@@ -550,11 +562,19 @@ int32_t run_substep(zsmpm_policy_s* pol, const zsmpm_model* model, const zsmpm_p
     CellScope(Workspace& w_, bool on) : w(w_) { w.cell = on; }
     ~CellScope() { w.cell = false; }
   } cell_scope(ws, cell);
-  // The stress pass reads F and logJp and writes ws.contrib; the sparsity
-  // stages read x only. It runs on the side stream beside them and P2G waits
-  // for both.
+  // P2G forms the stress from F. Where a pass of its own does (the closure,
+  // the FP64 SVD), it reads F and logJp and writes ws.contrib; the sparsity
+  // stages read x only, so it runs on the side stream beside them and P2G
+  // waits for both.
+  StressFrom st;
+  const bool cached = chain && chain->cached_stress;
+  if (!cached && !multi) st = stress_from(m, ps, pol->closure_on);
+  if (!cached && multi && !ss->fp64) {
+    st.F = ps.F;
+    st.store_lj = true;
+  }
   SideFork side(pol);
-  if (!chain || !chain->cached_stress) {
+  if (!cached && !st.F) {
     ZS_HIP(ensure_side(pol));
     ZS_HIP(side.fork());
     StageScope sc(pol, ZSMPM_STAGE_STRESS, pol->side);
@@ -588,7 +608,7 @@ int32_t run_substep(zsmpm_policy_s* pol, const zsmpm_model* model, const zsmpm_p
     // v = (mv + rhs)/m convention), so the update must not add channels 4..6
     StageScope sc(pol, ZSMPM_STAGE_P2G);
     ZS_HIP(zsmpm::p2g_scatter(ps, t, sv, grid->data, grid->capacity_blocks, dt, dx, true, ws, s,
-                              /*reset_queue=*/false, ss));
+                              /*reset_queue=*/false, ss, st));
   }
   {
     StageScope sc(pol, ZSMPM_STAGE_GRID_UPDATE);
@@ -792,6 +812,7 @@ int32_t upload_scenes(zsmpm_policy_s* pol, const zsmpm_batch_scene* sc, int32_t 
     pol->scene_bytes.swap(bytes);
   }
   out.n = ns;
+  for (const SceneParams& p : params) out.fp64 = out.fp64 || p.model.fp64_gap > 0.f;
   out.p = pol->scene_p;
   out.first = pol->scene_first;
   return ZSMPM_OK;
@@ -1133,14 +1154,15 @@ int32_t zsmpm_p2g__rocm(zsmpm_policy pol, const zsmpm_model* model, const zsmpm_
     StageScope sc(pol, ZSMPM_STAGE_BUCKET_SORT);
     ZS_TRY(run_buckets(pol, t, ps, grid->dx, sv));
   }
-  {
+  const StressFrom st = stress_from(m, ps, pol->closure_on);
+  if (!st.F) {
     StageScope sc(pol, ZSMPM_STAGE_STRESS);
     ZS_HIP(zsmpm::stress(m, ps, pol->ws, pol->stream, pol->closure_on ? &pol->closure : nullptr));
   }
   StageScope sc(pol, ZSMPM_STAGE_P2G);
   ZS_HIP(block_neighbours(t, pol->ws, pol->stream));
-  return from_hip(
-      zsmpm::p2g_scatter(ps, t, sv, grid->data, grid->capacity_blocks, dt, grid->dx, false, pol->ws, pol->stream));
+  return from_hip(zsmpm::p2g_scatter(ps, t, sv, grid->data, grid->capacity_blocks, dt, grid->dx, false, pol->ws,
+                                     pol->stream, true, nullptr, st));
 }
 
 int32_t zsmpm_grid_update__rocm(zsmpm_policy pol, const zsmpm_grid* grid, const zsmpm_table* table, float dt,
@@ -1208,14 +1230,15 @@ int32_t zsmpm_p2c2g__rocm(zsmpm_policy pol, const zsmpm_model* model, const zsmp
     StageScope sc(pol, ZSMPM_STAGE_BUCKET_SORT);
     ZS_TRY(run_buckets(pol, t, ps, grid->dx, sv));
   }
-  {
+  const StressFrom st = stress_from(m, ps, false);
+  if (!st.F) {
     StageScope sc(pol, ZSMPM_STAGE_STRESS);
     ZS_HIP(zsmpm::stress(m, ps, pol->ws, pol->stream));
   }
   StageScope sc(pol, ZSMPM_STAGE_P2G);
   ZS_HIP(block_neighbours(t, pol->ws, pol->stream));
-  return from_hip(
-      zsmpm::p2c2g_scatter(ps, t, sv, grid->data, grid->capacity_blocks, dt, grid->dx, pol->ws, pol->stream));
+  return from_hip(zsmpm::p2c2g_scatter(ps, t, sv, grid->data, grid->capacity_blocks, dt, grid->dx, pol->ws,
+                                       pol->stream, st));
 }
 
 int32_t zsmpm_g2c2p__rocm(zsmpm_policy pol, const zsmpm_particles* particles, const zsmpm_table* table,
@@ -1335,17 +1358,23 @@ static int32_t run_g2p2g(zsmpm_policy_s* pol, const Model& m, const ParticlesVie
     ZS_HIP(block_neighbours(t, pol->ws, s));
   }
   ZS_HIP(g2p2g_gather(ps, t, sv, v, grid->capacity_blocks, dt, grid->dx, Fn, pol->ws, s));
-  // the model's vol P F^T of the updated F into the workspace's stress array
+  // the scatter forms the model's vol P F^T of the updated F (logJp is read
+  // and left); with the FP64 SVD on, the stress pass writes it to the
+  // workspace first, on a copy of logJp
   ParticlesView pf = ps;
   pf.F = Fn;
-  if (m.kind == 1) {
-    if (ps.n > 0)
-      ZS_HIP(hipMemcpyAsync(lj, ps.logJp, sizeof(float) * (size_t)ps.n, hipMemcpyDeviceToDevice, s));
-    pf.logJp = lj;
+  StressFrom st = stress_from(m, pf, false);
+  st.store_lj = false;
+  if (!st.F) {
+    if (m.kind == 1) {
+      if (ps.n > 0)
+        ZS_HIP(hipMemcpyAsync(lj, ps.logJp, sizeof(float) * (size_t)ps.n, hipMemcpyDeviceToDevice, s));
+      pf.logJp = lj;
+    }
+    ZS_HIP(zsmpm::stress(m, pf, pol->ws, s));
   }
-  ZS_HIP(zsmpm::stress(m, pf, pol->ws, s));
   ZS_HIP(grid_clear(tg, t.cnt, grid->capacity_blocks, s));
-  ZS_HIP(p2g_force_scatter(ps, t, sv, tg, grid->capacity_blocks, -1.f, grid->dx, pol->ws, s));
+  ZS_HIP(p2g_force_scatter(ps, t, sv, tg, grid->capacity_blocks, -1.f, grid->dx, pol->ws, s, st));
   ZS_HIP(implicit_add_force(tg, grid->capacity_blocks, t, r, s));
   return ZSMPM_OK;
 }

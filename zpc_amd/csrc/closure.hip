@@ -925,7 +925,7 @@ __global__ __launch_bounds__(256) void fallback_kernel(Model m, ParticlesView ps
     for (int k = 0; k < 9; ++k) F[k] = ps.F[9 * p + k];
     float lj = ps.logJp[p];
     bool f64 = false;
-    stress_sand(m, F, lj, PF, nullptr, f64);
+    stress_any(m, F, lj, PF, f64);
     ps.logJp[p] = lj;
 #pragma unroll
     for (int k = 0; k < 9; ++k) contrib[9 * p + k] = PF[k];

@@ -16,11 +16,11 @@
 //     (Shun & Blelloch, "Phase-Concurrent Hash Tables for Determinism",
 //     SPAA 2014), i.e. the layout zpc's seq_exec path produces.
 // The bucket sort is stable by particle index (zpc's seq semantics of
-// SpatiallyCount/SpatiallyDistribute): a wave cuts its 64 particles into
+// SpatiallyCount/SpatiallyDistribute): tiles of 1,024 particles are cut into
 // segments of equal key; every segment takes a place in its bucket's list with
 // the one atomic that also counts it, and a workgroup per bucket orders the
 // list by first particle and writes the bucket's indices. No sort over the
-// whole set: the counts give the buckets, and a list has ~8 entries when the
+// whole set: the counts give the buckets, and a list has ~2 entries when the
 // particles are in bucket order (a few hundred when they are shuffled).
 // The substep's own build (build_begin .. build_place) numbers, places and
 // enlarges from one dedup hash and one clear, with no device-wide scan: 9
@@ -98,22 +98,21 @@ struct Dedup {
 __device__ __forceinline__ uint32_t dedup_home(uint64_t pk, uint32_t ts) { return (uint32_t)mix64(pk) & (ts - 1u); }
 
 // Finishes an insert whose look at slot s showed cur: probes on until the slot
-// is free or holds pk (ts probes in all), then lowers the slot's order; the
-// insert that claims a free slot marks it in `mask`. Returns the slot holding
-// pk, or ~0u when the scratch table is full. Plain loads come before the
-// atomics: keys are only ever added and orders only lowered, so a stale value
-// costs an atomic that was not needed and nothing else.
-__device__ __forceinline__ uint32_t dedup_finish(uint64_t pk, uint32_t order, uint32_t s, uint64_t cur,
-                                                 const Dedup& d, uint32_t* mask) {
+// is free or holds pk (ts probes in all); the insert that claims a free slot
+// marks it in `mask`. Returns the slot holding pk, or ~0u when the scratch
+// table is full. Plain loads come before the atomics: keys are only ever added,
+// so a stale value costs an atomic that was not needed and nothing else.
+__device__ __forceinline__ uint32_t dedup_finish(uint64_t pk, uint32_t s, uint64_t cur, const Dedup& d,
+                                                 uint32_t* mask) {
   for (uint32_t probe = 1;; ++probe) {
-    if (cur == pk) break;
+    if (cur == pk) return s;
     if (cur == kEmpty64) {
       cur = atomicCAS((unsigned long long*)&d.skey[s], (unsigned long long)kEmpty64, (unsigned long long)pk);
       if (cur == kEmpty64) {
         atomicOr(&mask[s >> 5], 1u << (s & 31u));
-        break;
+        return s;
       }
-      if (cur == pk) break;
+      if (cur == pk) return s;
     }
     if (probe >= d.ts) {
       atomicOr(d.err, kErrTableFull);
@@ -122,76 +121,152 @@ __device__ __forceinline__ uint32_t dedup_finish(uint64_t pk, uint32_t order, ui
     s = (s + 1u) & (d.ts - 1u);
     cur = d.skey[s];
   }
-  if (d.sorder[s] > order) atomicMin(&d.sorder[s], order);
-  return s;
+}
+
+// the slot's order lowered to `order` (orders are only lowered: a stale value
+// is never too low)
+__device__ __forceinline__ void dedup_order(uint32_t s, uint32_t order, const Dedup& d) {
+  if (s != ~0u && d.sorder[s] > order) atomicMin(&d.sorder[s], order);
 }
 
 __device__ __forceinline__ uint32_t dedup_insert(uint64_t pk, uint32_t order, const Dedup& d) {
-  const uint32_t s = dedup_home(pk, d.ts);
-  return dedup_finish(pk, order, s, d.skey[s], d, d.dmask);
+  uint32_t s = dedup_home(pk, d.ts);
+  s = dedup_finish(pk, s, d.skey[s], d, d.dmask);
+  dedup_order(s, order, d);
+  return s;
 }
 
-// The segments of a 64-particle group: bit l of heads is set where particle l
-// starts a segment (another key than particle l - 1's, or l = 0). Length of
-// the segment that starts at `lane`, cw particles in the group.
-__device__ __forceinline__ int segment_length(uint64_t heads, int lane, int cw) {
-  const uint64_t above = lane == 63 ? 0ull : heads >> (lane + 1);
-  const int next = above ? lane + __ffsll((long long)above) : cw;
-  return next - lane;
-}
-
-// Per group, its heads; per segment (the j-th of group g at 64 g + j), the
-// bucket it belongs to (a dedup slot or a block) and its place in that
-// bucket's list, from the atomic that counted it: `place` holds segments << 32
-// | particles per bucket.
+// The particles are cut into tiles of consecutive ones, and a tile into
+// segments of equal bucket. Per tile, the number of segments; per segment (the
+// j-th of the tile at its first particle's index + j) the bucket it belongs to (a dedup slot or a
+// block), its place in that bucket's list, from the atomic that counted it, and
+// where it lies in the tile (first | length << 16). `place` holds segments << 32
+// | particles per bucket. In bucket order a tile has ~3 segments and a bucket
+// ~2; one wave's 64 particles per segment cost four times the atomics (the
+// build's activation of 16M particles 136 us).
+constexpr int kWideTile = 4;  // items per thread: tiles of 1,024, or
+constexpr int kTightTile = 1; // of 256 below 2^21 particles, where workgroups are scarce
 struct Segments {
-  uint64_t* heads = nullptr;  // [groups]
-  uint2* in = nullptr;        // [64 groups]
+  uint32_t* count = nullptr;  // [tiles]
+  uint2* in = nullptr;        // [n, whole tiles]
+  uint32_t* where = nullptr;  // [n, whole tiles]
   uint64_t* place = nullptr;
 };
 
-// ComputeSparsity candidates: one per segment of a 64-particle group, by its
-// first particle (order = particle index). A wave takes kItems groups and
-// issues their x loads, then their first probes, together: the kernel is bound
-// by those round trips, not by bytes (one group per wave below 2^22 particles,
-// where waves are scarce). The dedup hash keeps the minimum order per key, so
-// the result does not depend on the order of the inserts. Inserting one lane
-// per segment, not per distinct key of the group, needs no loop over the
-// group's keys: 1M shuffled particles 143 -> 33 us, 16M in bucket order (where
-// the two are the same) 88 us either way. kSegs: the segments are
-// recorded for the bucket sort.
+// The segments of a tile from its particles' keys (item r of thread i is
+// particle r kThreads + i; `live` particles), listed in order: key and where
+// (first | length << 16); returns their number. A particle without a key (live
+// but out of range: kEmpty64) belongs to segments too.
+template <int kTileItems>
+struct TileLds {
+  static constexpr int kTile = kThreads * kTileItems;
+  uint64_t last[kTileItems][kThreads / kWave];
+  uint64_t heads[kTile / kWave];
+  uint64_t key[kTile];
+  uint32_t where[kTile];
+};
+template <int kTileItems>
+__device__ __forceinline__ uint32_t tile_segments(const uint64_t (&key)[kTileItems], int live,
+                                                  TileLds<kTileItems>& lds) {
+  const int lane = lane_id(), wave = uniform((int32_t)(threadIdx.x / kWave));
+  constexpr int kW = kThreads / kWave;
+#pragma unroll
+  for (int r = 0; r < kTileItems; ++r)
+    if (lane == kWave - 1) lds.last[r][wave] = key[r];
+  __syncthreads();
+  uint64_t heads[kTileItems];
+#pragma unroll
+  for (int r = 0; r < kTileItems; ++r) {
+    uint64_t prev = __shfl_up(key[r], 1, kWave);
+    const bool first = r == 0 && threadIdx.x == 0;
+    if (lane == 0 && !first) prev = wave > 0 ? lds.last[r][wave - 1] : lds.last[r > 0 ? r - 1 : 0][kW - 1];
+    heads[r] = ballot(r * kThreads + (int)threadIdx.x < live && (first || prev != key[r]));
+    if (lane == 0) lds.heads[r * kW + wave] = heads[r];
+  }
+  __syncthreads();
+  // lane q: heads before group q and the first head after it
+  constexpr int kGroups = TileLds<kTileItems>::kTile / kWave;
+  const uint64_t mq = lane < kGroups ? lds.heads[lane] : 0ull;
+  int before = __popcll(mq), next = live;
+  int first = mq ? lane * kWave + __ffsll((long long)mq) - 1 : live;
+#pragma unroll
+  for (int o = 1; o < kGroups; o <<= 1) {
+    const int u = __shfl_up(before, o, kWave), f = __shfl_down(first, o, kWave);
+    if (lane >= o) before += u;
+    if (lane + o < kGroups) first = min(first, f);
+  }
+  const uint32_t count = (uint32_t)__builtin_amdgcn_readlane(before, kGroups - 1);
+  before -= __popcll(mq);
+  const int after = __shfl_down(first, 1, kWave);
+  if (lane + 1 < kGroups) next = after;
+#pragma unroll
+  for (int r = 0; r < kTileItems; ++r) {
+    if (heads[r] == 0) continue;  // most groups start no segment
+    const int g = r * kW + wave, at = g * kWave + lane;
+    const uint64_t above = lane == 63 ? 0ull : heads[r] >> (lane + 1);
+    // read with the whole wave active: lane g holds group g's value
+    const int later = __builtin_amdgcn_readlane(next, g);
+    const int end = above ? at + __ffsll((long long)above) : later;
+    const int rank = __builtin_amdgcn_readlane(before, g) + __popcll(heads[r] & lanemask_lt());
+    if ((heads[r] >> lane) & 1ull) {
+      lds.key[rank] = key[r];
+      lds.where[rank] = (uint32_t)at | ((uint32_t)(end - at) << 16);
+    }
+  }
+  __syncthreads();
+  return count;
+}
+
+// ComputeSparsity candidates: one per segment of a tile, by its first particle
+// (order = particle index). The kernel is bound by dependent round trips, not
+// by bytes: a workgroup has its next tile's positions in flight while it
+// inserts this one's segments, and the first probes are issued together. The dedup
+// hash keeps the minimum order per key, so the result does not depend on the
+// order of the inserts. kSegs: the segments are recorded for the bucket sort.
 // kMulti (a batch, ss): particle p takes its scene's 1/dx, and its key is
 // shifted by the scene's offset (a key outside the scene's own range
 // [-512, 511) along axis 0 is a key-range error)
-template <bool kMulti, bool kSegs, int kItems>
+template <bool kMulti, bool kSegs, int kTileItems>
 __global__ __launch_bounds__(kThreads) void activate_kernel(const float* __restrict__ x, int64_t n,
                                                             float dxinv, int blockLen, int offset,
                                                             float disp, Dedup dd, Segments sg, SceneSet ss) {
+  constexpr int kTile = kThreads * kTileItems;
   uint32_t* err = dd.err;
-  const int64_t span = (int64_t)kThreads * kItems;
-  const int64_t stride = (int64_t)gridDim.x * span;
-  const int lane = lane_id();
+  const int64_t ntiles = (n + kTile - 1) / kTile;
   __shared__ int64_t sfirst[kMulti ? kMaxScenes + 1 : 1];
+  __shared__ TileLds<kTileItems> lds;
   if constexpr (kMulti) {
     for (int i = threadIdx.x; i <= ss.n; i += kThreads) sfirst[i] = ss.first[i];
     __syncthreads();
   }
-  for (int64_t base = (int64_t)blockIdx.x * span; base < n; base += stride) {
-    float cx[kItems], cy[kItems], cz[kItems];
+  float nx[kTileItems], ny[kTileItems], nz[kTileItems];  // the next tile's positions, in flight
+  auto load = [&](int64_t tile) {
 #pragma unroll
-    for (int r = 0; r < kItems; ++r) {
-      const int64_t p = base + (int64_t)r * kThreads + threadIdx.x;
-      cx[r] = cy[r] = cz[r] = 0.f;
+    for (int r = 0; r < kTileItems; ++r) {
+      const int64_t p = tile * kTile + (int64_t)r * kThreads + threadIdx.x;
+      nx[r] = ny[r] = nz[r] = 0.f;
       if (p < n) {
-        cx[r] = x[3 * p];
-        cy[r] = x[3 * p + 1];
-        cz[r] = x[3 * p + 2];
+        nx[r] = x[3 * p];
+        ny[r] = x[3 * p + 1];
+        nz[r] = x[3 * p + 2];
       }
     }
-    uint64_t pk[kItems], cur[kItems], heads[kItems];
-    uint32_t slot[kItems];
+  };
+  load(blockIdx.x);
+  for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    const int64_t base = tile * kTile;
+    const int live = (int)min((int64_t)kTile, n - base);
+    float cx[kTileItems], cy[kTileItems], cz[kTileItems];
 #pragma unroll
-    for (int r = 0; r < kItems; ++r) {
+    for (int r = 0; r < kTileItems; ++r) {
+      cx[r] = nx[r];
+      cy[r] = ny[r];
+      cz[r] = nz[r];
+    }
+    load(tile + gridDim.x);
+    uint64_t pk[kTileItems];
+#pragma unroll
+    for (int r = 0; r < kTileItems; ++r) {
       const int64_t p = base + (int64_t)r * kThreads + threadIdx.x;
       pk[r] = kEmpty64;
       if (p < n) {
@@ -212,42 +287,28 @@ __global__ __launch_bounds__(kThreads) void activate_kernel(const float* __restr
           atomicOr(err, kErrKeyRange);
         }
       }
-      const uint64_t left = __shfl_up(pk[r], 1, kWave);
-      const bool head = p < n && (lane == 0 || left != pk[r]);
-      heads[r] = ballot(head);
-      slot[r] = ~0u;
-      cur[r] = kEmpty64;
-      if (head && pk[r] != kEmpty64) {
-        slot[r] = dedup_home(pk[r], dd.ts);
-        cur[r] = dd.skey[slot[r]];
+    }
+    const uint32_t count = tile_segments(pk, live, lds);
+    for (uint32_t j = threadIdx.x; j < count; j += kThreads) {
+      const uint64_t key = lds.key[j];
+      const uint32_t w = lds.where[j], order = (uint32_t)(base + (w & 0xffffu));
+      uint32_t slot = ~0u, local = 0u;
+      if (key != kEmpty64) {
+        slot = dedup_home(key, dd.ts);
+        slot = dedup_finish(key, slot, dd.skey[slot], dd, dd.dmask);
+        dedup_order(slot, order, dd);
+        if (kSegs && slot != ~0u)
+          local = (uint32_t)(atomicAdd((unsigned long long*)&sg.place[slot],
+                                       (1ull << 32) | (unsigned long long)(w >> 16)) >>
+                             32);
+      }
+      if (kSegs) {
+        sg.in[base + j] = make_uint2(slot, local);
+        sg.where[base + j] = w;
       }
     }
-#pragma unroll
-    for (int r = 0; r < kItems; ++r) {
-      const int64_t p = base + (int64_t)r * kThreads + threadIdx.x;
-      if (slot[r] != ~0u) slot[r] = dedup_finish(pk[r], (uint32_t)p, slot[r], cur[r], dd, dd.dmask);
-    }
-    if constexpr (kSegs) {
-      uint32_t local[kItems];
-#pragma unroll
-      for (int r = 0; r < kItems; ++r) {
-        const int64_t g64 = base + (int64_t)r * kThreads + threadIdx.x - lane;  // the group's first particle
-        const int cw = (int)min((int64_t)kWave, n - g64);
-        local[r] = 0;
-        if (slot[r] != ~0u)
-          local[r] = (uint32_t)(atomicAdd((unsigned long long*)&sg.place[slot[r]],
-                                          (1ull << 32) | (unsigned long long)segment_length(heads[r], lane, cw)) >>
-                                32);
-      }
-#pragma unroll
-      for (int r = 0; r < kItems; ++r) {
-        const int64_t g64 = base + (int64_t)r * kThreads + threadIdx.x - lane;
-        if (g64 >= n) continue;
-        if (lane == 0) sg.heads[g64 >> 6] = heads[r];
-        if ((heads[r] >> lane) & 1ull)
-          sg.in[g64 + __popcll(heads[r] & lanemask_lt())] = make_uint2(slot[r], local[r]);
-      }
-    }
+    if (kSegs && threadIdx.x == 0) sg.count[tile] = count;
+    __syncthreads();
   }
 }
 
@@ -457,49 +518,61 @@ __global__ void query_kernel(TableView t, const int32_t* __restrict__ keys, int6
 }
 
 // ------------------------------------------------------- the substep's build
-// Ranks among set bits of a bitmap of orders without a scan: counts of the set
-// bits per 2^10, 2^17 and 2^24 orders (c1, c2, c3), added to as the bits are
-// set. rank(o) = c3 before o's 2^24 group + c2 before its 2^17 group in that +
-// c1 before its 2^10 group in that + the bits before it there: at most 32
-// words and 3 x 128 counts, read by 8 lanes per key.
+// Ranks among the set bits of a bitmap of orders: the bits are counted per
+// 2^shift orders as they are set (c1, at most kRankGroups counts, whose prefix
+// every workgroup of the numbering forms in LDS for itself: no scan launches),
+// and 8 lanes per key add up the words before the order in its group (32 words
+// up to 2^24 orders). Coarser counts set with the bits made the marking slow:
+// 36K atomics on 128 adjacent counters take 40 us.
+constexpr int kRankGroups = 12288;  // 48 KB of LDS
 struct Ranks {
   uint32_t* bitmap = nullptr;
   uint32_t* c1 = nullptr;
-  uint32_t* c2 = nullptr;
-  uint32_t* c3 = nullptr;
   uint32_t words = 0;  // of the bitmap
+  int32_t shift = 10;
+  int32_t groups = 0;  // of c1
 };
-constexpr int kR1 = 10, kR2 = 17, kR3 = 24;
-// entries of a count level, a whole number of vectors past the last one
-inline uint64_t rank_pad(uint64_t last) { return (last + 1 + 7) & ~(uint64_t)3; }
 
-// h3: the workgroup's own counts per 2^24 orders (a few addresses for the whole
-// launch: 36K atomics on one took 0.4 ms)
-__device__ __forceinline__ void rank_mark(const Ranks& r, uint32_t o, uint32_t* h3) {
+__device__ __forceinline__ void rank_mark(const Ranks& r, uint32_t o) {
   if ((o >> 5) >= r.words) return;  // reported where the rank is taken
   atomicOr(&r.bitmap[o >> 5], 1u << (o & 31u));
-  atomicAdd(&r.c1[o >> kR1], 1u);
-  atomicAdd(&r.c2[o >> kR2], 1u);
-  if (r.words > (1u << (kR3 - 5)) + 1u) atomicAdd(&h3[o >> kR3], 1u);
+  atomicAdd(&r.c1[o >> r.shift], 1u);
 }
 
-__device__ __forceinline__ uint32_t sum_range(const uint32_t* __restrict__ a, uint32_t lo, uint32_t hi, int j) {
-  // this lane's share (every 8th group of 4) of a[lo, hi), lo a multiple of 4
-  uint32_t s = 0;
-  for (uint32_t i = lo + 4 * j; i < hi; i += 32) {
-    const uint4 q = *reinterpret_cast<const uint4*>(a + i);  // the arrays are padded to whole vectors
-    s += q.x + (i + 1 < hi ? q.y : 0u) + (i + 2 < hi ? q.z : 0u) + (i + 3 < hi ? q.w : 0u);
+// exclusive prefix of c1 into lds[0, groups)
+__device__ __forceinline__ void rank_prefix(const Ranks& r, uint32_t* lds, uint32_t* wsum) {
+  const int lane = lane_id(), wave = threadIdx.x / kWave;
+  uint32_t carry = 0;
+  for (int base = 0; base < r.groups; base += 4 * kThreads) {  // uniform across the workgroup
+    const int i = base + 4 * threadIdx.x;
+    uint4 q = make_uint4(0u, 0u, 0u, 0u);
+    if (i < r.groups) q = *reinterpret_cast<const uint4*>(r.c1 + i);  // padded with zeros to a whole vector
+    const uint32_t mine = q.x + q.y + q.z + q.w;
+    uint32_t inc = mine;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const uint32_t u = __shfl_up(inc, o, kWave);
+      if (lane >= o) inc += u;
+    }
+    if (lane == kWave - 1) wsum[wave] = inc;
+    __syncthreads();
+    uint32_t run = carry + inc - mine;
+#pragma unroll
+    for (int w = 0; w < kThreads / kWave; ++w) {
+      run += w < wave ? wsum[w] : 0u;
+      carry += wsum[w];
+    }
+    if (i < r.groups) *reinterpret_cast<uint4*>(lds + i) = make_uint4(run, run + q.x, run + q.x + q.y, run + q.x + q.y + q.z);
+    __syncthreads();
   }
-  return s;
 }
 
 // set bits before order o; called by the 8 lanes of a key's group (j = lane & 7)
-__device__ __forceinline__ uint32_t rank_below(const Ranks& r, uint32_t o, int j) {
+__device__ __forceinline__ uint32_t rank_below(const Ranks& r, const uint32_t* lds, uint32_t o, int j) {
   uint32_t s = 0;
-  const uint32_t w0 = (o >> kR1) << (kR1 - 5), w1 = o >> 5;
-  const uint32_t i = w0 + 4 * j;
-  if (i <= w1) {
-    const uint4 q = *reinterpret_cast<const uint4*>(r.bitmap + i);
+  const uint32_t w0 = (o >> r.shift) << (r.shift - 5), w1 = o >> 5;
+  for (uint32_t i = w0 + 4 * j; i <= w1; i += 32) {
+    const uint4 q = *reinterpret_cast<const uint4*>(r.bitmap + i);  // padded to a whole vector
     const uint32_t v[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -507,12 +580,9 @@ __device__ __forceinline__ uint32_t rank_below(const Ranks& r, uint32_t o, int j
       s += (uint32_t)__popc(w < w1 ? v[k] : (w == w1 ? v[k] & ((1u << (o & 31u)) - 1u) : 0u));
     }
   }
-  s += sum_range(r.c1, (o >> kR2) << (kR2 - kR1), o >> kR1, j);
-  s += sum_range(r.c2, (o >> kR3) << (kR3 - kR2), o >> kR2, j);
-  s += sum_range(r.c3, 0, o >> kR3, j);
 #pragma unroll
   for (int d = 1; d < 8; d <<= 1) s += __shfl_xor(s, d, kWave);
-  return s;
+  return lds[o >> r.shift] + s;
 }
 
 // Everything the build reads before it writes it, in one launch.
@@ -554,8 +624,7 @@ __global__ __launch_bounds__(kThreads) void build_collect_kernel(const uint32_t*
                                                                  uint32_t* count, uint32_t* __restrict__ lorder,
                                                                  uint32_t* __restrict__ lslot) {
   __shared__ uint32_t buf[kWave * 32];
-  __shared__ uint32_t total, base, h3[1u << (32 - kR3)];
-  for (uint32_t i = threadIdx.x; i < (1u << (32 - kR3)); i += kThreads) h3[i] = 0u;
+  __shared__ uint32_t total, base;
   const uint32_t w = blockIdx.x * kWave + threadIdx.x;
   if (threadIdx.x < kWave) {
     uint32_t bits = w < nw ? mask[w] : 0u;
@@ -579,14 +648,9 @@ __global__ __launch_bounds__(kThreads) void build_collect_kernel(const uint32_t*
   __syncthreads();
   for (uint32_t i = threadIdx.x; i < total; i += kThreads) {
     const uint32_t s = buf[i], o = sorder[s];
-    rank_mark(rk, o, h3);
+    rank_mark(rk, o);
     lorder[base + i] = o;
     lslot[base + i] = s;
-  }
-  if (rk.words > (1u << (kR3 - 5)) + 1u) {
-    __syncthreads();
-    for (uint32_t i = threadIdx.x; i < (1u << (32 - kR3)); i += kThreads)
-      if (h3[i]) atomicAdd(&rk.c3[i], h3[i]);
   }
 }
 
@@ -594,16 +658,21 @@ __global__ __launch_bounds__(kThreads) void build_collect_kernel(const uint32_t*
 // kEnlarge (the particles' keys, first = 0): lane j also inserts the key's
 // j-th neighbour key + (j>>2, j>>1&1, j&1) -- EnlargeSparsity's loop order --
 // with order 8 b + j, and records its slot in nbr[8 b + j]: the 2^3 blocks the
-// bucket's stencils cover need no table probe later. bcnt receives the
-// bucket's segment and particle counts, part their sums per 1,024 blocks.
+// bucket's stencils cover need no table probe later. Only keys the particles
+// did not have take an order (mask marks those). bcnt receives the bucket's
+// segment and particle counts.
 template <bool kEnlarge>
 __global__ __launch_bounds__(kThreads) void build_number_kernel(const uint32_t* count, const uint32_t* first_count,
                                                                 const uint32_t* __restrict__ lorder,
                                                                 const uint32_t* __restrict__ lslot, Ranks rk,
                                                                 TableView t, Dedup dd, uint32_t* mask2,
                                                                 int32_t* slot_block, const uint64_t* scnt,
-                                                                uint64_t* bcnt, uint64_t* part, int32_t* nbr) {
+                                                                uint64_t* bcnt, int32_t* nbr) {
+  extern __shared__ uint32_t prefix[];  // [rk.groups], whole vectors
+  __shared__ uint32_t wsum[kThreads / kWave];
   const uint32_t nl = *count;
+  if ((int64_t)blockIdx.x * blockDim.x >= 8ll * nl) return;
+  rank_prefix(rk, prefix, wsum);
   const uint32_t first = kEnlarge ? 0u : *first_count;
   const int j = lane_id() & 7;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -613,52 +682,59 @@ __global__ __launch_bounds__(kThreads) void build_number_kernel(const uint32_t* 
       if (j == 0) atomicOr(dd.err, kErrCapacity);
       continue;
     }
-    const uint32_t rank = first + rank_below(rk, o, j);
+    int32_t k0, k1, k2;
+    unpack_key(dd.skey[sl], k0, k1, k2);
+    // the neighbour's first probe is in flight while the rank is taken
+    uint64_t pk = kEmpty64, cur = kEmpty64;
+    uint32_t s = ~0u;
+    if (kEnlarge && j != 0) {
+      const int32_t n0 = k0 + ((j >> 2) & 1), n1 = k1 + ((j >> 1) & 1), n2 = k2 + (j & 1);
+      if (key_packable(n0, n1, n2)) {
+        pk = pack_key(n0, n1, n2);
+        s = dedup_home(pk, dd.ts);
+        cur = dd.skey[s];
+      } else {
+        atomicOr(dd.err, kErrKeyRange);
+      }
+    }
+    const uint32_t rank = first + rank_below(rk, prefix, o, j);
     if (rank >= (uint32_t)t.T) {
       if (j == 0) atomicOr(dd.err, kErrTableFull);
       continue;
     }
-    int32_t k0, k1, k2;
-    unpack_key(dd.skey[sl], k0, k1, k2);
     if (j == 0) {
       slot_block[sl] = (int32_t)rank;
       if (kEnlarge) {
-        const uint64_t c = scnt[sl];
-        bcnt[rank] = c;
-        atomicAdd((unsigned long long*)&part[rank >> 10], (unsigned long long)c);
+        bcnt[rank] = scnt[sl];
         nbr[8 * (int64_t)rank] = (int32_t)sl;
       }
       place_block(t, rank, k0, k1, k2, dd.err);
     } else if (kEnlarge) {
-      k0 += (j >> 2) & 1;
-      k1 += (j >> 1) & 1;
-      k2 += j & 1;
-      int32_t r = -1;
-      if (!key_packable(k0, k1, k2)) {
-        atomicOr(dd.err, kErrKeyRange);
-      } else {
-        const uint64_t pk = pack_key(k0, k1, k2);
-        const uint32_t s = dedup_home(pk, dd.ts);
-        r = (int32_t)dedup_finish(pk, 8u * rank + (uint32_t)j, s, dd.skey[s], dd, mask2);
+      if (s != ~0u) {
+        s = dedup_finish(pk, s, cur, dd, mask2);
+        if (s != ~0u && !((dd.dmask[s >> 5] >> (s & 31u)) & 1u)) dedup_order(s, 8u * rank + (uint32_t)j, dd);
       }
-      nbr[8 * (int64_t)rank + j] = r;
+      nbr[8 * (int64_t)rank + j] = (int32_t)s;
     }
   }
 }
 
-// Bucket counts and offsets of every block (zero past the particles' blocks)
-// and the start of each bucket's segment list, from the counts per block and
-// their sums per 1,024: a workgroup adds up the sums before its blocks and
-// scans its own. bcnt, part: segments << 32 | particles.
-__device__ __forceinline__ void counts_scan(const uint64_t* __restrict__ bcnt, const uint64_t* __restrict__ part,
-                                            int32_t nb, const SortView& sv, uint32_t* __restrict__ segoff,
-                                            uint32_t* counters, uint64_t* lds) {
+// Bucket counts and offsets of the first nb blocks and the start of each
+// bucket's segment list, from the counts per block (segments << 32 |
+// particles): a workgroup adds up the counts before its 1,024 blocks and scans
+// its own (nb counts are at most a few hundred KB, in L2). The entries past nb
+// are filled by the emission.
+__device__ __forceinline__ void counts_scan(const uint64_t* __restrict__ bcnt, int32_t nb, const SortView& sv,
+                                            uint32_t* __restrict__ segoff, uint64_t* lds) {
   const int lane = lane_id(), wave = threadIdx.x / kWave;
-  const int64_t nchunk = ((int64_t)sv.cap_blocks + 1 + 1023) / 1024;
-  const int32_t nparts = (nb + 1023) / 1024;
+  const int64_t nchunk = ((int64_t)nb + 1023) / 1024;
   for (int64_t c = blockIdx.x; c < nchunk; c += gridDim.x) {
     uint64_t before = 0;
-    for (int32_t i = threadIdx.x; i < nparts && i < c; i += kThreads) before += part[i];
+#pragma unroll 4
+    for (int64_t i = 2 * (int64_t)threadIdx.x; i < c * 1024; i += 2 * kThreads) {
+      const ulonglong2 q = *reinterpret_cast<const ulonglong2*>(bcnt + i);
+      before += q.x + q.y;
+    }
 #pragma unroll
     for (int o = kWave / 2; o > 0; o >>= 1) before += __shfl_xor(before, o, kWave);
     uint64_t v[4], mine = 0;
@@ -685,12 +761,10 @@ __device__ __forceinline__ void counts_scan(const uint64_t* __restrict__ bcnt, c
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      if (b0 + k <= sv.cap_blocks) {
-        // the last entry past the buckets counts nothing
-        sv.counts[b0 + k] = b0 + k < sv.cap_blocks ? (int32_t)(uint32_t)v[k] : 0;
+      if (b0 + k < nb) {
+        sv.counts[b0 + k] = (int32_t)(uint32_t)v[k];
         sv.offsets[b0 + k] = (int32_t)(uint32_t)run;
-        if (b0 + k < nb) segoff[b0 + k] = (uint32_t)(run >> 32);
-        if (b0 + k == sv.cap_blocks) counters[kCtrRuns] = (uint32_t)(run >> 32);
+        segoff[b0 + k] = (uint32_t)(run >> 32);
       }
       run += v[k];
     }
@@ -704,8 +778,7 @@ __device__ __forceinline__ void counts_scan(const uint64_t* __restrict__ bcnt, c
 __global__ __launch_bounds__(kThreads) void build_finish_kernel(TableView t, uint32_t* counters, uint32_t* err,
                                                                 const int32_t* __restrict__ slot_block, uint32_t ts,
                                                                 int32_t* nbr, const uint64_t* __restrict__ bcnt,
-                                                                const uint64_t* __restrict__ part, SortView sv,
-                                                                uint32_t* segoff) {
+                                                                SortView sv, uint32_t* segoff) {
   __shared__ uint64_t lds[2 * (kThreads / kWave)];
   const int64_t na = min((int64_t)counters[kCtrList], (int64_t)t.T);
   const int64_t nb = min((int64_t)counters[kCtrList] + counters[kCtrListB], (int64_t)t.T);
@@ -735,7 +808,7 @@ __global__ __launch_bounds__(kThreads) void build_finish_kernel(TableView t, uin
     const uint32_t sl = (uint32_t)nbr[i];
     nbr[i] = sl < ts ? slot_block[sl] : -1;
   }
-  counts_scan(bcnt, part, (int32_t)min(na, (int64_t)sv.cap_blocks), sv, segoff, counters, lds);
+  counts_scan(bcnt, (int32_t)min(na, (int64_t)sv.cap_blocks), sv, segoff, lds);
 }
 
 // ------------------------------------------------------------ bucket sort
@@ -746,111 +819,117 @@ __global__ void zero_u32_kernel(uint32_t* p, int64_t n) {
 
 // The stand-alone bucket sort's segments: the block each one's key maps to,
 // from one table query per segment, counted per block.
+template <int kTileItems>
 __global__ __launch_bounds__(kThreads) void bucket_kernel(const float* __restrict__ x, int64_t n, float dxinv,
                                                           int blockLen, int offset, float disp, TableView t,
                                                           Segments sg, int32_t cap_blocks, uint32_t* err) {
-  const int lane = lane_id();
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < n; base += stride) {
-    const int64_t p = base + threadIdx.x;
-    const bool valid = p < n;
-    int32_t k0 = 0, k1 = 0, k2 = 0;
-    if (valid) block_key(x[3 * p], x[3 * p + 1], x[3 * p + 2], dxinv, blockLen, offset, disp, k0, k1, k2);
-    const int32_t q0 = __shfl_up(k0, 1, kWave), q1 = __shfl_up(k1, 1, kWave), q2 = __shfl_up(k2, 1, kWave);
-    const bool head = valid && (lane == 0 || q0 != k0 || q1 != k1 || q2 != k2);
-    const uint64_t heads = ballot(head);
-    const int64_t g64 = p - lane;
-    if (lane == 0 && valid) sg.heads[g64 >> 6] = heads;
-    if (!head) continue;
-    const int cw = (int)min((int64_t)kWave, n - g64);
-    int32_t b = table_find(t, k0, k1, k2);
-    if (b < 0) atomicOr(err, kErrMissingBlock);
-    if (b >= cap_blocks) {
-      atomicOr(err, kErrCapacity);
-      b = -1;
-    }
-    uint32_t local = 0;
-    if (b >= 0)
-      local = (uint32_t)(atomicAdd((unsigned long long*)&sg.place[b],
-                                   (1ull << 32) | (unsigned long long)segment_length(heads, lane, cw)) >>
-                         32);
-    sg.in[g64 + __popcll(heads & lanemask_lt())] = make_uint2((uint32_t)b, local);
-  }
-}
-
-// sums of the counts per 1,024 blocks
-__global__ __launch_bounds__(kThreads) void counts_part_kernel(const uint64_t* __restrict__ bcnt, const int32_t* nblocks,
-                                                               int32_t cap, uint64_t* part) {
-  __shared__ uint64_t lds[kThreads / kWave];
-  const int32_t nb = min(*nblocks, cap);
-  const int32_t nparts = (nb + 1023) / 1024;
-  for (int32_t c = blockIdx.x; c < nparts; c += gridDim.x) {
-    uint64_t s = 0;
-    for (int32_t b = c * 1024 + threadIdx.x; b < min(nb, (c + 1) * 1024); b += kThreads) s += bcnt[b];
+  constexpr int kTile = kThreads * kTileItems;
+  __shared__ TileLds<kTileItems> lds;
+  const int64_t ntiles = (n + kTile - 1) / kTile;
+  for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    const int64_t base = tile * kTile;
+    const int live = (int)min((int64_t)kTile, n - base);
+    uint64_t pk[kTileItems];
 #pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, kWave);
-    if (lane_id() == 0) lds[threadIdx.x / kWave] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      uint64_t g = 0;
-      for (int w = 0; w < kThreads / kWave; ++w) g += lds[w];
-      part[c] = g;
+    for (int r = 0; r < kTileItems; ++r) {
+      const int64_t p = base + (int64_t)r * kThreads + threadIdx.x;
+      int32_t k0 = 0, k1 = 0, k2 = 0;
+      if (p < n) block_key(x[3 * p], x[3 * p + 1], x[3 * p + 2], dxinv, blockLen, offset, disp, k0, k1, k2);
+      // no key the table can hold is out of the packed range
+      pk[r] = p < n && key_packable(k0, k1, k2) ? pack_key(k0, k1, k2) : kEmpty64;
     }
+    const uint32_t count = tile_segments(pk, live, lds);
+    for (uint32_t j = threadIdx.x; j < count; j += kThreads) {
+      const uint64_t key = lds.key[j];
+      const uint32_t w = lds.where[j];
+      int32_t b = -1;
+      if (key != kEmpty64) {
+        int32_t k0, k1, k2;
+        unpack_key(key, k0, k1, k2);
+        b = table_find(t, k0, k1, k2);
+      }
+      if (b < 0) atomicOr(err, kErrMissingBlock);
+      if (b >= cap_blocks) {
+        atomicOr(err, kErrCapacity);
+        b = -1;
+      }
+      uint32_t local = 0;
+      if (b >= 0)
+        local = (uint32_t)(atomicAdd((unsigned long long*)&sg.place[b],
+                                     (1ull << 32) | (unsigned long long)(w >> 16)) >>
+                           32);
+      sg.in[base + j] = make_uint2((uint32_t)b, local);
+      sg.where[base + j] = w;
+    }
+    if (threadIdx.x == 0) sg.count[tile] = count;
     __syncthreads();
   }
 }
 
 __global__ __launch_bounds__(kThreads) void counts_scan_kernel(const uint64_t* __restrict__ bcnt,
-                                                               const uint64_t* __restrict__ part,
                                                                const int32_t* nblocks, int32_t cap, SortView sv,
-                                                               uint32_t* segoff, uint32_t* counters) {
+                                                               uint32_t* segoff) {
   __shared__ uint64_t lds[2 * (kThreads / kWave)];
-  counts_scan(bcnt, part, min(min(*nblocks, cap), sv.cap_blocks), sv, segoff, counters, lds);
+  counts_scan(bcnt, min(min(*nblocks, cap), sv.cap_blocks), sv, segoff, lds);
 }
 
 // Every segment into its bucket's list: first particle | length << 32. A wave
-// takes 8 groups, their loads in flight together (three dependent round trips).
-// slot_block: the segments name dedup slots; null: blocks.
-constexpr int kEmitGroups = 8;
-__global__ __launch_bounds__(kThreads) void segment_emit_kernel(Segments sg, int64_t n,
+// takes a tile, a lane a segment. slot_block: the segments name dedup slots;
+// null: blocks. Also the counts and offsets past the counted blocks.
+__global__ __launch_bounds__(kThreads) void segment_emit_kernel(Segments sg, int64_t n, int32_t tile_size,
                                                                 const int32_t* __restrict__ slot_block, uint32_t ts,
                                                                 const uint32_t* __restrict__ segoff,
-                                                                const int32_t* nblocks, int32_t cap,
-                                                                uint64_t* __restrict__ list, uint32_t* err) {
+                                                                const uint64_t* __restrict__ bcnt,
+                                                                const int32_t* nblocks, int32_t cap, SortView sv,
+                                                                uint64_t* __restrict__ list, uint32_t* counters,
+                                                                uint32_t* err) {
   const int lane = lane_id();
-  const int64_t ngroups = (n + kWave - 1) / kWave;
+  const int64_t ntiles = (n + tile_size - 1) / tile_size;
   const int32_t nb = min(*nblocks, cap);
+  {
+    const int32_t total = nb > 0 ? sv.offsets[nb - 1] + sv.counts[nb - 1] : 0;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = nb + blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i <= sv.cap_blocks; i += stride) {
+      sv.counts[i] = 0;
+      sv.offsets[i] = total;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+      counters[kCtrRuns] = nb > 0 ? segoff[nb - 1] + (uint32_t)(bcnt[nb - 1] >> 32) : 0u;
+  }
   const int64_t nwaves = (int64_t)gridDim.x * (kThreads / kWave);
-  for (int64_t g0 = ((int64_t)blockIdx.x * (kThreads / kWave) + threadIdx.x / kWave) * kEmitGroups; g0 < ngroups;
-       g0 += nwaves * kEmitGroups) {
-    uint64_t heads[kEmitGroups];
-    uint2 e[kEmitGroups];
-    int32_t b[kEmitGroups];
+  constexpr int kAhead = 4;
+  for (int64_t tile = (int64_t)blockIdx.x * (kThreads / kWave) + threadIdx.x / kWave; tile < ntiles; tile += nwaves) {
+    const int64_t base = tile * tile_size;
+    const uint32_t count = min(sg.count[tile], (uint32_t)tile_size);
+    for (uint32_t j0 = 0; j0 < count; j0 += kAhead * kWave) {
+      uint2 e[kAhead];
+      uint32_t w[kAhead], at[kAhead];
+      int32_t b[kAhead];
 #pragma unroll
-    for (int k = 0; k < kEmitGroups; ++k) heads[k] = g0 + k < ngroups ? sg.heads[g0 + k] : 0ull;
+      for (int k = 0; k < kAhead; ++k) {
+        const uint32_t j = j0 + k * kWave + lane;
+        e[k] = make_uint2(~0u, 0u);
+        w[k] = 0u;
+        if (j < count) {
+          e[k] = sg.in[base + j];
+          w[k] = sg.where[base + j];
+        }
+      }
 #pragma unroll
-    for (int k = 0; k < kEmitGroups; ++k) {
-      e[k] = make_uint2(~0u, 0u);
-      if ((heads[k] >> lane) & 1ull) e[k] = sg.in[(g0 + k) * kWave + __popcll(heads[k] & lanemask_lt())];
-    }
+      for (int k = 0; k < kAhead; ++k) {
+        b[k] = (int32_t)e[k].x;
+        if (slot_block) b[k] = e[k].x < ts ? slot_block[e[k].x] : -1;
+      }
 #pragma unroll
-    for (int k = 0; k < kEmitGroups; ++k) {
-      b[k] = (int32_t)e[k].x;
-      if (slot_block) b[k] = e[k].x < ts ? slot_block[e[k].x] : -1;
-    }
-    uint32_t at[kEmitGroups];
+      for (int k = 0; k < kAhead; ++k) {
+        const bool ok = b[k] >= 0 && b[k] < nb;
+        at[k] = ok ? segoff[b[k]] + e[k].y : ~0u;
+        if (slot_block && !ok && w[k] != 0u) atomicOr(err, b[k] < 0 ? kErrMissingBlock : kErrCapacity);
+      }
 #pragma unroll
-    for (int k = 0; k < kEmitGroups; ++k) {
-      const bool ok = b[k] >= 0 && b[k] < nb;
-      at[k] = ok ? segoff[b[k]] + e[k].y : ~0u;
-      if (slot_block && !ok && ((heads[k] >> lane) & 1ull)) atomicOr(err, b[k] < 0 ? kErrMissingBlock : kErrCapacity);
-    }
-#pragma unroll
-    for (int k = 0; k < kEmitGroups; ++k) {
-      if (at[k] == ~0u || (int64_t)at[k] >= n) continue;
-      const int64_t g64 = (g0 + k) * kWave;
-      const int cw = (int)min((int64_t)kWave, n - g64);
-      list[at[k]] = (uint64_t)(uint32_t)(g64 + lane) | ((uint64_t)segment_length(heads[k], lane, cw) << 32);
+      for (int k = 0; k < kAhead; ++k)
+        if (at[k] != ~0u && (int64_t)at[k] < n)
+          list[at[k]] = (uint64_t)(uint32_t)(base + (w[k] & 0xffffu)) | ((uint64_t)(w[k] >> 16) << 32);
     }
   }
 }
@@ -862,11 +941,12 @@ __global__ __launch_bounds__(kThreads) void segment_emit_kernel(Segments sg, int
 // kPlaceLds: a bitonic sort in LDS and a scan of the lengths. Beyond (thousands
 // of particles per bucket, interleaved): a radix sort of the list in global
 // memory, 8 bits of the first particle at a time, `alt` the other buffer.
-constexpr int kPlaceLds = 4096;
+constexpr int kPlaceLds = 2048;  // 16 KB, eight workgroups per CU
 
+// first, step: this thread's share of the segment
 __device__ __forceinline__ void write_segment(int32_t* __restrict__ indices, int64_t n, int64_t at, uint32_t start,
-                                              uint32_t len, int lane) {
-  if ((uint32_t)lane < len && at + lane < n) indices[at + lane] = (int32_t)(start + lane);
+                                              uint32_t len, uint32_t first, uint32_t step) {
+  for (uint32_t q = first; q < len && at + q < n; q += step) indices[at + q] = (int32_t)(start + q);
 }
 
 // exclusive scan of one value per thread across the workgroup
@@ -901,12 +981,14 @@ __global__ __launch_bounds__(kThreads) void segment_place_kernel(const uint64_t*
   const int lane = lane_id(), wave = threadIdx.x / kWave;
   const int32_t nb = min(min(*nblocks, cap), sv.cap_blocks);
   for (int32_t b = blockIdx.x; b < nb; b += gridDim.x) {
-    const uint32_t R = (uint32_t)(bcnt[b] >> 32);
+    const uint64_t both = bcnt[b];
+    const uint32_t R = (uint32_t)(both >> 32), cnt = (uint32_t)both;
     const int64_t off = sv.offsets[b];
     const uint32_t s0 = segoff[b];
     if (R == 0 || (int64_t)s0 + R > n) continue;
     if (R <= (uint32_t)kWave) {
-      // every wave orders the list for itself and writes every fourth segment
+      // every wave orders the list for itself; short segments go to one wave
+      // each, long ones to the whole workgroup
       const uint64_t me = (uint32_t)lane < R ? list[s0 + lane] : ~0ull;
       const uint32_t start = (uint32_t)me, len = (uint32_t)lane < R ? (uint32_t)(me >> 32) : 0u;
       uint32_t before = 0;
@@ -915,11 +997,12 @@ __global__ __launch_bounds__(kThreads) void segment_place_kernel(const uint64_t*
         const uint32_t kl = (uint32_t)__builtin_amdgcn_readlane((int)len, (int)k);
         before += ks < start ? kl : 0u;
       }
-      for (uint32_t k = wave; k < R; k += kThreads / kWave) {
+      const bool wide = cnt >= 64u * R;
+      for (uint32_t k = wide ? 0 : wave; k < R; k += wide ? 1 : kThreads / kWave) {
         const uint32_t ks = (uint32_t)__builtin_amdgcn_readlane((int)start, (int)k);
         const uint32_t kl = (uint32_t)__builtin_amdgcn_readlane((int)len, (int)k);
         const uint32_t kb = (uint32_t)__builtin_amdgcn_readlane((int)before, (int)k);
-        write_segment(sv.indices, n, off + kb, ks, kl, lane);
+        write_segment(sv.indices, n, off + kb, ks, kl, wide ? threadIdx.x : lane, wide ? kThreads : kWave);
       }
       continue;
     }
@@ -946,7 +1029,7 @@ __global__ __launch_bounds__(kThreads) void segment_place_kernel(const uint64_t*
         }
       }
       uint32_t carry = 0;
-      const bool runs = (uint32_t)bcnt[b] >= 8u * R;  // long segments: a wave writes each
+      const bool runs = cnt >= 8u * R;  // long segments: a wave writes each
       for (uint32_t base = 0; base < R; base += kThreads) {  // uniform across the workgroup
         const uint32_t i = base + threadIdx.x;
         const uint64_t v = i < R ? seg[i] : 0ull;
@@ -957,7 +1040,7 @@ __global__ __launch_bounds__(kThreads) void segment_place_kernel(const uint64_t*
           for (int k = 0; k < kWave; ++k) {  // len 0 past the list
             const uint32_t kl = (uint32_t)__builtin_amdgcn_readlane((int)len, k);
             write_segment(sv.indices, n, off + (uint32_t)__builtin_amdgcn_readlane((int)at, k),
-                          (uint32_t)__builtin_amdgcn_readlane((int)start, k), kl, lane);
+                          (uint32_t)__builtin_amdgcn_readlane((int)start, k), kl, lane, kWave);
           }
         } else {
           for (uint32_t q = 0; q < len && off + at + q < n; ++q) sv.indices[off + at + q] = (int32_t)(start + q);
@@ -1073,30 +1156,40 @@ hipError_t table_clear(const TableView& t, Workspace& ws, hipStream_t s) {
 
 namespace {
 
-// the activation's insertion pass; particles per launch decide the groups per wave
+bool wide_tiles(int64_t n) { return n >= (int64_t)1 << 21; }
+int tile_size(int64_t n) { return kThreads * (wide_tiles(n) ? kWideTile : kTightTile); }
+// workgroups of a kernel that strides over the tiles: at most eight per CU of the 256 over wide ones
+int tile_groups(int64_t n) {
+  const int g = groups_for(n, tile_size(n));
+  return wide_tiles(n) && g > 2048 ? 2048 : g;
+}
+
+// the activation's insertion pass
 template <bool kSegs>
 void launch_activate(Workspace& ws, const float* x, int64_t n, float dx, int blockLen, int offset, float disp,
                      const Segments& sg, hipStream_t s, const SceneSet* ss) {
   const float dxinv = (float)1.0 / dx;
-  const bool wide = n >= (int64_t)1 << 22;
-  const int g = groups_for(n, kThreads * (wide ? 4 : 1));
-  const Dedup dd = dedup_of(ws);
-  if (ss && ss->n > 0) {
-    if (wide)
-      activate_kernel<true, kSegs, 4><<<g, kThreads, 0, s>>>(x, n, dxinv, blockLen, offset, disp, dd, sg, *ss);
-    else
-      activate_kernel<true, kSegs, 1><<<g, kThreads, 0, s>>>(x, n, dxinv, blockLen, offset, disp, dd, sg, *ss);
-  } else if (wide) {
-    activate_kernel<false, kSegs, 4><<<g, kThreads, 0, s>>>(x, n, dxinv, blockLen, offset, disp, dd, sg, SceneSet{});
-  } else {
-    activate_kernel<false, kSegs, 1><<<g, kThreads, 0, s>>>(x, n, dxinv, blockLen, offset, disp, dd, sg, SceneSet{});
-  }
+  const int g = tile_groups(n);
+  const bool multi = ss && ss->n > 0;
+  const SceneSet sset = multi ? *ss : SceneSet{};
+  auto launch = [&](auto kernel) {
+    kernel<<<g, kThreads, 0, s>>>(x, n, dxinv, blockLen, offset, disp, dedup_of(ws), sg, sset);
+  };
+  if (multi && wide_tiles(n))
+    launch(activate_kernel<true, kSegs, kWideTile>);
+  else if (multi)
+    launch(activate_kernel<true, kSegs, kTightTile>);
+  else if (wide_tiles(n))
+    launch(activate_kernel<false, kSegs, kWideTile>);
+  else
+    launch(activate_kernel<false, kSegs, kTightTile>);
 }
 
 Segments segments_of(const Workspace& ws, uint64_t* place) {
   Segments sg;
-  sg.heads = ws.seg_heads;
+  sg.count = ws.seg_count;
   sg.in = ws.seg_in;
+  sg.where = ws.seg_where;
   sg.place = place;
   return sg;
 }
@@ -1144,11 +1237,14 @@ namespace {
 // and the buckets' indices. slot_block as in segment_emit_kernel.
 hipError_t place_segments(Workspace& ws, int64_t n, const int32_t* slot_block, const int32_t* nblocks,
                           const SortView& out, hipStream_t s) {
-  const int64_t waves = (n + (int64_t)kWave * kEmitGroups - 1) / ((int64_t)kWave * kEmitGroups);
+  const int64_t tiles = (n + tile_size(n) - 1) / tile_size(n);
   const int32_t cap = out.cap_blocks < (int32_t)ws.ts_cap ? out.cap_blocks : (int32_t)ws.ts_cap;
-  segment_emit_kernel<<<groups_for(waves * kWave, kThreads), kThreads, 0, s>>>(
-      segments_of(ws, nullptr), n, slot_block, ws.ts_cap, ws.segoff, nblocks, cap, ws.seg_list, ws.err);
-  const int g = cap < 16384 ? cap : 16384;
+  const int ge = groups_for(tiles * kWave, kThreads), gc = groups_for((int64_t)cap + 1, kThreads * 4);
+  segment_emit_kernel<<<ge > gc ? ge : gc, kThreads, 0, s>>>(segments_of(ws, nullptr), n, tile_size(n), slot_block, ws.ts_cap,
+                                                             ws.segoff, ws.bcnt, nblocks, cap, out, ws.seg_list,
+                                                             ws.counters, ws.err);
+  if (n <= 0) return hipGetLastError();
+  const int g = cap < 32768 ? cap : 32768;
   segment_place_kernel<<<g, kThreads, 0, s>>>(ws.bcnt, ws.segoff, nblocks, cap, out, n, bits_for((uint64_t)n - 1),
                                               ws.seg_list, ws.seg_alt);
   return hipGetLastError();
@@ -1163,15 +1259,14 @@ hipError_t bucket_sort(const TableView& t, Workspace& ws, const float* x, int64_
   zero_u32_kernel<<<groups_for(2ll * ws.ts_cap, kThreads) < 2048 ? groups_for(2ll * ws.ts_cap, kThreads) : 2048,
                     kThreads, 0, s>>>((uint32_t*)ws.bcnt, 2ll * ws.ts_cap);
   const int32_t cap = out.cap_blocks < (int32_t)ws.ts_cap ? out.cap_blocks : (int32_t)ws.ts_cap;
-  if (n > 0)
-    bucket_kernel<<<groups_for(n, kThreads), kThreads, 0, s>>>(x, n, dxinv, blockLen, offset, disp, t,
-                                                               segments_of(ws, ws.bcnt), cap, ws.err);
-  const int gp = (cap + 1023) / 1024;
-  counts_part_kernel<<<gp < 1024 ? gp : 1024, kThreads, 0, s>>>(ws.bcnt, t.cnt, cap, ws.bpart);
-  const int gs = (out.cap_blocks + 1024) / 1024;
-  counts_scan_kernel<<<gs < 1024 ? gs : 1024, kThreads, 0, s>>>(ws.bcnt, ws.bpart, t.cnt, cap, out, ws.segoff,
-                                                                   ws.counters);
-  if (n <= 0) return hipGetLastError();
+  if (n > 0 && wide_tiles(n))
+    bucket_kernel<kWideTile><<<tile_groups(n), kThreads, 0, s>>>(x, n, dxinv, blockLen, offset, disp, t,
+                                                                 segments_of(ws, ws.bcnt), cap, ws.err);
+  else if (n > 0)
+    bucket_kernel<kTightTile><<<tile_groups(n), kThreads, 0, s>>>(x, n, dxinv, blockLen, offset, disp, t,
+                                                                  segments_of(ws, ws.bcnt), cap, ws.err);
+  const int gs = (cap + 1023) / 1024;
+  counts_scan_kernel<<<gs < 1024 ? gs : 1024, kThreads, 0, s>>>(ws.bcnt, t.cnt, cap, out, ws.segoff);
   return place_segments(ws, n, nullptr, t.cnt, out, s);
 }
 
@@ -1180,27 +1275,26 @@ namespace {
 
 // orders of the particles' keys are particle indices, those of the enlargement
 // candidates (8 b + j) lie below T while the particles' blocks fill at most T / 8
-Ranks ranks_a(const Workspace& ws, int64_t n) {
+Ranks ranks_of(uint32_t* bitmap, uint32_t* c1, uint64_t orders) {
   Ranks r;
-  r.bitmap = ws.bitmap;
-  r.c1 = ws.rank_a;
-  r.c2 = r.c1 + rank_pad(ws.n_cap >> kR1);
-  r.c3 = r.c2 + rank_pad(ws.n_cap >> kR2);
-  r.words = (uint32_t)((uint64_t)(n > 0 ? n : 1) / 32 + 1);
+  r.bitmap = bitmap;
+  r.c1 = c1;
+  r.words = (uint32_t)(orders / 32 + 1);
+  while ((((uint64_t)r.words * 32) >> r.shift) + 1 > (uint64_t)kRankGroups) ++r.shift;
+  r.groups = (int32_t)((((uint64_t)r.words * 32) >> r.shift) + 1);
   return r;
 }
+Ranks ranks_a(const Workspace& ws, int64_t n) { return ranks_of(ws.bitmap, ws.rank_a, (uint64_t)(n > 0 ? n : 1)); }
 Ranks ranks_b(const Workspace& ws, const TableView& t) {
-  Ranks r;
-  r.bitmap = ws.bitmap_b;
-  r.c1 = ws.rank_b;
-  r.c2 = r.c1 + rank_pad(ws.ts_cap >> kR1);
-  r.c3 = r.c2 + rank_pad(ws.ts_cap >> kR2);
-  const int32_t n0 = t.T / 8 > 0 ? t.T / 8 : 1;
-  r.words = (uint32_t)(8ull * (uint64_t)n0 / 32 + 1);
-  return r;
+  return ranks_of(ws.bitmap_b, ws.rank_b, 8ull * (uint64_t)(t.T / 8 > 0 ? t.T / 8 : 1));
 }
-int64_t rank_words(uint64_t orders) {
-  return (int64_t)(rank_pad(orders >> kR1) + rank_pad(orders >> kR2) + rank_pad(orders >> kR3));
+int64_t padded(int64_t groups) { return (groups + 3) & ~(int64_t)3; }
+// a workgroup of the numbering reads all of c1: few of them where there is much
+// of it (the LDS it fills also bounds them to two per CU then)
+int number_groups(const Ranks& r, uint32_t ts, int64_t most) {
+  const int g = groups_for(8ll * ts, kThreads);
+  const int cap = (int)(r.groups > 4096 ? 512 : most);
+  return g < cap ? g : cap;
 }
 int few(int64_t n, int most) {
   const int g = groups_for(n, kThreads);
@@ -1209,7 +1303,7 @@ int few(int64_t n, int most) {
 
 }  // namespace
 
-size_t rank_scratch_words(uint64_t orders) { return (size_t)rank_words(orders); }
+size_t rank_scratch_words() { return kRankGroups + 4; }
 
 hipError_t build_clear(const TableView& t, Workspace& ws, int64_t n, hipStream_t s) {
   ClearList c;
@@ -1229,10 +1323,9 @@ hipError_t build_clear(const TableView& t, Workspace& ws, int64_t n, hipStream_t
   add(ws.scnt, 2 * ts, 0u);
   add(ws.dmask, 2 * (ts / 32 + 1), 0u);  // both masks
   add(ws.bitmap, ranks_a(ws, n).words, 0u);
-  add(ws.rank_a, rank_words(ws.n_cap), 0u);
+  add(ws.rank_a, padded(ranks_a(ws, n).groups), 0u);
   add(ws.bitmap_b, ranks_b(ws, t).words, 0u);
-  add(ws.rank_b, rank_words(ws.ts_cap), 0u);
-  add(ws.bpart, 2 * (ts / 1024 + 2), 0u);
+  add(ws.rank_b, padded(ranks_b(ws, t).groups), 0u);
   build_clear_kernel<<<few(most / 4 + 1, 4096), kThreads, 0, s>>>(c, t, ws.counters);
   return hipGetLastError();
 }
@@ -1249,26 +1342,22 @@ hipError_t build_activate(const TableView& t, Workspace& ws, const float* x, int
 
 hipError_t build_enlarge(const TableView& t, Workspace& ws, int64_t n, const SortView& sv, hipStream_t s) {
   uint32_t* mask2 = ws.dmask + (ws.ts_cap / 32 + 1);
-  const int g = few(8ll * ws.ts_cap, 1024);
-  build_number_kernel<true><<<g, kThreads, 0, s>>>(ws.counters + kCtrList, nullptr, ws.la_key, ws.la_val,
-                                                   ranks_a(ws, n), t, dedup_of(ws), mask2, ws.slot_block, ws.scnt,
-                                                   ws.bcnt, ws.bpart, ws.nbr);
+  const Ranks ra = ranks_a(ws, n), rb = ranks_b(ws, t);
+  build_number_kernel<true><<<number_groups(ra, ws.ts_cap, 1024), kThreads, 4 * padded(ra.groups), s>>>(
+      ws.counters + kCtrList, nullptr, ws.la_key, ws.la_val, ra, t, dedup_of(ws), mask2, ws.slot_block, ws.scnt,
+      ws.bcnt, ws.nbr);
   const uint32_t nw = (ws.ts_cap + 31u) / 32u;
   build_collect_kernel<<<(int)((nw + kWave - 1) / kWave), kThreads, 0, s>>>(
-      mask2, nw, ws.sorder, ranks_b(ws, t), ws.counters + kCtrListB, ws.lb_key, ws.lb_val);
-  build_number_kernel<false><<<g, kThreads, 0, s>>>(ws.counters + kCtrListB, ws.counters + kCtrList, ws.lb_key,
-                                                    ws.lb_val, ranks_b(ws, t), t, dedup_of(ws), mask2, ws.slot_block,
-                                                    ws.scnt, ws.bcnt, ws.bpart, ws.nbr);
-  const int64_t chunks = ((int64_t)sv.cap_blocks + 1024) / 1024;
-  int gf = few(ws.ts_cap, 1024);
-  if (gf < chunks) gf = (int)(chunks < 1024 ? chunks : 1024);
-  build_finish_kernel<<<gf, kThreads, 0, s>>>(t, ws.counters, ws.err, ws.slot_block, ws.ts_cap, ws.nbr, ws.bcnt,
-                                              ws.bpart, sv, ws.segoff);
+      mask2, nw, ws.sorder, rb, ws.counters + kCtrListB, ws.lb_key, ws.lb_val);
+  build_number_kernel<false><<<number_groups(rb, ws.ts_cap, 256), kThreads, 4 * padded(rb.groups), s>>>(
+      ws.counters + kCtrListB, ws.counters + kCtrList, ws.lb_key, ws.lb_val, rb, t, dedup_of(ws), mask2,
+      ws.slot_block, ws.scnt, ws.bcnt, ws.nbr);
+  build_finish_kernel<<<few(ws.ts_cap, 1024), kThreads, 0, s>>>(t, ws.counters, ws.err, ws.slot_block, ws.ts_cap, ws.nbr, ws.bcnt, sv,
+                                              ws.segoff);
   return hipGetLastError();
 }
 
 hipError_t build_place(const TableView& t, Workspace& ws, int64_t n, const SortView& out, hipStream_t s) {
-  if (n <= 0) return hipSuccess;
   return place_segments(ws, n, ws.slot_block, reinterpret_cast<const int32_t*>(ws.counters + kCtrList), out, s);
 }
 

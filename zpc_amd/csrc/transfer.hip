@@ -266,20 +266,14 @@ __global__ __launch_bounds__(kThreads) void stress_kernel(Model m, ParticlesView
     }
     if (lane < cw) {
       bool f64 = false;
-      if (kKind == 0) {
-        stress_fixedcorotated(m, F, PF, f64);
-      } else if (kKind == 1) {
-        stress_sand(m, F, lj, PF, nullptr, f64);
-        ps.logJp[p] = lj;
+      if (kKind != 2) {
+        stress_any(m, F, lj, PF, f64);
+        if (kKind == 1) ps.logJp[p] = lj;
       } else {
         const Model ms = ss.p[scene_of_particle(sfirst, ss.n, p)].model;
-        if (ms.kind == 0) {
-          stress_fixedcorotated(ms, F, PF, f64);
-        } else {
-          lj = ps.logJp[p];
-          stress_sand(ms, F, lj, PF, nullptr, f64);
-          ps.logJp[p] = lj;
-        }
+        if (ms.kind != 0) lj = ps.logJp[p];
+        stress_any(ms, F, lj, PF, f64);
+        if (ms.kind != 0) ps.logJp[p] = lj;
       }
       fp64_used += f64 ? 1u : 0u;
     }
@@ -293,11 +287,16 @@ __global__ __launch_bounds__(kThreads) void stress_kernel(Model m, ParticlesView
 // if every particle were massless (v, C and m are not read), into channels
 // fch .. fch + 2. kMulti (a batch, ss): each bucket's dx and dt are its
 // scene's. kTile: the launch tile (p2g_threads, p2g_chunk).
+// The stress is either read (st.F == nullptr: contrib, an earlier pass's vol P
+// F^T) or formed here from st.F, particle by particle, before the record: a
+// pass of its own wrote and re-read 36 bytes per particle and read F itself
+// (72 of the substep's 370 bytes per particle).
 // kCell (mode 0, one scene): P2C2GTransfer's particle -> cell -> node kernel
 // (cell_w) in place of the quadratic B-spline, with C and the stress scaled
 // per column by the cell kernel's Dinv.
 template <int kMode, bool kMulti, bool kCell = false, int kTile = 0>
-__global__ __launch_bounds__(p2g_threads(kTile)) void p2g_kernel(ParticlesView ps, const float* __restrict__ contrib,
+__global__ __launch_bounds__(p2g_threads(kTile), 3) void p2g_kernel(ParticlesView ps, const float* __restrict__ contrib,
+                                                       StressFrom st,
                                                        TableView t, SortView sv, const int32_t* __restrict__ nbr_tab,
                                                        float* __restrict__ grid, int32_t grid_cap, float dt,
                                                        float dx, uint32_t* err, uint32_t* queue, SceneSet ss,
@@ -321,6 +320,7 @@ __global__ __launch_bounds__(p2g_threads(kTile)) void p2g_kernel(ParticlesView p
   __shared__ int32_t ccount[kMainCells + 1], cstart[kMainCells + 1], cfill[kMainCells + 1];
   __shared__ int32_t nbr[8];
 
+  const float* __restrict__ stress_rows = st.F ? st.F : contrib;
   const int32_t nb = bounded_blocks(t, sv, grid_cap, err);
   const float dx_inv = (float)1.0 / dx;
   const float D_inv = 4.f * dx_inv * dx_inv;
@@ -415,6 +415,8 @@ __global__ __launch_bounds__(p2g_threads(kTile)) void p2g_kernel(ParticlesView p
         float PF[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         float C[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         const float mass = (live && kMom) ? ps.m[p] : 0.f;
+        float lj = 0.f;
+        if (kStress && live && st.F && ps.logJp) lj = ps.logJp[p];
         if (contig) {
           RowLoad<3> lx, lv;
           RowLoad<9> lp, lc;
@@ -423,7 +425,7 @@ __global__ __launch_bounds__(p2g_threads(kTile)) void p2g_kernel(ParticlesView p
           __builtin_amdgcn_s_setprio(2);
           lx.issue(ps.x, p0, cw);
           if (kMom) lv.issue(ps.v, p0, cw);
-          if (kStress) lp.issue(contrib, p0, cw);
+          if (kStress) lp.issue(stress_rows, p0, cw);
           if (kMom) lc.issue(ps.C, p0, cw);
           __builtin_amdgcn_s_setprio(0);
           lx.finish(stage, cw, xv);
@@ -438,11 +440,24 @@ __global__ __launch_bounds__(p2g_threads(kTile)) void p2g_kernel(ParticlesView p
           }
 #pragma unroll
           for (int k = 0; k < 9; ++k) {
-            if (kStress) PF[k] = contrib[9 * p + k];
+            if (kStress) PF[k] = stress_rows[9 * p + k];
             if (kMom) C[k] = ps.C[9 * p + k];
           }
         }
         if (!live) continue;
+        if (kStress && st.F) {
+          float F[9];
+#pragma unroll
+          for (int k = 0; k < 9; ++k) F[k] = PF[k];
+          if constexpr (kMulti) {
+            const Model& ms = ss.p[bmeta[6]].model;
+            stress_plain(ms, F, lj, PF);
+            if (ms.kind != 0 && st.store_lj) ps.logJp[p] = lj;
+          } else {
+            stress_plain(st.m, F, lj, PF);
+            if (st.m.kind != 0 && st.store_lj) ps.logJp[p] = lj;
+          }
+        }
         const float x0 = xv[0], x1 = xv[1], x2 = xv[2];
         const float v0 = vv[0], v1 = vv[1], v2 = vv[2];
         // base node and local position in grid units (LocalArena::init, Utils.hpp:51-70)
@@ -1154,13 +1169,9 @@ __global__ __launch_bounds__(kT) void g2p_kernel(ParticlesView ps, ParticlesView
           float PF[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
           if (live) {
             bool f64 = false;
-            if (kNext == 0) {
-              stress_fixedcorotated(ns.m, Fn, PF, f64);
-            } else {
-              float lj = ljcopy;
-              stress_sand(ns.m, Fn, lj, PF, nullptr, f64);
-              ns.lj_next[q] = lj;
-            }
+            float lj = ljcopy;
+            stress_any(ns.m, Fn, lj, PF, f64);
+            if (kNext == 1) ns.lj_next[q] = lj;
             fp64_used += f64 ? 1u : 0u;
           }
           wave_store_rows<9>(ns.contrib, (int64_t)off + i0, cw, stage, PF);
@@ -1471,7 +1482,7 @@ hipError_t stress(const Model& m, const ParticlesView& ps, Workspace& ws, hipStr
 
 hipError_t p2g_scatter(const ParticlesView& ps, const TableView& t, const SortView& sv, float* grid,
                        int32_t grid_cap, float dt, float dx, bool fold, Workspace& ws, hipStream_t s,
-                       bool reset_queue, const SceneSet* ss) {
+                       bool reset_queue, const SceneSet* ss, const StressFrom& st) {
   const int g = ws.grid_p2g > 0 ? ws.grid_p2g : persistent_groups();
   if (reset_queue) reset_queue_kernel<<<1, 1, 0, s>>>(ws.counters);
   uint32_t* q = ws.counters + kCtrQueue;
@@ -1479,51 +1490,52 @@ hipError_t p2g_scatter(const ParticlesView& ps, const TableView& t, const SortVi
   const SceneSet sset = multi ? *ss : SceneSet{};
   const bool tile1 = ws.p2g_tile == 1;  // the folded launches take the tuned tile
   if (fold && ws.cell && !multi)  // the substep's P2C2G (one tile)
-    p2g_kernel<0, false, true><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, t, sv, ws.nbr, grid, grid_cap, dt, dx,
+    p2g_kernel<0, false, true><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx,
                                                          ws.err, q, sset, 1);
   else if (fold && multi && tile1)
-    p2g_kernel<0, true, false, 1><<<g, p2g_threads(1), 0, s>>>(ps, ws.contrib, t, sv, ws.nbr, grid, grid_cap, dt, dx,
+    p2g_kernel<0, true, false, 1><<<g, p2g_threads(1), 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx,
                                                                ws.err, q, sset, 1);
   else if (fold && multi)
-    p2g_kernel<0, true><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, q,
+    p2g_kernel<0, true><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, q,
                                                   sset, 1);
   else if (fold && tile1)
-    p2g_kernel<0, false, false, 1><<<g, p2g_threads(1), 0, s>>>(ps, ws.contrib, t, sv, ws.nbr, grid, grid_cap, dt,
+    p2g_kernel<0, false, false, 1><<<g, p2g_threads(1), 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt,
                                                                 dx, ws.err, q, sset, 1);
   else if (fold)
-    p2g_kernel<0, false><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, q,
+    p2g_kernel<0, false><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, q,
                                                    sset, 1);
   else if (multi) {
     // the force kept in channels 4..6: momentum, then the force
-    p2g_kernel<1, true><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, q,
+    p2g_kernel<1, true><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, q,
                                                   sset, 1);
     reset_queue_kernel<<<1, 1, 0, s>>>(ws.counters);
-    p2g_kernel<2, true><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, q,
+    p2g_kernel<2, true><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, q,
                                                   sset, 4);
   } else {
-    p2g_kernel<1, false><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, q,
+    p2g_kernel<1, false><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, q,
                                                    sset, 1);
     reset_queue_kernel<<<1, 1, 0, s>>>(ws.counters);
-    p2g_kernel<2, false><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, q,
+    p2g_kernel<2, false><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, q,
                                                    sset, 4);
   }
   return hipGetLastError();
 }
 
 hipError_t p2c2g_scatter(const ParticlesView& ps, const TableView& t, const SortView& sv, float* grid,
-                         int32_t grid_cap, float dt, float dx, Workspace& ws, hipStream_t s) {
+                         int32_t grid_cap, float dt, float dx, Workspace& ws, hipStream_t s, const StressFrom& st) {
   const int g = ws.grid_p2g > 0 ? ws.grid_p2g : persistent_groups();
   reset_queue_kernel<<<1, 1, 0, s>>>(ws.counters);
-  p2g_kernel<0, false, true><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, t, sv, ws.nbr, grid, grid_cap, dt, dx,
+  p2g_kernel<0, false, true><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx,
                                                        ws.err, ws.counters + kCtrQueue, SceneSet{}, 1);
   return hipGetLastError();
 }
 
 hipError_t p2g_force_scatter(const ParticlesView& ps, const TableView& t, const SortView& sv, float* grid,
-                             int32_t grid_cap, float dt, float dx, Workspace& ws, hipStream_t s) {
+                             int32_t grid_cap, float dt, float dx, Workspace& ws, hipStream_t s,
+                             const StressFrom& st) {
   const int g = ws.grid_p2g > 0 ? ws.grid_p2g : persistent_groups();
   reset_queue_kernel<<<1, 1, 0, s>>>(ws.counters);
-  p2g_kernel<2, false><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err,
+  p2g_kernel<2, false><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err,
                                                  ws.counters + kCtrQueue, SceneSet{}, 1);
   return hipGetLastError();
 }

@@ -93,6 +93,16 @@ struct SceneSet {
   int32_t n = 0;                   // 0: one scene, parameters from the launch arguments
   const SceneParams* p = nullptr;  // [n] device
   const int64_t* first = nullptr;  // [n + 1] device: first[0] = 0, first[n] = particle count
+  bool fp64 = false;               // some scene's model has the FP64 SVD on
+};
+
+// Where a P2G launch takes vol P F^T from: formed from the rows of F (in a
+// batch with each scene's model; only with the FP64 SVD off), or, with F null,
+// read from the workspace's stress array. store_lj: sand's logJp is written back.
+struct StressFrom {
+  const float* F = nullptr;
+  bool store_lj = false;
+  Model m{};
 };
 
 // scene of a block from the first component of its key, clamped to the
@@ -158,15 +168,15 @@ struct Workspace {
   uint32_t* lb_key = nullptr;
   uint32_t* lb_val = nullptr;
   uint32_t list_cap = 0;
-  // bucket sort: per 64-particle group the heads of its segments, per segment
-  // its bucket and place, and the buckets' segment lists (two, to order in)
-  uint64_t* seg_heads = nullptr;  // [n_cap / 64 + 2]
-  uint2* seg_in = nullptr;        // [n_cap + 64]
+  // bucket sort: segments per tile (256 or 1,024 particles), per segment its
+  // bucket and place and where it lies, and the buckets' segment lists (two, to order in)
+  uint32_t* seg_count = nullptr;  // [n_cap / 256 + 1]
+  uint2* seg_in = nullptr;        // [n_cap + 1024]
+  uint32_t* seg_where = nullptr;  // [n_cap + 1024]
   uint64_t* seg_list = nullptr;   // [n_cap]
   uint64_t* seg_alt = nullptr;    // [n_cap]
   uint64_t* scnt = nullptr;       // [ts_cap] per dedup slot: segments << 32 | particles
-  uint64_t* bcnt = nullptr;       // [ts_cap] the same per block
-  uint64_t* bpart = nullptr;      // [ts_cap / 1024 + 2] and summed per 1,024 blocks
+  uint64_t* bcnt = nullptr;       // [ts_cap] the same per block (ts_cap is even)
   uint32_t* segoff = nullptr;     // [ts_cap] start of each block's segment list
   uint32_t* scan_tmp = nullptr;  // tile sums for scans
   size_t scan_words = 0;
@@ -186,8 +196,8 @@ struct Workspace {
   uint32_t* bm_prefix = nullptr; // [bm_words] exclusive prefix of the bit counts
   uint32_t bm_words = 0;
   uint32_t* bitmap_b = nullptr;  // [ts_cap / 32 + 10] the same of the substep's enlargement orders
-  uint32_t* rank_a = nullptr;    // [rank_scratch_words(n_cap)] marked orders counted by size class (sparsity.hip)
-  uint32_t* rank_b = nullptr;    // [rank_scratch_words(ts_cap)]
+  uint32_t* rank_a = nullptr;    // [rank_scratch_words()] marked orders counted by group (sparsity.hip)
+  uint32_t* rank_b = nullptr;    // [rank_scratch_words()]
   int32_t* slot_block = nullptr; // [ts_cap] block number of the key in each scratch slot
   uint32_t* dmask = nullptr;     // [2 (ts_cap / 32 + 1)] one bit per dedup slot claimed by a pass
 };
@@ -242,7 +252,7 @@ hipError_t table_enlarge(const TableView& t, Workspace& ws, const int32_t lo[3],
 hipError_t table_query(const TableView& t, const int32_t* keys, int64_t n, int32_t* out, hipStream_t s);
 hipError_t bucket_sort(const TableView& t, Workspace& ws, const float* x, int64_t n, float dx,
                        int blockLen, int offset, float disp, const SortView& out, hipStream_t s);
-size_t rank_scratch_words(uint64_t orders);
+size_t rank_scratch_words();
 // The substep's build: clear, activation (blockLen 4, offset -2, displacement
 // 0.5), enlargement by {0,1}^3 and bucket sort in one chain. The table, the
 // buckets (counts and offsets after build_enlarge, indices after build_place)
@@ -263,7 +273,9 @@ hipError_t block_neighbours(const TableView& t, Workspace& ws, hipStream_t s);
 // every transfer kernel's static LDS fits the device's per-workgroup limit
 hipError_t check_launch_limits(int device);
 hipError_t grid_clear(float* grid, const int32_t* nblocks_dev, int32_t cap_blocks, hipStream_t s);
-// P2G = stress (per particle, writes ws.contrib and logJp) + scatter (per bucket).
+// The stress as a pass of its own (per particle, writes ws.contrib and logJp):
+// the closure's, the FP64 SVD's and the stress entry point's. P2G otherwise
+// forms it inside the scatter (StressFrom).
 // beside_sparsity: the pass runs on a second stream next to the sparsity
 // stages, and leaves room on every CU for them (at most three of its
 // workgroups per CU)
@@ -288,11 +300,11 @@ hipError_t closure_launch_limits();
 // bucket's or node's scene, read from its block key
 hipError_t p2g_scatter(const ParticlesView& ps, const TableView& t, const SortView& sv, float* grid,
                        int32_t grid_cap, float dt, float dx, bool fold, Workspace& ws, hipStream_t s,
-                       bool reset_queue = true, const SceneSet* ss = nullptr);
+                       bool reset_queue = true, const SceneSet* ss = nullptr, const StressFrom& st = StressFrom{});
 // P2C2GTransfer as a scatter of each particle's cell-kernel stencil (folded
-// into m and mv, channels 0..3) with the stress already in ws.contrib
+// into m and mv, channels 0..3)
 hipError_t p2c2g_scatter(const ParticlesView& ps, const TableView& t, const SortView& sv, float* grid,
-                         int32_t grid_cap, float dt, float dx, Workspace& ws, hipStream_t s);
+                         int32_t grid_cap, float dt, float dx, Workspace& ws, hipStream_t s, const StressFrom& st);
 // G2C2PTransfer with its pre and post passes, in place: v, B (in C), F, x
 hipError_t g2c2p(const ParticlesView& ps, const TableView& t, const SortView& sv, const float* grid, int32_t grid_cap,
                  float dt, float dx, Workspace& ws, hipStream_t s);
@@ -318,10 +330,11 @@ inline int persistent_groups() { return 4096; }
 // ---- implicit step (implicit.hip; the projection in transfer.hip) ----
 // Vectors hold 3 floats per node (node = block * 64 + cell) for the blocks the
 // table holds (read on the device), at most grid_cap.
-// P2G's folded scatter of the stress in ws.contrib alone (as if every
-// particle were massless; v, C and m are not read): G2P2G's force half
+// P2G's folded scatter of the stress alone (as if every particle were
+// massless; v, C and m are not read): G2P2G's force half
 hipError_t p2g_force_scatter(const ParticlesView& ps, const TableView& t, const SortView& sv, float* grid,
-                             int32_t grid_cap, float dt, float dx, Workspace& ws, hipStream_t s);
+                             int32_t grid_cap, float dt, float dx, Workspace& ws, hipStream_t s,
+                             const StressFrom& st);
 // G2P2G's gather half, per bucket: Fout[9 p] = (I + dt C(v)) F_old
 hipError_t g2p2g_gather(const ParticlesView& ps, const TableView& t, const SortView& sv, const float* v,
                         int32_t grid_cap, float dt, float dx, float* Fout, Workspace& ws, hipStream_t s);
