@@ -1827,8 +1827,8 @@ constexpr int32_t kMaxLaunchGroups = 1 << 20;
 
 int32_t zsmpm_policy_launch_widths__rocm(zsmpm_policy pol, int32_t* p2g_groups, int32_t* g2p_groups) {
   if (!pol || !p2g_groups || !g2p_groups) return ZSMPM_INVALID_ARGUMENT;
-  *p2g_groups = pol->tuned_p2g > 0 ? pol->tuned_p2g : persistent_groups();
-  *g2p_groups = pol->tuned_g2p > 0 ? pol->tuned_g2p : persistent_groups();
+  *p2g_groups = pol->tuned_p2g > 0 ? pol->tuned_p2g : default_p2g_groups();
+  *g2p_groups = pol->tuned_g2p > 0 ? pol->tuned_g2p : default_g2p_groups();
   return ZSMPM_OK;
 }
 

@@ -103,10 +103,13 @@ __device__ __forceinline__ int32_t bounded_blocks(const TableView& t, const Sort
   return nb;
 }
 
-// P2G hands buckets out in order from a queue (one atomic per bucket), so a
-// workgroup that drew small buckets takes more: bucket sizes range from 0
-// (enlarged-only blocks) to several hundred particles. Every workgroup leaves
-// once the queue passes the bucket count.
+// P2G: workgroup i starts with bucket i, and the buckets past the grid are
+// handed out in order from a queue, so a workgroup that drew small buckets
+// takes more: bucket sizes range from 0 (enlarged-only blocks) to several
+// hundred particles. Every workgroup leaves once the queue passes the bucket
+// count; where the grid covers the buckets nobody touches it (a pop by each of
+// 4,096 workgroups, most of them without a bucket, was 20 of the 60 us that P2G
+// took on a small scene).
 __global__ void reset_queue_kernel(uint32_t* counters) { counters[kCtrQueue] = 0u; }
 
 // neighbour blocks key + (d>>2&1, d>>1&1, d&1) of bucket b, from the
@@ -162,10 +165,11 @@ __device__ __forceinline__ void lane_cell(int l, int& i, int& j, int& k) {
 }
 
 // quadratic B-spline weights from the local position l in [0.5, 1.5)
-// (quadratic_bspline_weights, math/curve/InterpolationKernel.hpp:95-130)
+// (quadratic_bspline_weights, math/curve/InterpolationKernel.hpp:95-130, whose
+// floor(l - 0.5) is 0 there: l is X - floor(X - 0.5), exact for X >= 0.5)
 __device__ __forceinline__ void bspline_w(float l, float (&w)[3]) {
 #pragma clang fp contract(off)
-  const float d0 = l - (float)(int32_t)floorf(l - 0.5f);
+  const float d0 = l;
   w[0] = 0.5f * (1.5f - d0) * (1.5f - d0);
   const float d1 = d0 - 1.0f;
   w[1] = 0.75f - d1 * d1;
@@ -326,7 +330,12 @@ __global__ __launch_bounds__(p2g_threads(kTile), 3) void p2g_kernel(ParticlesVie
   const float D_inv = 4.f * dx_inv * dx_inv;
   const float scale = -dt * D_inv;
   const int wave = uniform((int32_t)(threadIdx.x / kWave)), lane = lane_id();
-  // Buckets come from the queue one ahead: thread 0 pops the next bucket
+  if ((int32_t)blockIdx.x >= nb) return;
+  auto pop = [&]() -> int32_t {
+    if ((int64_t)gridDim.x >= nb) return nb;
+    return (int32_t)min((uint64_t)gridDim.x + atomicAdd(queue, 1u), (uint64_t)nb);
+  };
+  // Buckets come one ahead: thread 0 pops the next bucket
   // after the last chunk's counting sort and loads its count, offset and key
   // while phase C runs (bmeta, published by the barrier that ends the chunk);
   // every thread then issues the loads of its particle indices in the next
@@ -336,7 +345,7 @@ __global__ __launch_bounds__(p2g_threads(kTile), 3) void p2g_kernel(ParticlesVie
   __shared__ int32_t bmeta[7];  // bucket, count, offset, key, scene
   const int32_t nscenes = kMulti ? ss.n : 0;
   if (threadIdx.x == 0)
-    bucket_meta((int32_t)min(atomicAdd(queue, 1u), 0x7fffffffu), nb, sv, t, ps.n, bmeta, nscenes);
+    bucket_meta((int32_t)blockIdx.x, nb, sv, t, ps.n, bmeta, nscenes);
   for (int c = threadIdx.x; c <= kMainCells; c += kT) {
     ccount[c] = 0;
     cfill[c] = 0;
@@ -360,7 +369,7 @@ __global__ __launch_bounds__(p2g_threads(kTile), 3) void p2g_kernel(ParticlesVie
     if (cnt == 0) {  // empty or out-of-range bucket: take the next one now
       __syncthreads();
       if (threadIdx.x == 0)
-        bucket_meta((int32_t)min(atomicAdd(queue, 1u), 0x7fffffffu), nb, sv, t, ps.n, bmeta, nscenes);
+        bucket_meta(pop(), nb, sv, t, ps.n, bmeta, nscenes);
       __syncthreads();
       prefetch();
       continue;
@@ -374,7 +383,7 @@ __global__ __launch_bounds__(p2g_threads(kTile), 3) void p2g_kernel(ParticlesVie
       bscale = -sp.dt * (4.f * bdx_inv * bdx_inv);
     }
     load_neighbours(nbr_tab, b, nbr, err);
-    uint32_t nxt = 0;  // thread 0: the next bucket, popped during the last chunk
+    int32_t nxt = nb;  // thread 0: the next bucket, popped during the last chunk
 
     for (int32_t c0 = 0; c0 < cnt; c0 += kChunk) {
       const int32_t nch = min(kChunk, cnt - c0);
@@ -391,14 +400,20 @@ __global__ __launch_bounds__(p2g_threads(kTile), 3) void p2g_kernel(ParticlesVie
       // consecutive chunk slots (i = threadIdx.x + k * kT, as phase B
       // expects); a contiguous run of particles is read with 16-byte vectors,
       // staged in the wave's own (not yet written) record slots.
-#pragma unroll
+      // Not unrolled: the loop body with both stress paths is 3,000
+      // instructions, and three copies of it (110 KB with the rest) overflow the
+      // 64 KB instruction cache two CUs share.
+#pragma clang loop unroll(disable)
       for (int kk = 0; kk < kPre; ++kk) {
         const int32_t i0 = wave * kWave + kk * kT;
         if (i0 >= nch) break;
+        int32_t pre_kk = pre[0];
+#pragma unroll
+        for (int q = 1; q < kPre; ++q) pre_kk = kk == q ? pre[q] : pre_kk;
         const int32_t i = i0 + lane;
         const int32_t cw = min(kWave, nch - i0);
         const bool valid = lane < cw;
-        const int64_t p = valid ? (int64_t)(c0 == 0 ? pre[kk] : sv.indices[off + c0 + i]) : -1;
+        const int64_t p = valid ? (int64_t)(c0 == 0 ? pre_kk : sv.indices[off + c0 + i]) : -1;
         const bool bad = valid && (p < 0 || p >= ps.n);
         if (bad) {
           atomicOr(err, kErrCapacity);
@@ -552,7 +567,7 @@ __global__ __launch_bounds__(p2g_threads(kTile), 3) void p2g_kernel(ParticlesVie
       }
       __syncthreads();
       const bool last = c0 + kChunk >= cnt;
-      if (last && threadIdx.x == 0) nxt = atomicAdd(queue, 1u);
+      if (last && threadIdx.x == 0) nxt = pop();
       // ---- C: rounds, lane = main cell
       {
         const int32_t lcount = ccount[lane];
@@ -621,36 +636,44 @@ __global__ __launch_bounds__(p2g_threads(kTile), 3) void p2g_kernel(ParticlesVie
           }
         }
       }
-      // ---- overflow particles: global atomics straight into the grid
+      // ---- overflow particles (rare): global atomics straight into the grid
+      if (ccount[kMainCells] > 0) {
+#pragma clang loop unroll(disable)
+        for (int k = 0; k < kPre; ++k) {
+          const int32_t i = threadIdx.x + k * kT;
+          uint32_t base = keep[0], home = keepc[0];
 #pragma unroll
-      for (int k = 0; k < kPre; ++k) {
-        const int32_t i = threadIdx.x + k * kT;
-        if (i >= nch || keepc[k] != kMainCells) continue;
-        const int r0 = (keep[k] >> 6) & 7, r1 = (keep[k] >> 3) & 7, r2 = keep[k] & 7;
-        const float4 q0 = rec[i], q1 = rec[kChunk + i], q2 = rec[2 * kChunk + i], q3 = rec[3 * kChunk + i];
-        const float Am[9] = {q2.x, q2.y, q2.z, q2.w, q3.x, q3.y, q3.z, q3.w, q1.w};
-        float w0[3], w1[3], w2[3];
-        stencil_w<kCell>(q1.x, w0);
-        stencil_w<kCell>(q1.y, w1);
-        stencil_w<kCell>(q1.z, w2);
-        for (int a = 0; a < 3; ++a)
-          for (int bb = 0; bb < 3; ++bb)
-            for (int c = 0; c < 3; ++c) {
-              const float W = w0[a] * w1[bb] * w2[c];
-              int nbi, cell;
-              node_home(r0 + a, r1 + bb, r2 + c, nbi, cell);
-              const int32_t gb = nbr[nbi];
-              if (gb < 0 || gb >= grid_cap) continue;
-              float* gp = grid + grid_at(gb, 0, cell);
-              const float fa = (float)a, fb = (float)bb, fc = (float)c;
-              float* gv = kMom ? gp + kBlockCells : gp + fch * kBlockCells;  // momentum or force channels
-              if (kMom) unsafeAtomicAdd(gp, q0.x * W);
-              unsafeAtomicAdd(gv, W * (q0.y + Am[0] * fa + Am[3] * fb + Am[6] * fc));
-              unsafeAtomicAdd(gv + kBlockCells, W * (q0.z + Am[1] * fa + Am[4] * fb + Am[7] * fc));
-              unsafeAtomicAdd(gv + 2 * kBlockCells, W * (q0.w + Am[2] * fa + Am[5] * fb + Am[8] * fc));
-            }
+          for (int q = 1; q < kPre; ++q) {
+            base = k == q ? keep[q] : base;
+            home = k == q ? keepc[q] : home;
+          }
+          if (i >= nch || home != (uint32_t)kMainCells) continue;
+          const int r0 = (base >> 6) & 7, r1 = (base >> 3) & 7, r2 = base & 7;
+          const float4 q0 = rec[i], q1 = rec[kChunk + i], q2 = rec[2 * kChunk + i], q3 = rec[3 * kChunk + i];
+          float w0[3], w1[3], w2[3];
+          stencil_w<kCell>(q1.x, w0);
+          stencil_w<kCell>(q1.y, w1);
+          stencil_w<kCell>(q1.z, w2);
+#pragma clang loop unroll(disable)
+          for (int o = 0; o < 27; ++o) {
+            const int a = o / 9, bb = o / 3 % 3, c = o % 3;
+            const float W = (a == 0 ? w0[0] : a == 1 ? w0[1] : w0[2]) *
+                            (bb == 0 ? w1[0] : bb == 1 ? w1[1] : w1[2]) * (c == 0 ? w2[0] : c == 1 ? w2[1] : w2[2]);
+            int nbi, cell;
+            node_home(r0 + a, r1 + bb, r2 + c, nbi, cell);
+            const int32_t gb = nbr[nbi];
+            if (gb < 0 || gb >= grid_cap) continue;
+            float* gp = grid + grid_at(gb, 0, cell);
+            const float fa = (float)a, fb = (float)bb, fc = (float)c;
+            float* gv = kMom ? gp + kBlockCells : gp + fch * kBlockCells;  // momentum or force channels
+            if (kMom) unsafeAtomicAdd(gp, q0.x * W);
+            unsafeAtomicAdd(gv, W * (q0.y + q2.x * fa + q2.w * fb + q3.z * fc));
+            unsafeAtomicAdd(gv + kBlockCells, W * (q0.z + q2.y * fa + q3.x * fb + q3.w * fc));
+            unsafeAtomicAdd(gv + 2 * kBlockCells, W * (q0.w + q2.z * fa + q3.y * fb + q1.w * fc));
+          }
+        }
       }
-      if (last && threadIdx.x == 0) bucket_meta((int32_t)min(nxt, 0x7fffffffu), nb, sv, t, ps.n, bmeta, nscenes);
+      if (last && threadIdx.x == 0) bucket_meta(nxt, nb, sv, t, ps.n, bmeta, nscenes);
       __syncthreads();
     }
     prefetch();  // the next bucket's first-chunk indices (bmeta is the next bucket's now)
@@ -1480,10 +1503,33 @@ hipError_t stress(const Model& m, const ParticlesView& ps, Workspace& ws, hipStr
   return hipGetLastError();
 }
 
+namespace {
+
+// Workgroups of the per-bucket kernels: the policy's counts, else P2G as many
+// as are resident (three of four waves per CU, or six of two) -- more only
+// queue behind each other -- and G2P one per bucket up to 32,768; no more than
+// there can be buckets.
+int bucket_bound(const SortView& sv, int32_t grid_cap) {
+  const int32_t cap = grid_cap < sv.cap_blocks ? grid_cap : sv.cap_blocks;
+  return cap > 1 ? cap : 1;
+}
+int p2g_groups(const Workspace& ws, const SortView& sv, int32_t grid_cap) {
+  const int g = ws.grid_p2g > 0 ? ws.grid_p2g : (ws.p2g_tile == 1 ? 2 : 1) * default_p2g_groups();
+  const int cap = bucket_bound(sv, grid_cap);
+  return g < cap ? g : cap;
+}
+int g2p_groups(const Workspace& ws, const SortView& sv, int32_t grid_cap) {
+  const int g = ws.grid_g2p > 0 ? ws.grid_g2p : default_g2p_groups();
+  const int cap = bucket_bound(sv, grid_cap);
+  return g < cap ? g : cap;
+}
+
+}  // namespace
+
 hipError_t p2g_scatter(const ParticlesView& ps, const TableView& t, const SortView& sv, float* grid,
                        int32_t grid_cap, float dt, float dx, bool fold, Workspace& ws, hipStream_t s,
                        bool reset_queue, const SceneSet* ss, const StressFrom& st) {
-  const int g = ws.grid_p2g > 0 ? ws.grid_p2g : persistent_groups();
+  const int g = p2g_groups(ws, sv, grid_cap);
   if (reset_queue) reset_queue_kernel<<<1, 1, 0, s>>>(ws.counters);
   uint32_t* q = ws.counters + kCtrQueue;
   const bool multi = ss && ss->n > 0;
@@ -1523,7 +1569,7 @@ hipError_t p2g_scatter(const ParticlesView& ps, const TableView& t, const SortVi
 
 hipError_t p2c2g_scatter(const ParticlesView& ps, const TableView& t, const SortView& sv, float* grid,
                          int32_t grid_cap, float dt, float dx, Workspace& ws, hipStream_t s, const StressFrom& st) {
-  const int g = ws.grid_p2g > 0 ? ws.grid_p2g : persistent_groups();
+  const int g = p2g_groups(ws, sv, grid_cap);
   reset_queue_kernel<<<1, 1, 0, s>>>(ws.counters);
   p2g_kernel<0, false, true><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx,
                                                        ws.err, ws.counters + kCtrQueue, SceneSet{}, 1);
@@ -1533,7 +1579,7 @@ hipError_t p2c2g_scatter(const ParticlesView& ps, const TableView& t, const Sort
 hipError_t p2g_force_scatter(const ParticlesView& ps, const TableView& t, const SortView& sv, float* grid,
                              int32_t grid_cap, float dt, float dx, Workspace& ws, hipStream_t s,
                              const StressFrom& st) {
-  const int g = ws.grid_p2g > 0 ? ws.grid_p2g : persistent_groups();
+  const int g = p2g_groups(ws, sv, grid_cap);
   reset_queue_kernel<<<1, 1, 0, s>>>(ws.counters);
   p2g_kernel<2, false><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err,
                                                  ws.counters + kCtrQueue, SceneSet{}, 1);
@@ -1543,14 +1589,14 @@ hipError_t p2g_force_scatter(const ParticlesView& ps, const TableView& t, const 
 hipError_t g2p2g_gather(const ParticlesView& ps, const TableView& t, const SortView& sv, const float* v,
                         int32_t grid_cap, float dt, float dx, float* Fout, Workspace& ws, hipStream_t s) {
   if (ps.n == 0) return hipSuccess;
-  const int g = ws.grid_g2p > 0 ? ws.grid_g2p : persistent_groups();
+  const int g = g2p_groups(ws, sv, grid_cap);
   g2p2g_gather_kernel<<<g, kG2PThreads, 0, s>>>(ps, t, sv, ws.nbr, v, grid_cap, dt, dx, Fout, ws.err);
   return hipGetLastError();
 }
 
 hipError_t g2c2p(const ParticlesView& ps, const TableView& t, const SortView& sv, const float* grid, int32_t grid_cap,
                  float dt, float dx, Workspace& ws, hipStream_t s) {
-  const int g = ws.grid_g2p > 0 ? ws.grid_g2p : persistent_groups();
+  const int g = g2p_groups(ws, sv, grid_cap);
   g2p_kernel<false, -1, false, true><<<g, kG2PThreads, 0, s>>>(ps, ps, t, sv, ws.nbr, grid, grid_cap, dt, dx,
                                                                NextStress{}, ws.err, ws.counters, SceneSet{});
   return hipGetLastError();
@@ -1580,7 +1626,7 @@ hipError_t grid_angular_momentum(const float* grid, int32_t grid_cap, const Tabl
 hipError_t g2p(const ParticlesView& ps, const ParticlesView* out, const TableView& t, const SortView& sv,
                const float* grid, int32_t grid_cap, float dt, float dx, Workspace& ws, hipStream_t s,
                const NextStress* next, const SceneSet* ss) {
-  const int g = ws.grid_g2p > 0 ? ws.grid_g2p : persistent_groups();
+  const int g = g2p_groups(ws, sv, grid_cap);
   NextStress ns{};
   if (next) ns = *next;
   const SceneSet sset = ss ? *ss : SceneSet{};

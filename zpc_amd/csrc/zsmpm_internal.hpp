@@ -186,7 +186,7 @@ struct Workspace {
   int32_t* nbr = nullptr;        // [8 ts_cap] block index of key_b + (d>>2&1, d>>1&1, d&1), or -1
   int32_t* fb = nullptr;         // [n_cap] particles queued for the closure's SVD fallback
   uint32_t* wq = nullptr;        // [n_cap / 64 + 2] per wave: 1 where the closure's network must run
-  int32_t grid_p2g = 0;          // P2G / G2P workgroups (0: persistent_groups()), set by the policy
+  int32_t grid_p2g = 0;          // P2G / G2P workgroups (0: the defaults below), set by the policy
   int32_t grid_g2p = 0;
   int32_t p2g_tile = 0;     // folded P2G launch tile: 0 four waves / 576-particle chunks, 1 two waves / 256
   int32_t g2p_threads = 0;  // sorted G2P threads per bucket: 256, else 128
@@ -326,6 +326,9 @@ hipError_t reorder_particles(const ParticlesView& in, const ParticlesView& out, 
 
 // grid-stride launch width for kernels that loop over a device-resident count
 inline int persistent_groups() { return 4096; }
+// P2G / G2P workgroups where the policy sets none
+inline int default_p2g_groups() { return 768; }
+inline int default_g2p_groups() { return 32768; }
 
 // ---- implicit step (implicit.hip; the projection in transfer.hip) ----
 // Vectors hold 3 floats per node (node = block * 64 + cell) for the blocks the
