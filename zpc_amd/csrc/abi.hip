@@ -583,7 +583,7 @@ int32_t run_substep(zsmpm_policy_s* pol, const zsmpm_model* model, const zsmpm_p
   }
   {
     StageScope sc(pol, ZSMPM_STAGE_TABLE_CLEAR);
-    // also resets the P2G bucket queue and the max |v|^2 counter
+    // also resets the max |v|^2 counter
     ZS_HIP(build_clear(t, ws, ps.n, s));
   }
   {
@@ -608,7 +608,7 @@ int32_t run_substep(zsmpm_policy_s* pol, const zsmpm_model* model, const zsmpm_p
     // v = (mv + rhs)/m convention), so the update must not add channels 4..6
     StageScope sc(pol, ZSMPM_STAGE_P2G);
     ZS_HIP(zsmpm::p2g_scatter(ps, t, sv, grid->data, grid->capacity_blocks, dt, dx, true, ws, s,
-                              /*reset_queue=*/false, ss, st));
+                              ss, st));
   }
   {
     StageScope sc(pol, ZSMPM_STAGE_GRID_UPDATE);
@@ -1162,7 +1162,7 @@ int32_t zsmpm_p2g__rocm(zsmpm_policy pol, const zsmpm_model* model, const zsmpm_
   StageScope sc(pol, ZSMPM_STAGE_P2G);
   ZS_HIP(block_neighbours(t, pol->ws, pol->stream));
   return from_hip(zsmpm::p2g_scatter(ps, t, sv, grid->data, grid->capacity_blocks, dt, grid->dx, false, pol->ws,
-                                     pol->stream, true, nullptr, st));
+                                     pol->stream, nullptr, st));
 }
 
 int32_t zsmpm_grid_update__rocm(zsmpm_policy pol, const zsmpm_grid* grid, const zsmpm_table* table, float dt,

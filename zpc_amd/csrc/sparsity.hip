@@ -611,7 +611,6 @@ __global__ __launch_bounds__(kThreads) void build_clear_kernel(ClearList c, Tabl
     *t.cnt = 0;
     counters[kCtrList] = 0u;
     counters[kCtrListB] = 0u;
-    counters[kCtrQueue] = 0u;
     counters[kCtrMaxVel] = 0u;
   }
 }

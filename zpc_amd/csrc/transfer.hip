@@ -103,15 +103,6 @@ __device__ __forceinline__ int32_t bounded_blocks(const TableView& t, const Sort
   return nb;
 }
 
-// P2G: workgroup i starts with bucket i, and the buckets past the grid are
-// handed out in order from a queue, so a workgroup that drew small buckets
-// takes more: bucket sizes range from 0 (enlarged-only blocks) to several
-// hundred particles. Every workgroup leaves once the queue passes the bucket
-// count; where the grid covers the buckets nobody touches it (a pop by each of
-// 4,096 workgroups, most of them without a bucket, was 20 of the 60 us that P2G
-// took on a small scene).
-__global__ void reset_queue_kernel(uint32_t* counters) { counters[kCtrQueue] = 0u; }
-
 // neighbour blocks key + (d>>2&1, d>>1&1, d&1) of bucket b, from the
 // per-substep neighbour table
 __device__ __forceinline__ void load_neighbours(const int32_t* __restrict__ nbr_tab, int32_t b, int32_t* nbr,
@@ -121,34 +112,6 @@ __device__ __forceinline__ void load_neighbours(const int32_t* __restrict__ nbr_
     nbr[threadIdx.x] = r;
     if (r < 0) atomicOr(err, kErrMissingBlock);
   }
-}
-
-// Count, offset, block key and scene of bucket b (0 for b >= nb or a bucket
-// whose range is not within the particles), written to m[0..6] by one
-// thread. In a batch of nscenes > 0 scenes the key is the scene's own
-// (offset removed).
-__device__ __forceinline__ void bucket_meta(int32_t b, int32_t nb, const SortView& sv, const TableView& t,
-                                            int64_t n, int32_t* m, int32_t nscenes = 0) {
-  int32_t cnt = 0, off = 0, k0 = 0, k1 = 0, k2 = 0, sc = 0;
-  if (b < nb) {
-    cnt = sv.counts[b];
-    off = sv.offsets[b];
-    if (cnt <= 0 || off < 0 || (int64_t)off + cnt > n) cnt = 0;
-    k0 = t.active[3 * (int64_t)b];
-    k1 = t.active[3 * (int64_t)b + 1];
-    k2 = t.active[3 * (int64_t)b + 2];
-    if (nscenes > 0) {
-      sc = scene_of_key(k0, nscenes);
-      k0 -= sc * kSceneKeyStride;
-    }
-  }
-  m[0] = b;
-  m[1] = cnt;
-  m[2] = off;
-  m[3] = k0;
-  m[4] = k1;
-  m[5] = k2;
-  m[6] = sc;
 }
 
 // Main base cell (i, j, k) in [0,4)^3 <-> lane of the scatter rounds. Lane
@@ -303,8 +266,7 @@ __global__ __launch_bounds__(p2g_threads(kTile), 3) void p2g_kernel(ParticlesVie
                                                        StressFrom st,
                                                        TableView t, SortView sv, const int32_t* __restrict__ nbr_tab,
                                                        float* __restrict__ grid, int32_t grid_cap, float dt,
-                                                       float dx, uint32_t* err, uint32_t* queue, SceneSet ss,
-                                                       int32_t fch) {
+                                                       float dx, uint32_t* err, SceneSet ss, int32_t fch) {
   static_assert(kMode >= 0 && kMode <= 2 && (!kCell || kMode == 0), "P2G modes");
   constexpr bool kMom = kMode != 2;     // mass, v and C are read
   constexpr bool kStress = kMode != 1;  // the stress is read
@@ -330,76 +292,97 @@ __global__ __launch_bounds__(p2g_threads(kTile), 3) void p2g_kernel(ParticlesVie
   const float D_inv = 4.f * dx_inv * dx_inv;
   const float scale = -dt * D_inv;
   const int wave = uniform((int32_t)(threadIdx.x / kWave)), lane = lane_id();
-  if ((int32_t)blockIdx.x >= nb) return;
-  auto pop = [&]() -> int32_t {
-    if ((int64_t)gridDim.x >= nb) return nb;
-    return (int32_t)min((uint64_t)gridDim.x + atomicAdd(queue, 1u), (uint64_t)nb);
-  };
-  // Buckets come one ahead: thread 0 pops the next bucket
-  // after the last chunk's counting sort and loads its count, offset and key
-  // while phase C runs (bmeta, published by the barrier that ends the chunk);
-  // every thread then issues the loads of its particle indices in the next
-  // bucket's first chunk before the flush, so they are in flight across the
-  // flush and the next bucket's set-up instead of starting phase A.
-  constexpr int kPre = (kChunk + kT - 1) / kT;  // chunk slots per thread
-  __shared__ int32_t bmeta[7];  // bucket, count, offset, key, scene
+  // Workgroup i takes the buckets i, i + grid, ... (a queue in their place cost
+  // an atomic and two round trips per bucket and balanced no better: a workgroup
+  // has ~50 buckets at 16M particles) in items of up to kChunk particles, and
+  // keeps the next item's loads in flight: its bucket's count, offset and key
+  // during phase A, its particle indices from the counting sort on, its first
+  // 64 rows per wave during phase C and the flush; within phase A, the next
+  // round's rows while this round's records are formed. With each lane loading
+  // its own rows (load_row) and the divisions, zero fills and scale products
+  // gone from phase A, 1.03 -> 0.81 ms at 16M particles; what bounds it now is
+  // the arithmetic (0.59 ms of vector issue; 2.2 GB of traffic are 0.46 ms).
+  constexpr int kPre = (kChunk + kT - 1) / kT;  // rounds of 64 rows per wave
   const int32_t nscenes = kMulti ? ss.n : 0;
-  if (threadIdx.x == 0)
-    bucket_meta((int32_t)blockIdx.x, nb, sv, t, ps.n, bmeta, nscenes);
+  auto in_range = [&](int32_t cnt, int32_t off) { return cnt > 0 && off >= 0 && (int64_t)off + cnt <= ps.n; };
+  int32_t b = blockIdx.x, cnt = 0, off = 0, c0 = 0;
+  for (; b < nb; b += gridDim.x) {  // the first bucket with particles
+    cnt = uniform(sv.counts[b]);
+    off = uniform(sv.offsets[b]);
+    if (in_range(cnt, off)) break;
+  }
+  if (b >= nb) return;
+  int32_t key[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) key[d] = uniform(t.active[3 * (int64_t)b + d]);
   for (int c = threadIdx.x; c <= kMainCells; c += kT) {
     ccount[c] = 0;
     cfill[c] = 0;
   }
-  __syncthreads();
+  struct Rows {
+    float x[3], v[3], P[9], C[9], m, lj;
+  };
+  Rows ahead;  // rows in flight
+  ahead.m = ahead.lj = 0.f;
+  if (!kMom)
+    for (int d = 0; d < 3; ++d) ahead.v[d] = 0.f;
+  // an index out of range loads row 0, which nobody uses
+  auto load_rows = [&](int32_t q) {
+    if (q < 0 || q >= ps.n) q = 0;
+    // a wave issues its loads ahead of other waves' scatter arithmetic
+    __builtin_amdgcn_s_setprio(2);
+    load_row(ps.x, q, ahead.x);
+    if (kMom) load_row(ps.v, q, ahead.v);
+    if (kStress) load_row(stress_rows, q, ahead.P);
+    if (kMom) load_row(ps.C, q, ahead.C);
+    if (kMom) ahead.m = ps.m[q];
+    if (kStress && st.F && ps.logJp) ahead.lj = ps.logJp[q];
+    __builtin_amdgcn_s_setprio(0);
+  };
   int32_t pre[kPre];
-  auto prefetch = [&]() {
-    const int32_t lim = min(bmeta[1], kChunk), po = bmeta[2];
+  auto load_indices = [&](int32_t icnt, int32_t ioff, int32_t ic0) {
+    const int32_t lim = min(icnt - ic0, kChunk);
 #pragma unroll
     for (int k = 0; k < kPre; ++k) {
       const int32_t i = threadIdx.x + k * kT;
-      pre[k] = i < lim ? sv.indices[po + i] : -1;
+      pre[k] = i < lim ? sv.indices[ioff + ic0 + i] : -1;
     }
   };
-  prefetch();
+  load_indices(cnt, off, 0);
+  load_rows(pre[0]);
+  __syncthreads();
 
   for (;;) {
-    const int32_t b = bmeta[0], cnt = bmeta[1], off = bmeta[2];
-    if (b >= nb) break;
-    const int32_t o0 = bmeta[3] * 4, o1 = bmeta[4] * 4, o2 = bmeta[5] * 4;
-    if (cnt == 0) {  // empty or out-of-range bucket: take the next one now
-      __syncthreads();
-      if (threadIdx.x == 0)
-        bucket_meta(pop(), nb, sv, t, ps.n, bmeta, nscenes);
-      __syncthreads();
-      prefetch();
-      continue;
+    const int32_t nch = min(kChunk, cnt - c0);
+    const bool last = c0 + kChunk >= cnt;
+    // the next bucket's count, offset and key, in flight during phase A
+    int32_t nx_b = last ? b + (int32_t)gridDim.x : b;
+    int32_t nx_cnt = 0, nx_off = 0, nx_key[3] = {0, 0, 0};
+    if (last && nx_b < nb) {
+      nx_cnt = sv.counts[nx_b];
+      nx_off = sv.offsets[nx_b];
+#pragma unroll
+      for (int d = 0; d < 3; ++d) nx_key[d] = t.active[3 * (int64_t)nx_b + d];
     }
+    int32_t nbr_r = 0;
+    if (c0 == 0 && threadIdx.x < 8) nbr_r = nbr_tab[8 * (int64_t)b + threadIdx.x];
+    int32_t k0 = key[0];
     // the bucket's grid spacing and force scale (its scene's, in a batch)
     float bdx = dx, bscale = scale;
+    const Model* bmodel = &st.m;
     if constexpr (kMulti) {
-      const SceneParams& sp = ss.p[bmeta[6]];
+      const int32_t sc = scene_of_key(k0, nscenes);
+      k0 -= sc * kSceneKeyStride;
+      const SceneParams& sp = ss.p[sc];
       bdx = sp.dx;
       const float bdx_inv = (float)1.0 / bdx;
       bscale = -sp.dt * (4.f * bdx_inv * bdx_inv);
+      bmodel = &sp.model;
     }
-    load_neighbours(nbr_tab, b, nbr, err);
-    int32_t nxt = nb;  // thread 0: the next bucket, popped during the last chunk
-
-    for (int32_t c0 = 0; c0 < cnt; c0 += kChunk) {
-      const int32_t nch = min(kChunk, cnt - c0);
-      if (c0 > 0) {
-        // later chunks clear the cell counters here; a bucket's first chunk
-        // finds them cleared by the previous bucket's flush (or the prologue)
-        for (int c = threadIdx.x; c <= kMainCells; c += kT) {  // 64 main cells + overflow
-          ccount[c] = 0;
-          cfill[c] = 0;
-        }
-        __syncthreads();
-      }
+    const int32_t o0 = k0 * 4, o1 = key[1] * 4, o2 = key[2] * 4;
+    {
       // ---- A: stress + affine record per particle. Each wave takes 64
-      // consecutive chunk slots (i = threadIdx.x + k * kT, as phase B
-      // expects); a contiguous run of particles is read with 16-byte vectors,
-      // staged in the wave's own (not yet written) record slots.
+      // consecutive chunk slots (i = threadIdx.x + k * kT, as phase B expects).
       // Not unrolled: the loop body with both stress paths is 3,000
       // instructions, and three copies of it (110 KB with the rest) overflow the
       // 64 KB instruction cache two CUs share.
@@ -407,71 +390,34 @@ __global__ __launch_bounds__(p2g_threads(kTile), 3) void p2g_kernel(ParticlesVie
       for (int kk = 0; kk < kPre; ++kk) {
         const int32_t i0 = wave * kWave + kk * kT;
         if (i0 >= nch) break;
-        int32_t pre_kk = pre[0];
+        int32_t p = pre[0], pnext = -1;
 #pragma unroll
-        for (int q = 1; q < kPre; ++q) pre_kk = kk == q ? pre[q] : pre_kk;
+        for (int q = 1; q < kPre; ++q) {
+          p = kk == q ? pre[q] : p;
+          pnext = kk == q - 1 ? pre[q] : pnext;
+        }
         const int32_t i = i0 + lane;
-        const int32_t cw = min(kWave, nch - i0);
-        const bool valid = lane < cw;
-        const int64_t p = valid ? (int64_t)(c0 == 0 ? pre_kk : sv.indices[off + c0 + i]) : -1;
-        const bool bad = valid && (p < 0 || p >= ps.n);
-        if (bad) {
+        const bool valid = i < nch;
+        const bool live = valid && p >= 0 && p < ps.n;
+        if (valid && !live) {
           atomicOr(err, kErrCapacity);
           cellof[i] = 255;
           list[i] = 0;
         }
-        const bool live = valid && !bad;
-        int64_t p0;
-        // the wave's arena is free during the first chunk's phase A (it is
-        // cleared right after): it stages the vector row loads
-        const bool contig = c0 == 0 && wave_contiguous(p, live, p0) && ballot(bad) == 0;
-        float* stage = reinterpret_cast<float*>(arena[wave]);
-        float xv[3] = {0.f, 0.f, 0.f}, vv[3] = {0.f, 0.f, 0.f};
-        float PF[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        float C[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        const float mass = (live && kMom) ? ps.m[p] : 0.f;
-        float lj = 0.f;
-        if (kStress && live && st.F && ps.logJp) lj = ps.logJp[p];
-        if (contig) {
-          RowLoad<3> lx, lv;
-          RowLoad<9> lp, lc;
-          // the wave issues its row loads ahead of other waves' scatter
-          // arithmetic (0.763 -> 0.757 ms at 16M particles)
-          __builtin_amdgcn_s_setprio(2);
-          lx.issue(ps.x, p0, cw);
-          if (kMom) lv.issue(ps.v, p0, cw);
-          if (kStress) lp.issue(stress_rows, p0, cw);
-          if (kMom) lc.issue(ps.C, p0, cw);
-          __builtin_amdgcn_s_setprio(0);
-          lx.finish(stage, cw, xv);
-          if (kMom) lv.finish(stage, cw, vv);
-          if (kStress) lp.finish(stage, cw, PF);
-          if (kMom) lc.finish(stage, cw, C);
-        } else if (live) {
-#pragma unroll
-          for (int d = 0; d < 3; ++d) {
-            xv[d] = ps.x[3 * p + d];
-            if (kMom) vv[d] = ps.v[3 * p + d];
-          }
-#pragma unroll
-          for (int k = 0; k < 9; ++k) {
-            if (kStress) PF[k] = stress_rows[9 * p + k];
-            if (kMom) C[k] = ps.C[9 * p + k];
-          }
-        }
+        const Rows row = ahead;
+        if (i0 + kT < nch) load_rows(pnext);
         if (!live) continue;
-        if (kStress && st.F) {
-          float F[9];
+        const float (&xv)[3] = row.x;
+        const float (&vv)[3] = row.v;
+        const float (&C)[9] = row.C;
+        const float mass = row.m;
+        float PF[9];
 #pragma unroll
-          for (int k = 0; k < 9; ++k) F[k] = PF[k];
-          if constexpr (kMulti) {
-            const Model& ms = ss.p[bmeta[6]].model;
-            stress_plain(ms, F, lj, PF);
-            if (ms.kind != 0 && st.store_lj) ps.logJp[p] = lj;
-          } else {
-            stress_plain(st.m, F, lj, PF);
-            if (st.m.kind != 0 && st.store_lj) ps.logJp[p] = lj;
-          }
+        for (int k = 0; k < 9; ++k) PF[k] = row.P[k];
+        if (kStress && st.F) {
+          float lj = row.lj;
+          stress_plain(*bmodel, row.P, lj, PF);
+          if (bmodel->kind != 0 && st.store_lj) ps.logJp[p] = lj;
         }
         const float x0 = xv[0], x1 = xv[1], x2 = xv[2];
         const float v0 = vv[0], v1 = vv[1], v2 = vv[2];
@@ -481,9 +427,11 @@ __global__ __launch_bounds__(p2g_threads(kTile), 3) void p2g_kernel(ParticlesVie
         {
 #pragma clang fp contract(off)
           const float xs[3] = {x0, x1, x2};
+          const bool pow2 = is_pow2(bdx);
+          const float bdx_inv = 1.f / bdx;
 #pragma unroll
           for (int d = 0; d < 3; ++d) {
-            const float X = xs[d] / bdx;
+            const float X = pow2 ? xs[d] * bdx_inv : xs[d] / bdx;
             base[d] = (int32_t)floorf(X - 0.5f);
             l[d] = X - (float)base[d];
           }
@@ -512,9 +460,9 @@ __global__ __launch_bounds__(p2g_threads(kTile), 3) void p2g_kernel(ParticlesVie
         } else {
 #pragma unroll
           for (int k = 0; k < 9; ++k) {
-            if (kMode == 0) A[k] = (mass * C[k] + PF[k] * bscale) * bdx;
-            if (kMode == 1) A[k] = mass * C[k] * bdx;
-            if (kMode == 2) A[k] = PF[k] * bscale * bdx;
+            if (kMode == 0) A[k] = (mass * bdx) * C[k] + PF[k] * (bscale * bdx);
+            if (kMode == 1) A[k] = (mass * bdx) * C[k];
+            if (kMode == 2) A[k] = PF[k] * (bscale * bdx);
           }
         }
 #pragma unroll
@@ -528,9 +476,10 @@ __global__ __launch_bounds__(p2g_threads(kTile), 3) void p2g_kernel(ParticlesVie
         list[i] = (uint16_t)((r0 << 6) | (r1 << 3) | r2);  // base offsets; the list is rebuilt in B
       }
       if (c0 == 0) {
-        // the first chunk's loads are done with the wave's arena as stage:
-        // clear it for the bucket's accumulation
-        wave_lds_barrier();
+        if (threadIdx.x < 8) {
+          nbr[threadIdx.x] = nbr_r;
+          if (nbr_r < 0) atomicOr(err, kErrMissingBlock);
+        }
         for (int k = lane; k < kArena6; k += kWave) arena[wave][k] = make_float4(0.f, 0.f, 0.f, 0.f);
       }
       __syncthreads();
@@ -566,8 +515,30 @@ __global__ __launch_bounds__(p2g_threads(kTile), 3) void p2g_kernel(ParticlesVie
         }
       }
       __syncthreads();
-      const bool last = c0 + kChunk >= cnt;
-      if (last && threadIdx.x == 0) nxt = pop();
+      // the next item; its indices load during the first slab
+      int32_t nx_c0 = 0;
+      if (last) {
+        nx_cnt = uniform(nx_cnt);
+        nx_off = uniform(nx_off);
+#pragma unroll
+        for (int d = 0; d < 3; ++d) nx_key[d] = uniform(nx_key[d]);
+        while (nx_b < nb && !in_range(nx_cnt, nx_off)) {  // an empty (enlarged-only) block
+          nx_b += gridDim.x;
+          if (nx_b >= nb) break;
+          nx_cnt = uniform(sv.counts[nx_b]);
+          nx_off = uniform(sv.offsets[nx_b]);
+#pragma unroll
+          for (int d = 0; d < 3; ++d) nx_key[d] = uniform(t.active[3 * (int64_t)nx_b + d]);
+        }
+      } else {
+        nx_cnt = cnt;
+        nx_off = off;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) nx_key[d] = key[d];
+        nx_c0 = c0 + kChunk;
+      }
+      const bool more = nx_b < nb;
+      if (more) load_indices(nx_cnt, nx_off, nx_c0);
       // ---- C: rounds, lane = main cell
       {
         const int32_t lcount = ccount[lane];
@@ -634,6 +605,7 @@ __global__ __launch_bounds__(p2g_threads(kTile), 3) void p2g_kernel(ParticlesVie
                 ar[n] = v;
               }
           }
+          if (a == 0 && more) load_rows(pre[0]);  // in flight across the other slabs and the flush
         }
       }
       // ---- overflow particles (rare): global atomics straight into the grid
@@ -673,15 +645,23 @@ __global__ __launch_bounds__(p2g_threads(kTile), 3) void p2g_kernel(ParticlesVie
           }
         }
       }
-      if (last && threadIdx.x == 0) bucket_meta(nxt, nb, sv, t, ps.n, bmeta, nscenes);
       __syncthreads();
-    }
-    prefetch();  // the next bucket's first-chunk indices (bmeta is the next bucket's now)
-    // the next bucket's first chunk finds its cell counters cleared (they are
-    // not read from here on; the barrier after the flush orders the clear)
-    for (int c = threadIdx.x; c <= kMainCells; c += kT) {
-      ccount[c] = 0;
-      cfill[c] = 0;
+      // the next item finds its cell counters cleared (they are not read from
+      // here on; the barrier after the flush orders the clear)
+      for (int c = threadIdx.x; c <= kMainCells; c += kT) {
+        ccount[c] = 0;
+        cfill[c] = 0;
+      }
+      b = nx_b;
+      cnt = nx_cnt;
+      off = nx_off;
+      c0 = nx_c0;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) key[d] = nx_key[d];
+      if (!last) {  // the bucket's next chunk adds to the same arenas
+        __syncthreads();
+        continue;
+      }
     }
     // ---- flush: sum the wave arenas, one global atomic per touched node/channel
     for (int n = threadIdx.x; n < kArena6; n += kT) {
@@ -711,6 +691,7 @@ __global__ __launch_bounds__(p2g_threads(kTile), 3) void p2g_kernel(ParticlesVie
         }
       }
     }
+    if (b >= nb) break;
     __syncthreads();
   }
 }
@@ -844,9 +825,10 @@ __device__ __forceinline__ void resolve_general(const GeneralCollider& c, const 
 // k; cols is the kernel argument or a scene's colliders in a batch.
 // kLocal: k0_local is the key's first component with a batch's scene offset
 // removed; otherwise the table's own key is read.
-template <bool kLocal = false, typename Cols>
+// kGen: general colliders or a level-set boundary are set.
+template <bool kLocal, bool kGen, typename Cols, typename Gen>
 __device__ __forceinline__ void node_velocity(float* gp, float mass, int fold, float e0, float e1, float e2,
-                                              const Cols& cols, const GeneralColliders& gen, const TableView& t,
+                                              const Cols& cols, const Gen& gen, const TableView& t,
                                               int32_t b, int32_t k0_local, int cell, float dx, float& vmax) {
   // rounded as written (no FMA contraction): a node on a collider plane has
   // phi = 0 in exact arithmetic, and the sign of the rounded phi must be the
@@ -861,7 +843,7 @@ __device__ __forceinline__ void node_velocity(float* gp, float mass, int fold, f
   }
   float v[3] = {mv0 * inv + e0, mv1 * inv + e1, mv2 * inv + e2};
   vmax = fmaxf(vmax, v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-  if (mass > 0.f && (cols.n > 0 || gen.n > 0 || gen.ls.on)) {
+  if (mass > 0.f && (cols.n > 0 || kGen)) {
     const int32_t k0 = kLocal ? k0_local : t.active[3 * (int64_t)b];
     const int32_t k1 = t.active[3 * (int64_t)b + 1], k2 = t.active[3 * (int64_t)b + 2];
     const float pos[3] = {((float)k0 * 4.f + (float)((cell >> 4) & 3)) * dx,
@@ -884,20 +866,27 @@ __device__ __forceinline__ void node_velocity(float* gp, float mass, int fold, f
         }
       }
     }
-    for (int c = 0; c < gen.n; ++c) resolve_general(gen.c[c], pos, v);
-    if (gen.ls.on) levelset_resolve(gen.ls, pos, v);
+    if constexpr (kGen) {
+      for (int c = 0; c < gen.n; ++c) resolve_general(gen.c[c], pos, v);
+      if (gen.ls.on) levelset_resolve(gen.ls, pos, v);
+    }
   }
   gp[1 * kBlockCells] = v[0];
   gp[2 * kBlockCells] = v[1];
   gp[3 * kBlockCells] = v[2];
 }
 
-template <bool kMulti>
+// Gen: GeneralColliders, or NoColliders where none are set: the general
+// colliders' code (180 KB with the level set) and arguments stay out of the
+// ordinary update.
+struct NoColliders {};
+template <bool kMulti, typename Gen>
 __global__ __launch_bounds__(kThreads) void grid_update_kernel(float* __restrict__ grid, int32_t grid_cap,
                                                                TableView t, float dt, float g0, float g1,
                                                                float g2, Colliders cols, float dx, int fold,
                                                                uint32_t* counters, uint32_t* err, SceneSet ss,
-                                                               GeneralColliders gen) {
+                                                               Gen gen) {
+  constexpr bool kGen = std::is_same<Gen, GeneralColliders>::value;
   int32_t nb = *t.cnt;
   if (nb > grid_cap) {
     if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(err, kErrCapacity);
@@ -921,10 +910,10 @@ __global__ __launch_bounds__(kThreads) void grid_update_kernel(float* __restrict
           const int32_t sc = scene_of_key(k0, ss.n);
           const SceneParams& sp = ss.p[sc];
           k0 -= sc * kSceneKeyStride;
-          node_velocity<true>(gp, mass, fold, sp.g[0] * sp.dt, sp.g[1] * sp.dt, sp.g[2] * sp.dt, sp.cols, gen, t, b,
+          node_velocity<true, kGen>(gp, mass, fold, sp.g[0] * sp.dt, sp.g[1] * sp.dt, sp.g[2] * sp.dt, sp.cols, gen, t, b,
                               k0, cell, sp.dx, vmax);
         } else {
-          node_velocity(gp, mass, fold, e0, e1, e2, cols, gen, t, b, 0, cell, dx, vmax);
+          node_velocity<false, kGen>(gp, mass, fold, e0, e1, e2, cols, gen, t, b, 0, cell, dx, vmax);
         }
       } else if (fold) {
         // the fold covers every node, massless ones included (their
@@ -1077,18 +1066,9 @@ __global__ __launch_bounds__(kT) void g2p_kernel(ParticlesView ps, ParticlesView
         if (ps.logJp) ljcopy = ns.lj_src ? ns.lj_src[p] : ps.logJp[p];
         idcopy = ps.id ? ps.id[p] : (int32_t)p;
       }
-      if (contig) {
-        RowLoad<3> lx;
-        RowLoad<9> lf;
-        lx.issue(ps.x, p0, cw);
-        lf.issue(ps.F, p0, cw);
-        lx.finish(stage, cw, x);
-        lf.finish(stage, cw, F);
-      } else if (live) {
-#pragma unroll
-        for (int d = 0; d < 3; ++d) x[d] = ps.x[3 * p + d];
-#pragma unroll
-        for (int k = 0; k < 9; ++k) F[k] = ps.F[9 * p + k];
+      if (live) {
+        load_row(ps.x, p, x);
+        load_row(ps.F, p, F);
       }
       Arena ar;
       make_arena(x[0], x[1], x[2], dx, ar);
@@ -1528,41 +1508,31 @@ int g2p_groups(const Workspace& ws, const SortView& sv, int32_t grid_cap) {
 
 hipError_t p2g_scatter(const ParticlesView& ps, const TableView& t, const SortView& sv, float* grid,
                        int32_t grid_cap, float dt, float dx, bool fold, Workspace& ws, hipStream_t s,
-                       bool reset_queue, const SceneSet* ss, const StressFrom& st) {
+                       const SceneSet* ss, const StressFrom& st) {
   const int g = p2g_groups(ws, sv, grid_cap);
-  if (reset_queue) reset_queue_kernel<<<1, 1, 0, s>>>(ws.counters);
-  uint32_t* q = ws.counters + kCtrQueue;
   const bool multi = ss && ss->n > 0;
   const SceneSet sset = multi ? *ss : SceneSet{};
   const bool tile1 = ws.p2g_tile == 1;  // the folded launches take the tuned tile
   if (fold && ws.cell && !multi)  // the substep's P2C2G (one tile)
     p2g_kernel<0, false, true><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx,
-                                                         ws.err, q, sset, 1);
+                                                         ws.err, sset, 1);
   else if (fold && multi && tile1)
     p2g_kernel<0, true, false, 1><<<g, p2g_threads(1), 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx,
-                                                               ws.err, q, sset, 1);
+                                                               ws.err, sset, 1);
   else if (fold && multi)
-    p2g_kernel<0, true><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, q,
-                                                  sset, 1);
+    p2g_kernel<0, true><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, sset, 1);
   else if (fold && tile1)
     p2g_kernel<0, false, false, 1><<<g, p2g_threads(1), 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt,
-                                                                dx, ws.err, q, sset, 1);
+                                                                dx, ws.err, sset, 1);
   else if (fold)
-    p2g_kernel<0, false><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, q,
-                                                   sset, 1);
+    p2g_kernel<0, false><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, sset, 1);
   else if (multi) {
     // the force kept in channels 4..6: momentum, then the force
-    p2g_kernel<1, true><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, q,
-                                                  sset, 1);
-    reset_queue_kernel<<<1, 1, 0, s>>>(ws.counters);
-    p2g_kernel<2, true><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, q,
-                                                  sset, 4);
+    p2g_kernel<1, true><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, sset, 1);
+    p2g_kernel<2, true><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, sset, 4);
   } else {
-    p2g_kernel<1, false><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, q,
-                                                   sset, 1);
-    reset_queue_kernel<<<1, 1, 0, s>>>(ws.counters);
-    p2g_kernel<2, false><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, q,
-                                                   sset, 4);
+    p2g_kernel<1, false><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, sset, 1);
+    p2g_kernel<2, false><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, sset, 4);
   }
   return hipGetLastError();
 }
@@ -1570,9 +1540,8 @@ hipError_t p2g_scatter(const ParticlesView& ps, const TableView& t, const SortVi
 hipError_t p2c2g_scatter(const ParticlesView& ps, const TableView& t, const SortView& sv, float* grid,
                          int32_t grid_cap, float dt, float dx, Workspace& ws, hipStream_t s, const StressFrom& st) {
   const int g = p2g_groups(ws, sv, grid_cap);
-  reset_queue_kernel<<<1, 1, 0, s>>>(ws.counters);
   p2g_kernel<0, false, true><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx,
-                                                       ws.err, ws.counters + kCtrQueue, SceneSet{}, 1);
+                                                       ws.err, SceneSet{}, 1);
   return hipGetLastError();
 }
 
@@ -1580,9 +1549,7 @@ hipError_t p2g_force_scatter(const ParticlesView& ps, const TableView& t, const 
                              int32_t grid_cap, float dt, float dx, Workspace& ws, hipStream_t s,
                              const StressFrom& st) {
   const int g = p2g_groups(ws, sv, grid_cap);
-  reset_queue_kernel<<<1, 1, 0, s>>>(ws.counters);
-  p2g_kernel<2, false><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err,
-                                                 ws.counters + kCtrQueue, SceneSet{}, 1);
+  p2g_kernel<2, false><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, SceneSet{}, 1);
   return hipGetLastError();
 }
 
@@ -1605,15 +1572,22 @@ hipError_t g2c2p(const ParticlesView& ps, const TableView& t, const SortView& sv
 hipError_t grid_update(float* grid, int32_t grid_cap, const TableView& t, float dt, const float extf[3],
                        const Colliders& cols, float dx, int fold_rhs, Workspace& ws, hipStream_t s,
                        const SceneSet* ss, const GeneralColliders* gen) {
-  const GeneralColliders g = gen ? *gen : GeneralColliders{};
-  if (ss && ss->n > 0)
-    grid_update_kernel<true><<<persistent_groups(), kThreads, 0, s>>>(grid, grid_cap, t, dt, extf[0], extf[1],
-                                                                     extf[2], cols, dx, fold_rhs, ws.counters,
-                                                                     ws.err, *ss, g);
-  else
-    grid_update_kernel<false><<<persistent_groups(), kThreads, 0, s>>>(grid, grid_cap, t, dt, extf[0], extf[1],
-                                                                      extf[2], cols, dx, fold_rhs, ws.counters,
-                                                                      ws.err, SceneSet{}, g);
+  const bool multi = ss && ss->n > 0;
+  const SceneSet sset = multi ? *ss : SceneSet{};
+  auto launch = [&](auto kernel, auto g) {
+    kernel<<<persistent_groups(), kThreads, 0, s>>>(grid, grid_cap, t, dt, extf[0], extf[1], extf[2], cols, dx,
+                                                    fold_rhs, ws.counters, ws.err, sset, g);
+  };
+  if (gen && (gen->n > 0 || gen->ls.on)) {
+    if (multi)
+      launch(grid_update_kernel<true, GeneralColliders>, *gen);
+    else
+      launch(grid_update_kernel<false, GeneralColliders>, *gen);
+  } else if (multi) {
+    launch(grid_update_kernel<true, NoColliders>, NoColliders{});
+  } else {
+    launch(grid_update_kernel<false, NoColliders>, NoColliders{});
+  }
   return hipGetLastError();
 }
 

@@ -90,6 +90,12 @@ __device__ __forceinline__ uint64_t mix64(uint64_t z) {
   return z;
 }
 
+// a positive normal power of two: x / d and x * (1 / d) round alike
+__device__ __forceinline__ bool is_pow2(float d) {
+  const uint32_t u = __float_as_uint(d);
+  return (u & 0x7fffffu) == 0u && u > 0x00800000u && u < 0x7e800000u;
+}
+
 // ---------------------------------------------------------------------------
 // wavefront helpers (wave64)
 // ---------------------------------------------------------------------------
@@ -183,6 +189,23 @@ struct RowLoad {
     wave_lds_barrier();
   }
 };
+
+// Row p of W floats (W a multiple of 3) by one lane, in 12-byte loads (rows are
+// 4-byte aligned). Consecutive lanes read consecutive rows: the three loads of
+// a 9-float row touch the same lines one after another.
+typedef float zs_f3 __attribute__((ext_vector_type(3), aligned(4)));
+template <int W>
+__device__ __forceinline__ void load_row(const float* __restrict__ base, int64_t p, float (&out)[W]) {
+  static_assert(W % 3 == 0, "rows of 3-vectors");
+  const float* r = base + (int64_t)W * p;
+#pragma unroll
+  for (int k = 0; k < W; k += 3) {
+    const zs_f3 t = *reinterpret_cast<const zs_f3*>(r + k);
+    out[k] = t.x;
+    out[k + 1] = t.y;
+    out[k + 2] = t.z;
+  }
+}
 
 // One-shot form: issue and finish.
 template <int W>
@@ -700,9 +723,14 @@ __device__ __forceinline__ int series_sand(const Model& m, const float* F, float
   const float trE = E[0] + E[1] + E[2];
   const float sum_eps = trE - 3.f * m.cohesion;
   const float tr = sum_eps + logJp;
-  const float shift = m.cohesion + tr / 3.f;  // eps - tr/3: the deviator zpc projects (logJp included)
+  const float shift = m.cohesion + tr * (1.f / 3.f);  // eps - tr/3: the deviator zpc projects (logJp included)
   const float d0 = E[0] - shift, d1 = E[1] - shift, d2 = E[2] - shift;
-  const float ehn = sqrtf(d0 * d0 + d1 * d1 + d2 * d2 + 2.f * (E[3] * E[3] + E[4] * E[4] + E[5] * E[5]));
+  // its norm and inverse norm from one reciprocal root and a Newton step (0 and
+  // a huge number at a zero deviator, which is never projected)
+  const float eh2 = d0 * d0 + d1 * d1 + d2 * d2 + 2.f * (E[3] * E[3] + E[4] * E[4] + E[5] * E[5]);
+  float inv = __builtin_amdgcn_rsqf(fmaxf(eh2, 1e-37f));
+  inv = inv * (1.5f - 0.5f * eh2 * inv * inv);
+  const float ehn = eh2 * inv;
   const float smu = 2.f * m.mu;
   int which = 1;
   float keep = 1.f, add = 0.f;  // H = keep E + add I
@@ -717,8 +745,8 @@ __device__ __forceinline__ int series_sand(const Model& m, const float* F, float
     const float dg = ehn + kt;
     if (!(dg <= 0.f)) {
       which = 3;  // E - dg / ehn (E - shift I)
-      keep = -kt / ehn;
-      add = dg / ehn * shift;
+      keep = -kt * inv;
+      add = dg * inv * shift;
     }
   }
   const float iso = (m.lambda * (keep * trE + 3.f * add) + smu * add) * m.volume;
@@ -875,9 +903,11 @@ struct Arena {
 __device__ __forceinline__ void make_arena(float x0, float x1, float x2, float dx, Arena& ar) {
 #pragma clang fp contract(off)
   const float xs[3] = {x0, x1, x2};
+  const bool pow2 = is_pow2(dx);
+  const float dx_inv = 1.f / dx;
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
-    const float X = xs[d] / dx;
+    const float X = pow2 ? xs[d] * dx_inv : xs[d] / dx;
     const int32_t b = (int32_t)floorf(X - 0.5f);
     const float l = X - (float)b;
     const float d0 = l - (float)(int32_t)floorf(l - 0.5f);

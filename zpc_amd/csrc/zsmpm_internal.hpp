@@ -133,7 +133,6 @@ enum : int {
   kCtrFp64 = 3,     // particles that took the FP64 SVD path
   kCtrFallback = 4, // particles that took the SVD fallback of the learned closure
   kCtrMaxVel = 5,   // max |v|^2 as float bits
-  kCtrQueue = 6,    // next bucket of the running per-bucket launch
   kCtrFbQueue = 7,  // length of the closure's SVD fallback queue (per pass)
   kCtrNetQueue = 8, // waves the closure's network pass took (per pass)
   kCtrNetWaves = 9, // waves that evaluated the closure's network (all passes)
@@ -258,7 +257,7 @@ size_t rank_scratch_words();
 // buckets (counts and offsets after build_enlarge, indices after build_place)
 // and errors are those of table_clear, table_activate, table_enlarge and
 // bucket_sort; ws.nbr holds the neighbours of the blocks with particles.
-// build_clear also resets the P2G bucket queue and the max |v|^2 counter.
+// build_clear also resets the max |v|^2 counter.
 // ss (a batch): each particle's key uses its scene's dx and is shifted by the
 // scene's key offset
 hipError_t build_clear(const TableView& t, Workspace& ws, int64_t n, hipStream_t s);
@@ -300,7 +299,7 @@ hipError_t closure_launch_limits();
 // bucket's or node's scene, read from its block key
 hipError_t p2g_scatter(const ParticlesView& ps, const TableView& t, const SortView& sv, float* grid,
                        int32_t grid_cap, float dt, float dx, bool fold, Workspace& ws, hipStream_t s,
-                       bool reset_queue = true, const SceneSet* ss = nullptr, const StressFrom& st = StressFrom{});
+                       const SceneSet* ss = nullptr, const StressFrom& st = StressFrom{});
 // P2C2GTransfer as a scatter of each particle's cell-kernel stencil (folded
 // into m and mv, channels 0..3)
 hipError_t p2c2g_scatter(const ParticlesView& ps, const TableView& t, const SortView& sv, float* grid,
