@@ -836,7 +836,7 @@ int32_t substeps_driver(zsmpm_policy_s* pol, const zsmpm_model* model, const zsm
   if ((flags & ZSMPM_SUBSTEPS_AUTOTUNE) && nsteps >= 8 && !fuse) {
     DeviceGuard g(pol->devid);
     const int32_t cand_p2g[4] = {1024, 2048, 2048, 4096}, cand_g2p[4] = {32768, 65536, 32768, 65536};
-    const int32_t cand_p2g_tile[4] = {0, 0, 1, 1}, cand_g2p_threads[4] = {128, 128, 256, 256};
+    const int32_t cand_p2g_tile[4] = {0, 0, 1, 1}, cand_g2p_threads[4] = {0, 0, 256, 256};
     const bool prof = pol->profile;
     ZS_HIP(hipStreamSynchronize(pol->stream));
     harvest_events(pol);
@@ -1858,7 +1858,7 @@ int32_t zsmpm_policy_set_launch_tiles__rocm(zsmpm_policy pol, int32_t p2g_chunk,
       (g2p_threads != 0 && g2p_threads != 128 && g2p_threads != 256))
     return ZSMPM_INVALID_ARGUMENT;
   pol->tuned_p2g_tile = p2g_chunk == 256 ? 1 : 0;
-  pol->tuned_g2p_threads = g2p_threads == 256 ? 256 : 0;
+  pol->tuned_g2p_threads = g2p_threads;
   return ZSMPM_OK;
 }
 

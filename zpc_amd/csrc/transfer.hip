@@ -56,14 +56,29 @@ __device__ __forceinline__ int vel_at(int r0, int r1, int r2) { return r0 * kVel
 // (the register limit, 4 waves per SIMD) keep more buckets' loads in flight
 // than four workgroups of four waves (0.82 -> 0.79 ms at 16M particles)
 constexpr int kG2PThreads = 128;
+// G2P of a small scene: as many waves as a full bucket has rounds of rows. With
+// two, a bucket's rounds ran one after another while most CUs idled: substep
+// 84 -> 74 us at 64K particles, 95 -> 91 at 256K, equal at 512K (1,000 buckets
+// of two waves fill the card).
+constexpr int kG2PWide = 512;
+constexpr int64_t kG2PWideParticles = 262144;
 constexpr int kP2GThreads = 256;  // one workgroup per bucket
 constexpr int kP2GWaves = kP2GThreads / kWave;
 // Launch tiles the autotuner chooses between. P2G tile 0: four waves and
 // chunks of Rec::kChunk particles (a whole bucket of up to 576, three
 // workgroups per CU); tile 1: two waves and chunks of 256 (six workgroups per
 // CU, for sparser buckets). G2P: 128 or 256 threads per bucket.
-constexpr int p2g_threads(int tile) { return tile == 0 ? kP2GThreads : 128; }
-constexpr int p2g_chunk(int tile, int fold_chunk) { return tile == 0 ? fold_chunk : 256; }
+// kWideTile, P2G of a small scene: a wave per round of a full bucket's rows
+// (records and scatter in one round each, no serial chain of three). One such
+// workgroup fits a CU, so it pays while a CU has no second bucket: up to 256
+// buckets of some 300 particles, counting the partly filled ones at a body's
+// surface. Substep 70.3 -> 65.4 us at 4K particles, 74.1 -> 70.8 at 64K; past
+// the line 76.7 -> 80.9 at 96K (343 buckets). Splitting a bucket over four
+// workgroups instead gained 3 us at 4K and lost 15 at 64K.
+constexpr int64_t kP2GWideParticles = 256 * 300;
+constexpr int kWideTile = 2, kWideP2GThreads = 576;
+constexpr int p2g_threads(int tile) { return tile == kWideTile ? kWideP2GThreads : tile == 1 ? 128 : kP2GThreads; }
+constexpr int p2g_chunk(int tile, int fold_chunk) { return tile == 1 ? 256 : fold_chunk; }
 
 inline int groups_for(int64_t n, int threads) {
   int64_t g = (n + threads - 1) / threads;
@@ -1015,6 +1030,10 @@ __global__ __launch_bounds__(kT) void g2p_kernel(ParticlesView ps, ParticlesView
     const int32_t cnt = sv.counts[b];
     const int32_t off = sv.offsets[b];
     if (cnt <= 0 || off < 0 || (int64_t)off + cnt > ps.n) continue;
+    // the wave's first 64 particles: indices, then rows, load while the
+    // velocities are staged
+    int32_t pnext = -1;
+    if (wave * kWave + lane < cnt) pnext = sv.indices[off + wave * kWave + lane];
     load_neighbours(nbr_tab, b, nbr, err);
     int32_t k0 = t.active[3 * (int64_t)b];
     // the bucket's grid spacing and time step (its scene's, in a batch)
@@ -1028,10 +1047,22 @@ __global__ __launch_bounds__(kT) void g2p_kernel(ParticlesView ps, ParticlesView
       D_inv = 4.f * dx_inv * dx_inv;
     }
     const int32_t o0 = k0 * 4, o1 = t.active[3 * (int64_t)b + 1] * 4, o2 = t.active[3 * (int64_t)b + 2] * 4;
-    // the wave's first 64 particle indices load while the velocities are staged
-    int32_t first = -1;
-    if (wave * kWave + lane < cnt) first = sv.indices[off + wave * kWave + lane];
     __syncthreads();
+    // x, F and the attributes the reorder only moves, of the next round; an
+    // index out of range loads row 0, which nobody uses
+    float xr[3], Fr[9], mr = 0.f, ljr = 0.f;
+    int32_t idr = 0;
+    auto load_ahead = [&](int32_t q) {
+      if (q < 0 || q >= ps.n) q = 0;
+      load_row(ps.x, q, xr);
+      load_row(ps.F, q, Fr);
+      if (kReorder) {
+        mr = ps.m[q];
+        if (ps.logJp) ljr = ns.lj_src ? ns.lj_src[q] : ps.logJp[q];
+        idr = ps.id ? ps.id[q] : q;
+      }
+    };
+    load_ahead(pnext);
     // stage node velocities: slot s -> (neighbour block s>>6, cell s&63), stored at vel_at(r0, r1, r2)
     for (int s = threadIdx.x; s < kArena8; s += kT) {
       const int nbi = s >> 6, cell = s & 63;
@@ -1051,25 +1082,21 @@ __global__ __launch_bounds__(kT) void g2p_kernel(ParticlesView ps, ParticlesView
     for (int32_t i0 = wave * kWave; i0 < cnt; i0 += kT) {
       const int32_t cw = min(kWave, cnt - i0);
       const bool valid = lane < cw;
-      const int64_t p = valid ? (int64_t)(i0 == wave * kWave ? first : sv.indices[off + i0 + lane]) : -1;
+      const int64_t p = pnext;
+      const bool more = i0 + kT < cnt;  // uniform across the wave
+      if (more) pnext = i0 + kT + lane < cnt ? sv.indices[off + i0 + kT + lane] : -1;
       const bool bad = valid && (p < 0 || p >= ps.n);
       if (bad) atomicOr(err, kErrCapacity);
       const bool live = valid && !bad;
       int64_t p0;
       const bool contig = wave_contiguous(p, live, p0) && ballot(bad) == 0;
-      float x[3] = {0.f, 0.f, 0.f}, F[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      // the attributes the reorder only moves, loaded with the rest
-      float mcopy = 0.f, ljcopy = 0.f;
-      int32_t idcopy = 0;
-      if (kReorder && live) {
-        mcopy = ps.m[p];
-        if (ps.logJp) ljcopy = ns.lj_src ? ns.lj_src[p] : ps.logJp[p];
-        idcopy = ps.id ? ps.id[p] : (int32_t)p;
-      }
-      if (live) {
-        load_row(ps.x, p, x);
-        load_row(ps.F, p, F);
-      }
+      float x[3], F[9];
+#pragma unroll
+      for (int d = 0; d < 3; ++d) x[d] = xr[d];
+#pragma unroll
+      for (int k = 0; k < 9; ++k) F[k] = Fr[k];
+      const float mcopy = mr, ljcopy = ljr;
+      const int32_t idcopy = idr;
       Arena ar;
       make_arena(x[0], x[1], x[2], dx, ar);
       if constexpr (kCell) {
@@ -1154,6 +1181,7 @@ __global__ __launch_bounds__(kT) void g2p_kernel(ParticlesView ps, ParticlesView
           C[k] = outside ? ps.C[9 * p + k] : 0.f;
         }
       }
+      if (more) load_ahead(pnext);
       if (kReorder) {
         // destination slots off + i0 + lane are contiguous by construction
         const int64_t q = (int64_t)off + i0 + lane;
@@ -1441,6 +1469,9 @@ hipError_t check_launch_limits(int device) {
       reinterpret_cast<const void*>(&g2p_kernel<false, -1, false, true>),
       reinterpret_cast<const void*>(&p2g_kernel<0, false, false, 1>),
       reinterpret_cast<const void*>(&p2g_kernel<0, true, false, 1>),
+      reinterpret_cast<const void*>(&p2g_kernel<0, false, false, kWideTile>),
+      reinterpret_cast<const void*>(&g2p_kernel<true, -1, false, false, kG2PWide>),
+      reinterpret_cast<const void*>(&g2p_kernel<false, -1, false, false, kG2PWide>),
       reinterpret_cast<const void*>(&g2p_kernel<true, -1, false, false, 256>),
       reinterpret_cast<const void*>(&g2p_kernel<true, -1, true, false, 256>),
       reinterpret_cast<const void*>(&g2p2g_gather_kernel),
@@ -1524,6 +1555,9 @@ hipError_t p2g_scatter(const ParticlesView& ps, const TableView& t, const SortVi
   else if (fold && tile1)
     p2g_kernel<0, false, false, 1><<<g, p2g_threads(1), 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt,
                                                                 dx, ws.err, sset, 1);
+  else if (fold && ps.n <= kP2GWideParticles)
+    p2g_kernel<0, false, false, kWideTile><<<g, p2g_threads(kWideTile), 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid,
+                                                                               grid_cap, dt, dx, ws.err, sset, 1);
   else if (fold)
     p2g_kernel<0, false><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx, ws.err, sset, 1);
   else if (multi) {
@@ -1629,6 +1663,13 @@ hipError_t g2p(const ParticlesView& ps, const ParticlesView* out, const TableVie
   } else if (out && ws.g2p_threads == 256) {
     g2p_kernel<true, -1, false, false, 256><<<g, 256, 0, s>>>(ps, *out, t, sv, ws.nbr, grid, grid_cap, dt, dx, ns,
                                                               ws.err, ws.counters, sset);
+  } else if (sset.n == 0 && ws.g2p_threads == 0 && ps.n <= kG2PWideParticles) {
+    if (out)
+      g2p_kernel<true, -1, false, false, kG2PWide><<<g, kG2PWide, 0, s>>>(ps, *out, t, sv, ws.nbr, grid, grid_cap, dt,
+                                                                          dx, ns, ws.err, ws.counters, sset);
+    else
+      g2p_kernel<false, -1, false, false, kG2PWide><<<g, kG2PWide, 0, s>>>(ps, ps, t, sv, ws.nbr, grid, grid_cap, dt,
+                                                                           dx, ns, ws.err, ws.counters, sset);
   } else if (out) {
     g2p_kernel<true, -1><<<g, kG2PThreads, 0, s>>>(ps, *out, t, sv, ws.nbr, grid, grid_cap, dt, dx, ns, ws.err,
                                                    ws.counters, sset);
