@@ -271,11 +271,11 @@ hipError_t exclusive_scan_u32(const uint32_t* in, uint32_t* out, const uint32_t*
 }
 
 hipError_t exclusive_scan_popc_u32(const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* scratch,
-                                   hipStream_t s) {
+                                   hipStream_t s, uint32_t* total_out) {
   if (n == 0) return hipSuccess;
   const uint32_t G = groups_for_cap(n);
   scan_reduce_kernel<true><<<G, kThreads, 0, s>>>(in, nullptr, n, scratch);
-  scan_small_kernel<1><<<1, kSmallThreads, 0, s>>>(scratch, G, nullptr);
+  scan_small_kernel<1><<<1, kSmallThreads, 0, s>>>(scratch, G, total_out);
   scan_down_kernel<true><<<G, kThreads, 0, s>>>(in, out, nullptr, n, scratch);
   return hipGetLastError();
 }

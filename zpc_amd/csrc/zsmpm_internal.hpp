@@ -237,7 +237,7 @@ hipError_t exclusive_scan_u32(const uint32_t* in, uint32_t* out, const uint32_t*
                               uint32_t* tile_sums, uint32_t* total_out, hipStream_t s);
 // exclusive scan of the population counts of n words
 hipError_t exclusive_scan_popc_u32(const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* scratch,
-                                   hipStream_t s);
+                                   hipStream_t s, uint32_t* total_out = nullptr);
 hipError_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_t* vals_alt,
                             const uint32_t* n_dev, uint32_t n_cap, int bits, uint32_t* scratch,
                             hipStream_t s, bool* result_in_alt);
