@@ -18,8 +18,9 @@ using namespace zsmpm;
 struct zsmpm_policy_s {
   int devid = 0;
   hipStream_t stream = nullptr;
-  // second stream of the substep: the stress pass runs on it while the
-  // sparsity stages run on `stream` (created on first use, default priority)
+  // second stream of the substep: a stress pass of its own (closure, FP64
+  // gap) runs on it while the sparsity stages run on `stream` (created on
+  // first use, default priority)
   hipStream_t side = nullptr;
   hipEvent_t fork_ev = nullptr, join_ev = nullptr;
   // captured pair of substeps (ZSMPM_SUBSTEPS_GRAPH): the capture stream, the
@@ -829,13 +830,13 @@ int32_t substeps_driver(zsmpm_policy_s* pol, const zsmpm_model* model, const zsm
   // Autotuning: the first 8 substeps (real ones, in pairs a -> b -> a) run
   // with four P2G and four G2P launch configurations (tile and workgroup
   // count), timed per kernel with the stage events; each kernel keeps its
-  // fastest. P2G: four waves with 576-particle chunks at 1,024 and 2,048
+  // fastest. P2G: four waves with 576-particle chunks at 1,024 and 768 (resident)
   // workgroups, two waves with 256-particle chunks at 2,048 and 4,096; G2P:
   // 128 and 256 threads per bucket at 32,768 and 65,536 workgroups.
   int32_t done = 0;
   if ((flags & ZSMPM_SUBSTEPS_AUTOTUNE) && nsteps >= 8 && !fuse) {
     DeviceGuard g(pol->devid);
-    const int32_t cand_p2g[4] = {1024, 2048, 2048, 4096}, cand_g2p[4] = {32768, 65536, 32768, 65536};
+    const int32_t cand_p2g[4] = {1024, 768, 2048, 4096}, cand_g2p[4] = {32768, 65536, 32768, 65536};
     const int32_t cand_p2g_tile[4] = {0, 0, 1, 1}, cand_g2p_threads[4] = {0, 0, 256, 256};
     const bool prof = pol->profile;
     ZS_HIP(hipStreamSynchronize(pol->stream));
@@ -1821,8 +1822,8 @@ int32_t zsmpm_policy_colliders__rocm(zsmpm_policy pol, const zsmpm_collider* col
   return ZSMPM_OK;
 }
 
-// P2G takes buckets from a work queue and G2P strides over them, so any
-// positive workgroup count is correct; the bound keeps a grid launchable.
+// P2G and G2P stride over the buckets, so any positive workgroup count is
+// correct; the bound keeps a grid launchable.
 constexpr int32_t kMaxLaunchGroups = 1 << 20;
 
 int32_t zsmpm_policy_launch_widths__rocm(zsmpm_policy pol, int32_t* p2g_groups, int32_t* g2p_groups) {
