@@ -44,7 +44,7 @@ def stage_bytes(stage: str, n: int, blocks: int, plastic: bool, table_size: int)
     nodes = 64 * blocks
     lj = 4 if plastic else 0
     if stage == "p2g":
-        # read x, v, C, vol P F^T, m and the bucket permutation; flush m and the
+        # read x, v, C, F (or a stress pass's vol P F^T), m and the bucket permutation; flush m and the
         # force-folded momentum (4 channels) once per node
         return n * (12 + 12 + 36 + 36 + 4 + 4) + nodes * 16
     if stage == "g2p":
