@@ -19,7 +19,9 @@ hipError_t table_clear(const TableView&, Workspace&, hipStream_t s) { return tou
 hipError_t table_activate(const TableView&, Workspace&, const float*, int64_t, float, int, int, float, hipStream_t s) { return touch(s); }
 hipError_t build_clear(const TableView&, Workspace&, int64_t, hipStream_t s) { return touch(s); }
 hipError_t build_activate(const TableView&, Workspace&, const float*, int64_t, float, hipStream_t s, const SceneSet* ss) { return scenes_ok(ss, s); }
-hipError_t build_enlarge(const TableView&, Workspace&, int64_t, const SortView&, hipStream_t s) { return touch(s); }
+hipError_t build_enlarge(const TableView&, Workspace&, int64_t, const SortView&, float*, int32_t, hipStream_t s) {
+  return touch(s);
+}
 hipError_t build_place(const TableView&, Workspace&, int64_t, const SortView&, hipStream_t s) { return touch(s); }
 size_t rank_scratch_words() { return 64; }
 hipError_t table_enlarge(const TableView&, Workspace&, const int32_t*, const int32_t*, int32_t, hipStream_t s) { return touch(s); }

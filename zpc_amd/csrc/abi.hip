@@ -593,15 +593,11 @@ int32_t run_substep(zsmpm_policy_s* pol, const zsmpm_model* model, const zsmpm_p
   }
   {
     StageScope sc(pol, ZSMPM_STAGE_ENLARGE);
-    ZS_HIP(build_enlarge(t, ws, ps.n, sv, s));
+    ZS_HIP(build_enlarge(t, ws, ps.n, sv, grid->data, grid->capacity_blocks, s));
   }
   {
     StageScope sc(pol, ZSMPM_STAGE_BUCKET_SORT);
     ZS_HIP(build_place(t, ws, ps.n, sv, s));
-  }
-  {
-    StageScope sc(pol, ZSMPM_STAGE_GRID_CLEAR);
-    ZS_HIP(zsmpm::grid_clear(grid->data, t.cnt, grid->capacity_blocks, s));
   }
   ZS_HIP(side.join());
   {

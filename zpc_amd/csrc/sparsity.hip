@@ -773,11 +773,14 @@ __device__ __forceinline__ void counts_scan(const uint64_t* __restrict__ bcnt, i
 
 // The last of the build's bookkeeping: the keys[] of every placed block (block
 // r probes from its home until it finds the slot holding r), the block count,
-// the neighbours' block numbers in place of their slots, the bucket offsets.
+// the neighbours' block numbers in place of their slots, the bucket offsets, and
+// the grid channels of every block cleared: a launch of its own for that cost 2 us
+// of a small substep (77.2 -> 74.8 at 4K particles) and 18 at 16M.
 __global__ __launch_bounds__(kThreads) void build_finish_kernel(TableView t, uint32_t* counters, uint32_t* err,
                                                                 const int32_t* __restrict__ slot_block, uint32_t ts,
                                                                 int32_t* nbr, const uint64_t* __restrict__ bcnt,
-                                                                SortView sv, uint32_t* segoff) {
+                                                                SortView sv, uint32_t* segoff,
+                                                                float4* __restrict__ grid, int32_t grid_cap) {
   __shared__ uint64_t lds[2 * (kThreads / kWave)];
   const int64_t na = min((int64_t)counters[kCtrList], (int64_t)t.T);
   const int64_t nb = min((int64_t)counters[kCtrList] + counters[kCtrListB], (int64_t)t.T);
@@ -807,6 +810,8 @@ __global__ __launch_bounds__(kThreads) void build_finish_kernel(TableView t, uin
     const uint32_t sl = (uint32_t)nbr[i];
     nbr[i] = sl < ts ? slot_block[sl] : -1;
   }
+  const int64_t quads = min(nb, (int64_t)grid_cap) * (kChannels * kBlockCells / 4);
+  for (int64_t i = i0; i < quads; i += stride) grid[i] = make_float4(0.f, 0.f, 0.f, 0.f);
   counts_scan(bcnt, (int32_t)min(na, (int64_t)sv.cap_blocks), sv, segoff, lds);
 }
 
@@ -1339,7 +1344,8 @@ hipError_t build_activate(const TableView& t, Workspace& ws, const float* x, int
   return hipGetLastError();
 }
 
-hipError_t build_enlarge(const TableView& t, Workspace& ws, int64_t n, const SortView& sv, hipStream_t s) {
+hipError_t build_enlarge(const TableView& t, Workspace& ws, int64_t n, const SortView& sv, float* grid,
+                         int32_t grid_cap, hipStream_t s) {
   uint32_t* mask2 = ws.dmask + (ws.ts_cap / 32 + 1);
   const Ranks ra = ranks_a(ws, n), rb = ranks_b(ws, t);
   build_number_kernel<true><<<number_groups(ra, ws.ts_cap, 1024), kThreads, 4 * padded(ra.groups), s>>>(
@@ -1351,8 +1357,9 @@ hipError_t build_enlarge(const TableView& t, Workspace& ws, int64_t n, const Sor
   build_number_kernel<false><<<number_groups(rb, ws.ts_cap, 256), kThreads, 4 * padded(rb.groups), s>>>(
       ws.counters + kCtrListB, ws.counters + kCtrList, ws.lb_key, ws.lb_val, rb, t, dedup_of(ws), mask2,
       ws.slot_block, ws.scnt, ws.bcnt, ws.nbr);
-  build_finish_kernel<<<few(ws.ts_cap, 1024), kThreads, 0, s>>>(t, ws.counters, ws.err, ws.slot_block, ws.ts_cap, ws.nbr, ws.bcnt, sv,
-                                              ws.segoff);
+  build_finish_kernel<<<few(ws.ts_cap, 2048), kThreads, 0, s>>>(t, ws.counters, ws.err, ws.slot_block, ws.ts_cap,
+                                                                ws.nbr, ws.bcnt, sv, ws.segoff,
+                                                                reinterpret_cast<float4*>(grid), grid_cap);
   return hipGetLastError();
 }
 

@@ -257,13 +257,15 @@ size_t rank_scratch_words();
 // buckets (counts and offsets after build_enlarge, indices after build_place)
 // and errors are those of table_clear, table_activate, table_enlarge and
 // bucket_sort; ws.nbr holds the neighbours of the blocks with particles.
+// build_enlarge also clears the grid channels of every block.
 // build_clear also resets the max |v|^2 counter.
 // ss (a batch): each particle's key uses its scene's dx and is shifted by the
 // scene's key offset
 hipError_t build_clear(const TableView& t, Workspace& ws, int64_t n, hipStream_t s);
 hipError_t build_activate(const TableView& t, Workspace& ws, const float* x, int64_t n, float dx, hipStream_t s,
                           const SceneSet* ss);
-hipError_t build_enlarge(const TableView& t, Workspace& ws, int64_t n, const SortView& sv, hipStream_t s);
+hipError_t build_enlarge(const TableView& t, Workspace& ws, int64_t n, const SortView& sv, float* grid,
+                         int32_t grid_cap, hipStream_t s);
 hipError_t build_place(const TableView& t, Workspace& ws, int64_t n, const SortView& out, hipStream_t s);
 // ws.nbr for every active block (the 2x2x2 blocks a bucket's stencils cover)
 hipError_t block_neighbours(const TableView& t, Workspace& ws, hipStream_t s);
