@@ -47,6 +47,34 @@ def test_insert_edges(T, n, run):
     assert np.all(got[first & (rank >= T - 20)] == O.BHT_FAILURE)
 
 
+def test_insert_far_over_the_table_on_used_scratch():
+    """More distinct keys than the table's hash takes, and more than the waves
+    in flight hold: tiles that begin after the hash was found full are skipped,
+    and what the scratch holds there from another insertion must not be read."""
+    import torch
+    from zpc_amd import rocm
+
+    pol = rocm.Policy()
+    g = torch.Generator().manual_seed(5)
+    keys = torch.randint(-400000, 400000, (5000011, 3), generator=g, dtype=torch.int32)  # all distinct
+    # another layout of the same scratch, filled with slots, indices and packed keys
+    big = rocm.DeviceBht(1 << 20, pol)
+    big.insert((keys % 64).contiguous().cuda())
+    pol.sync()
+    assert big.size() == 64 ** 3
+    T = 64
+    t = rocm.DeviceBht(T, pol)
+    got = t.insert(keys.cuda()).cpu().numpy()
+    with pytest.raises(rocm.ZsmpmError) as e:
+        pol.sync()
+    assert e.value.code == -7
+    rank = np.arange(keys.shape[0])
+    assert np.all((got == rank) | (got == O.BHT_FAILURE))
+    assert np.all(got[T - 20:] == O.BHT_FAILURE)
+    kept = got[got != O.BHT_FAILURE]
+    assert np.array_equal(t.active.cpu().numpy()[kept], keys.numpy()[kept])
+
+
 @pytest.mark.parametrize("order", ["sorted", "shuffled"])
 @pytest.mark.parametrize("n", [1, 65, 30001])
 def test_sample_orders(n, order):

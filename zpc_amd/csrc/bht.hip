@@ -111,8 +111,10 @@ __global__ __launch_bounds__(kBT) void dedup_clear_kernel(uint64_t* skey, uint32
 // common: neighbouring particles share a block), and only those (head, a bit
 // per key) are looked at again. slot_of is written for every key where kAll,
 // else for the heads.
-// A key that finds no slot in kProbes steps raises *full and the caller starts
-// again with the hash sized for n distinct keys. What bounds it is the latency
+// A key that finds no slot in kProbes steps raises *full; the tiles not yet
+// begun are then skipped (their head and slot_of stay as they were, and nothing
+// reads them) and the caller starts again with the hash sized for n distinct
+// keys. What bounds it is the latency
 // of the probe, so a thread takes four keys in a row (a run that a wave
 // boundary cuts goes to the hash once per 256 keys) and an index that cannot
 // lower a slot's minimum (a few blocks collect all runs) does no atomic. With
@@ -187,17 +189,20 @@ __global__ __launch_bounds__(kBT) void dedup_insert_kernel(Keys keys, int64_t n,
   }
 }
 
-// a bit per key: the first occurrence of a key the table does not hold yet. A
-// thread per byte of head: few bits are set where neighbours share a block, and
-// eight in a row are the most it follows.
+// a bit per key: the first occurrence of a key the table does not hold yet; none
+// after a hash that was too small (*full), whose skipped tiles left head and
+// slot_of unwritten. A thread per byte of head: few bits are set where
+// neighbours share a block, and eight in a row are the most it follows.
 template <typename Keys>
 __global__ __launch_bounds__(kBT) void first_kernel(Keys keys, int64_t n, int64_t bytes,
                                                     const uint8_t* __restrict__ head, const uint32_t* slot_of,
-                                                    const uint32_t* smin, BhtView t, uint8_t* __restrict__ flag) {
+                                                    const uint32_t* smin, const uint32_t* full, BhtView t,
+                                                    uint8_t* __restrict__ flag) {
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  const bool complete = *full == 0u;
   for (int64_t w = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; w < bytes; w += stride) {
     uint32_t out = 0;
-    for (uint32_t bits = 8 * w < n ? head[w] : 0u; bits; bits &= bits - 1u) {
+    for (uint32_t bits = complete && 8 * w < n ? head[w] : 0u; bits; bits &= bits - 1u) {
       const int b = __ffs(bits) - 1;
       const int64_t i = 8 * w + b;
       const uint32_t s = slot_of[i];
@@ -540,8 +545,8 @@ int32_t insert_keys(const BhtView& t, const Keys& keys, int64_t n, int32_t* out,
     dedup_clear_kernel<<<groups_n(S), kBT, 0, s>>>(c.skey, c.smin, S, c.total);
     dedup_insert_kernel<kAll><<<groups_n(n, kBT * kDedupItems), kBT, 0, s>>>(keys, n, c.skey, c.smin, S, bounded,
                                                                             c.slot_of, c.head, c.total + 1, err);
-    first_kernel<<<groups_n(8 * words), kBT, 0, s>>>(keys, n, 8 * words, c.head, c.slot_of, c.smin, t,
-                                                    (uint8_t*)c.flag);
+    first_kernel<<<groups_n(8 * words), kBT, 0, s>>>(keys, n, 8 * words, c.head, c.slot_of, c.smin,
+                                                    c.total + 1, t, (uint8_t*)c.flag);
     e = exclusive_scan_popc_u32(c.flag, c.rank, (uint32_t)(2 * words), c.scan, s, c.total);
     if (e != hipSuccess) return ZSMPM_DEVICE_ERROR;
     compact_kernel<<<groups_n(2 * words), kBT, 0, s>>>(keys, 2 * words, c.flag, c.rank, c.nk, c.level);
