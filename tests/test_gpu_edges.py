@@ -185,3 +185,50 @@ def test_key_range_reported(sand):
         sim2.substep()
         sim2.sync()
     assert ei.value.code == -8
+
+
+def test_more_blocks_than_the_table_on_a_larger_scratch():
+    """A table of 64 slots under a policy reserved for 4,096 and buckets with
+    room for 512 blocks: the scratch numbers more blocks than the table holds.
+    The substep reports TABLE_FULL and writes nothing outside the buckets'
+    arrays; the same policy then runs the scene on a table that holds it."""
+    import torch
+
+    rocm = _rocm()
+    sc = S.tiny_scene(n_cells=(24, 24, 24), dx=1.0 / 64, lo=(12, 13, 14))
+    room = dataclasses.replace(sc, table_size=4096)
+    sim = rocm.Simulator(room, reorder=True, grid_capacity=512)
+    sim.substep()  # leaves its block numbers and offsets in the scratch
+    sim.sync()
+    assert 64 < sim.nblocks() <= 512
+    guard, n, cap = 4096, sc.n, 512
+    whole = {k: torch.full((guard + size + guard,), -77, dtype=torch.int32, device="cuda")
+             for k, size in (("counts", cap + 1), ("offsets", cap + 1), ("indices", n))}
+    size = {"counts": cap + 1, "offsets": cap + 1, "indices": n}
+    b = type(sim.buckets.desc).from_buffer_copy(sim.buckets.desc)
+    b.capacity_blocks = cap
+    for k in whole:
+        setattr(b, k, whole[k].data_ptr() + 4 * guard)
+    small = rocm.DeviceTable(64)
+    grid = rocm.DeviceGrid(sc.dx, cap)
+    for _ in range(2):
+        rocm.check(sim.L.zsmpm_substep_sorted__rocm(
+            sim.pol.h, C.byref(sim.model), C.byref(sim.parts.desc), C.byref(sim.spare.desc), C.byref(small.desc),
+            C.byref(b), C.byref(grid.desc), float(sc.dt), C.byref(sim.extf), sim.cols, sim.ncols), "substep_sorted")
+        with pytest.raises(rocm.ZsmpmError) as ei:
+            sim.sync()
+        assert ei.value.code == -7
+        for k, t in whole.items():
+            assert bool((t[:guard] == -77).all()) and bool((t[guard + size[k]:] == -77).all()), k
+        off = whole["offsets"][guard:guard + cap + 1].cpu().numpy()
+        assert np.all((off >= 0) & (off <= n))
+    x = sim.parts.x.clone()
+    sim.substep()
+    sim.sync()
+    ref = rocm.Simulator(dataclasses.replace(room, x=x.cpu().numpy(), v=sim.spare.v.cpu().numpy(),
+                                             C=sim.spare.C.cpu().numpy(), F=sim.spare.F.cpu().numpy()), reorder=True,
+                         grid_capacity=512)
+    ref.substep()
+    ref.sync()
+    assert np.array_equal(sim.table.host()["keys"], ref.table.host()["keys"])
+    assert np.array_equal(sim.buckets.indices.cpu().numpy(), ref.buckets.indices.cpu().numpy())

@@ -1238,11 +1238,14 @@ hipError_t table_query(const TableView& t, const int32_t* keys, int64_t n, int32
 namespace {
 
 // segments counted per block (bcnt) and scanned (offsets, segoff): the lists
-// and the buckets' indices. slot_block as in segment_emit_kernel.
-hipError_t place_segments(Workspace& ws, int64_t n, const int32_t* slot_block, const int32_t* nblocks,
-                          const SortView& out, hipStream_t s) {
+// and the buckets' indices. slot_block as in segment_emit_kernel. *nblocks may
+// exceed T where a larger scratch took more keys than the table (reported as
+// full): only the first T blocks were numbered, counted and scanned.
+hipError_t place_segments(const TableView& t, Workspace& ws, int64_t n, const int32_t* slot_block,
+                          const int32_t* nblocks, const SortView& out, hipStream_t s) {
   const int64_t tiles = (n + tile_size(n) - 1) / tile_size(n);
-  const int32_t cap = out.cap_blocks < (int32_t)ws.ts_cap ? out.cap_blocks : (int32_t)ws.ts_cap;
+  int32_t cap = out.cap_blocks < (int32_t)ws.ts_cap ? out.cap_blocks : (int32_t)ws.ts_cap;
+  cap = cap < t.T ? cap : t.T;
   const int ge = groups_for(tiles * kWave, kThreads), gc = groups_for((int64_t)cap + 1, kThreads * 4);
   segment_emit_kernel<<<ge > gc ? ge : gc, kThreads, 0, s>>>(segments_of(ws, nullptr), n, tile_size(n), slot_block, ws.ts_cap,
                                                              ws.segoff, ws.bcnt, nblocks, cap, out, ws.seg_list,
@@ -1271,7 +1274,7 @@ hipError_t bucket_sort(const TableView& t, Workspace& ws, const float* x, int64_
                                                                   segments_of(ws, ws.bcnt), cap, ws.err);
   const int gs = (cap + 1023) / 1024;
   counts_scan_kernel<<<gs < 1024 ? gs : 1024, kThreads, 0, s>>>(ws.bcnt, t.cnt, cap, out, ws.segoff);
-  return place_segments(ws, n, nullptr, t.cnt, out, s);
+  return place_segments(t, ws, n, nullptr, t.cnt, out, s);
 }
 
 // ------------------------------------------------------- the substep's build
@@ -1364,7 +1367,7 @@ hipError_t build_enlarge(const TableView& t, Workspace& ws, int64_t n, const Sor
 }
 
 hipError_t build_place(const TableView& t, Workspace& ws, int64_t n, const SortView& out, hipStream_t s) {
-  return place_segments(ws, n, ws.slot_block, reinterpret_cast<const int32_t*>(ws.counters + kCtrList), out, s);
+  return place_segments(t, ws, n, ws.slot_block, reinterpret_cast<const int32_t*>(ws.counters + kCtrList), out, s);
 }
 
 }  // namespace zsmpm
