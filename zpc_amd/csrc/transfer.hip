@@ -142,12 +142,20 @@ __device__ __forceinline__ void lane_cell(int l, int& i, int& j, int& k) {
   j = ((l >> 3) & 1) | (((l >> 5) & 1) << 1);
 }
 
-// quadratic B-spline weights from the local position l in [0.5, 1.5)
-// (quadratic_bspline_weights, math/curve/InterpolationKernel.hpp:95-130, whose
-// floor(l - 0.5) is 0 there: l is X - floor(X - 0.5), exact for X >= 0.5)
-__device__ __forceinline__ void bspline_w(float l, float (&w)[3]) {
+// The quadratic B-spline's argument (quadratic_bspline_weights,
+// math/curve/InterpolationKernel.hpp:95-130): the local position l = X -
+// floor(X - 0.5) less floor(l - 0.5). That floor is 0 for X >= 0.5, where l is
+// exact; at negative X the rounding of X - 0.5 can leave l just below 0.5 (X =
+// -127.50001 has base -128) and the floor is -1, as in make_arena. It is taken
+// once per record, not in the scatter's three passes.
+__device__ __forceinline__ float bspline_arg(float l) {
 #pragma clang fp contract(off)
-  const float d0 = l;
+  return l - (float)(int32_t)floorf(l - 0.5f);
+}
+
+// its weights on the nodes base .. base + 2
+__device__ __forceinline__ void bspline_w(float d0, float (&w)[3]) {
+#pragma clang fp contract(off)
   w[0] = 0.5f * (1.5f - d0) * (1.5f - d0);
   const float d1 = d0 - 1.0f;
   w[1] = 0.75f - d1 * d1;
@@ -169,6 +177,7 @@ __device__ __forceinline__ void cell_w(float l, float (&w)[3]) {
   w[2] = t * 0.5f;
 }
 
+// weights from a record's l: the local position (cell kernel) or bspline_arg of it
 template <bool kCell>
 __device__ __forceinline__ void stencil_w(float l, float (&w)[3]) {
   if constexpr (kCell)
@@ -190,7 +199,8 @@ __device__ __forceinline__ void cell_dinv(const float (&x)[3], float dx, float d
 }
 
 // Record layout (float4 units): q0 = (m, B0, B1, B2), q1 = (l0, l1, l2, A8),
-// q2 = A0..A3, q3 = A4..A7 with A column-major (A[d + 3e]) already times dx.
+// q2 = A0..A3, q3 = A4..A7 with A column-major (A[d + 3e]) already times dx; l
+// is the argument of stencil_w.
 struct Rec {
   static constexpr int kQuads = 4;
   // particles staged per pass. 576 (nine waves) holds a whole bucket at 8
@@ -483,6 +493,9 @@ __global__ __launch_bounds__(p2g_threads(kTile), 3) void p2g_kernel(ParticlesVie
 #pragma unroll
         for (int d = 0; d < 3; ++d) Bv[d] = mv[d] - (A[d] * l[0] + A[d + 3] * l[1] + A[d + 6] * l[2]);
         rec[0 * kChunk + i] = make_float4(mass, Bv[0], Bv[1], Bv[2]);
+        if constexpr (!kCell)
+#pragma unroll
+          for (int d = 0; d < 3; ++d) l[d] = bspline_arg(l[d]);
         rec[1 * kChunk + i] = make_float4(l[0], l[1], l[2], A[8]);
         rec[2 * kChunk + i] = make_float4(A[0], A[1], A[2], A[3]);
         rec[3 * kChunk + i] = make_float4(A[4], A[5], A[6], A[7]);
