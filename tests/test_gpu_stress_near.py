@@ -91,3 +91,32 @@ def test_stress_series_and_svd(kind, scale, turn):
     if kind == S.DRUCKER_PRAGER:
         ljtol = np.where(near, 3e-6 * strain + 3 * floor, 1e-3)
         assert np.all(np.abs(dl.cpu().numpy() - lj_ref) <= ljtol + 1e-30)
+
+
+@pytest.mark.parametrize("stretch", [1e3, 2.0e6, 2.2e6, 2.5e6, 1e9])
+def test_stress_of_huge_stretches(stretch):
+    """Isotropic stretches around 2e6, where det(F F^T + I) is finite and its
+    reciprocal is not: sand at the cone's tip, H = cohesion on each axis and
+    logJp raised by the whole volume strain. log sigma is a float32 logarithm
+    (2 ulp) and H exact up to its rounding: 1e-5."""
+    import torch
+
+    from zpc_amd import rocm
+
+    n = 65
+    mat = S.Material.drucker_prager(3.5e5, 0.3, 1e3, volume=1e-6, cohesion=1e-3)
+    F = np.zeros((n, 9), np.float32)
+    F[:, ::4] = np.float32(stretch) * (1 + np.arange(n, dtype=np.float32)[:, None] / 1024)
+    F[0, ::4] = 1.0  # a near lane in the same wave
+    dF, dl = torch.as_tensor(F).cuda(), torch.zeros(n, dtype=torch.float32, device="cuda")
+    PF = torch.empty((n, 9), dtype=torch.float32, device="cuda")
+    pol = rocm.Policy()
+    model = rocm.model_desc(mat)
+    rocm.check(pol.L.zsmpm_stress__rocm(pol.h, rocm.C.byref(model), dF.data_ptr(), dl.data_ptr(), n, PF.data_ptr()),
+               "stress")
+    pol.sync()
+    M = F.astype(np.float64).reshape(n, 3, 3).transpose(0, 2, 1)
+    ref, _, _, lj = _reference(mat, M, np.zeros(n))
+    assert np.allclose(dl.cpu().numpy()[1:], lj[1:], rtol=1e-5, atol=0)
+    got = PF.cpu().numpy().reshape(n, 3, 3).transpose(0, 2, 1)
+    assert np.allclose(got[1:], ref[1:], rtol=1e-5, atol=1e-5 * np.abs(ref[1:]).max())

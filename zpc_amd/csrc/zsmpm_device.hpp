@@ -585,6 +585,11 @@ struct NearB {
   float i1, i2, i3;        // invariants of Z
 };
 constexpr float kNearZ2 = 0.09f;  // largest ||Z||_F^2 of the series
+// No ||A||_F^2 above this is near: A's eigenvalues are a = 2 z / (1 - z), so |z| <=
+// 0.3 gives |a| <= |z| 2 / 0.7 and the sum of a^2 at most 0.09 (2 / 0.7)^2 = 0.7347.
+// It is looked at before det(b + I), which overflows its reciprocal for stretches
+// beyond 2e6 (Z would come out 0), and ends a far wave's attempt early.
+constexpr float kNearA2 = 0.74f;
 
 __device__ __forceinline__ void sym_mul(const float (&a)[6], const float (&b)[6], float (&c)[6]) {
   // product of two symmetric matrices that commute (so it is symmetric)
@@ -607,8 +612,10 @@ __device__ __forceinline__ bool near_identity(const float* F, NearB& n) {
     const int i = I[k], j = J[k];
     n.A[k] = (G[i + 3 * j] + G[j + 3 * i]) + (G[i] * G[j] + G[i + 3] * G[j + 3] + G[i + 6] * G[j + 6]);
   }
-  // (b + I)^-1 from the adjugate; b + I >= I, so the determinant is >= 1
   const float (&A)[6] = n.A;
+  if (!(A[0] * A[0] + A[1] * A[1] + A[2] * A[2] + 2.f * (A[3] * A[3] + A[4] * A[4] + A[5] * A[5]) <= kNearA2))
+    return false;
+  // (b + I)^-1 from the adjugate; b + I >= I, so the determinant is >= 1
   const float m0 = 2.f + A[0], m1 = 2.f + A[1], m2 = 2.f + A[2];
   float adj[6];
   adj[0] = m1 * m2 - A[5] * A[5];
