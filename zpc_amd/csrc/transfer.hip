@@ -213,10 +213,12 @@ struct Rec {
 // Per-particle constitutive part of P2G (P2G.hpp:57-100): vol P F^T from the
 // stored F (fixed-corotated or the Drucker-Prager return mapping, which
 // writes logJp back). Particles in array order, 64 consecutive per wave, so
-// rows always move as 16-byte vectors.
+// the results leave as 16-byte vectors.
 // kKind: 0 fixed-corotated, 1 Drucker-Prager, 2 each particle its scene's
-// model (a batch, ss)
-template <int kKind>
+// model (a batch, ss; only where some scene has the FP64 SVD on). kGap: the
+// model has the FP64 SVD on; its code stays out of the other instances, which
+// it held to three waves per SIMD
+template <int kKind, bool kGap>
 __global__ __launch_bounds__(kThreads) void stress_kernel(Model m, ParticlesView ps, float* __restrict__ contrib,
                                                           uint32_t* counters, SceneSet ss) {
   __shared__ float4 stage4[kWaves][stage_floats(9) / 4];
@@ -229,37 +231,37 @@ __global__ __launch_bounds__(kThreads) void stress_kernel(Model m, ParticlesView
     for (int i = threadIdx.x; i <= ss.n; i += kThreads) sfirst[i] = ss.first[i];
     __syncthreads();
   }
-  // The next group's F rows and logJp are in flight while this group's SVD
-  // runs (stress pass 0.70 -> 0.67 ms beside the sparsity stages at 16M
-  // particles). Two groups ahead made the pass faster still (0.61 ms) but
-  // took enough of the machine to slow the bucket sort beside it by more.
-  RowLoad<9> ld;
+  // The next group's F row and logJp are in flight while this group's SVD runs
+  // (stress pass 0.70 -> 0.67 ms beside the sparsity stages at 16M particles).
+  // Two groups ahead made the pass faster still (0.61 ms) but took enough of the
+  // machine to slow the bucket sort beside it by more. Each lane loads its own
+  // row (through LDS 125 -> 128 us for 4.2M strained particles with the FP64 SVD
+  // on: vector instructions bound it); past the end row 0, which nobody uses.
+  float Fn[9], lj_next = 0.f;
   int64_t w = (int64_t)blockIdx.x * kWaves + wave;
-  float lj_next = 0.f;
-  if (w * kWave < ps.n) {
-    const int64_t q0 = w * kWave;
-    const int32_t qw = (int32_t)min((int64_t)kWave, ps.n - q0);
-    ld.issue(ps.F, q0, qw);
-    if (kKind == 1 && lane < qw) lj_next = ps.logJp[q0 + lane];
-  }
+  auto load = [&](int64_t group) {
+    int64_t q = group * kWave + lane;
+    if (q >= ps.n) q = 0;
+    load_row(ps.F, q, Fn);
+    if (kKind == 1) lj_next = ps.logJp[q];
+  };
+  if (w * kWave < ps.n) load(w);
   for (; w * kWave < ps.n; w += nwaves) {
     const int64_t p0 = w * kWave;
     const int32_t cw = (int32_t)min((int64_t)kWave, ps.n - p0);
     const int64_t p = p0 + lane;
     float F[9], PF[9];
     float lj = lj_next;
-    ld.finish(stage, cw, F);
-    const int64_t wn = w + nwaves;
-    if (wn * kWave < ps.n) {
-      const int64_t q0 = wn * kWave;
-      const int32_t qw = (int32_t)min((int64_t)kWave, ps.n - q0);
-      ld.issue(ps.F, q0, qw);
-      if (kKind == 1 && lane < qw) lj_next = ps.logJp[q0 + lane];
-    }
+#pragma unroll
+    for (int k = 0; k < 9; ++k) F[k] = Fn[k];
+    if ((w + nwaves) * kWave < ps.n) load(w + nwaves);
     if (lane < cw) {
       bool f64 = false;
-      if (kKind != 2) {
-        stress_any(m, F, lj, PF, f64);
+      if constexpr (kKind != 2) {
+        if constexpr (kGap)
+          stress_gap(m, F, lj, PF, f64);
+        else
+          stress_plain(m, F, lj, PF);
         if (kKind == 1) ps.logJp[p] = lj;
       } else {
         const Model ms = ss.p[scene_of_particle(sfirst, ss.n, p)].model;
@@ -1466,8 +1468,9 @@ hipError_t check_launch_limits(int device) {
   hipError_t e = hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device);
   if (e != hipSuccess) return e;
   const void* kernels[] = {
-      reinterpret_cast<const void*>(&stress_kernel<0>), reinterpret_cast<const void*>(&stress_kernel<1>),
-      reinterpret_cast<const void*>(&stress_kernel<2>), reinterpret_cast<const void*>(&p2g_kernel<0, false>),
+      reinterpret_cast<const void*>(&stress_kernel<0, false>), reinterpret_cast<const void*>(&stress_kernel<1, false>),
+      reinterpret_cast<const void*>(&stress_kernel<0, true>), reinterpret_cast<const void*>(&stress_kernel<1, true>),
+      reinterpret_cast<const void*>(&stress_kernel<2, true>), reinterpret_cast<const void*>(&p2g_kernel<0, false>),
       reinterpret_cast<const void*>(&p2g_kernel<1, false>), reinterpret_cast<const void*>(&p2g_kernel<0, true>),
       reinterpret_cast<const void*>(&p2g_kernel<1, true>),
       reinterpret_cast<const void*>(&g2p_kernel<false, -1>), reinterpret_cast<const void*>(&g2p_kernel<true, -1>),
@@ -1491,7 +1494,7 @@ hipError_t check_launch_limits(int device) {
     hipFuncAttributes attr;
     e = hipFuncGetAttributes(&attr, kernels[i]);
     if (e != hipSuccess) return e;
-    const size_t extra = i < 3 ? kStressLdsReserve : 0;  // the stress kernels' reserve
+    const size_t extra = i < 5 ? kStressLdsReserve : 0;  // the stress kernels' reserve
     if (attr.sharedSizeBytes + extra > (size_t)max_lds) return hipErrorInvalidConfiguration;
   }
   return closure_launch_limits();
@@ -1510,17 +1513,20 @@ hipError_t stress(const Model& m, const ParticlesView& ps, Workspace& ws, hipStr
   const int64_t waves = (ps.n + kWave - 1) / kWave;
   const int g = groups_for(waves * kWave, kThreads);
   const size_t lds = beside_sparsity ? kStressLdsReserve : 0;
-  if (ss && ss->n > 0) {
-    if (closure) return hipErrorNotSupported;
-    stress_kernel<2><<<g, kThreads, lds, s>>>(m, ps, out, ws.counters, *ss);
+  const bool multi = ss && ss->n > 0;
+  const SceneSet sset = multi ? *ss : SceneSet{};
+  auto launch = [&](auto kernel) {
+    kernel<<<g, kThreads, lds, s>>>(m, ps, out, ws.counters, sset);
     return hipGetLastError();
+  };
+  if (multi) {  // a batch without the FP64 SVD has no stress pass
+    if (closure) return hipErrorNotSupported;
+    return launch(stress_kernel<2, true>);
   }
   if (closure && m.kind == 1 && m.mu != 0.f) return stress_closure(m, *closure, ps, out, ws, s);
-  if (m.kind == 0)
-    stress_kernel<0><<<g, kThreads, lds, s>>>(m, ps, out, ws.counters, SceneSet{});
-  else
-    stress_kernel<1><<<g, kThreads, lds, s>>>(m, ps, out, ws.counters, SceneSet{});
-  return hipGetLastError();
+  const bool gap = m.fp64_gap > 0.f;
+  if (m.kind == 0) return gap ? launch(stress_kernel<0, true>) : launch(stress_kernel<0, false>);
+  return gap ? launch(stress_kernel<1, true>) : launch(stress_kernel<1, false>);
 }
 
 namespace {

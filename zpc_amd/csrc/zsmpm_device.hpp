@@ -237,6 +237,11 @@ __device__ __forceinline__ void wave_store_rows(float* __restrict__ base, int64_
   wave_lds_barrier();
 }
 
+// The SVD and the stress up to the arena below: products are fused with sums
+// within an expression (decided once, here), not across statements by each
+// kernel's own schedule, so that instances agree bit by bit.
+#pragma clang fp contract(on)
+
 // ---------------------------------------------------------------------------
 // 3x3 SVD: McAdams et al. 2011 ("Computing the SVD of 3x3 matrices with
 // minimal branching and elementary floating point operations"), the method
@@ -652,20 +657,21 @@ __device__ __forceinline__ void near_poly(const NearB& n, const float (&p)[N], f
   }
 }
 
-// P F^T volume for P = U diag(Ph) V^T (the tail both models share).
-__device__ __forceinline__ void pft_volume(const float (&U)[3][3], const float (&Ph)[3],
-                                           const float (&V)[3][3], const float* F, float vol,
-                                           float* PF) {
-  float P[3][3];
+// P F^T = U diag(tau) U^T of an isotropic model, tau the principal Kirchhoff
+// stresses (times the volume): with F = U diag(s) V^T and P = U diag(Ph) V^T,
+// tau_i = Ph_i s_i and V^T V = I drops out. Symmetric: 6 entries, and V is not
+// needed past A V. Against 64 bits it is closer than P F^T multiplied out,
+// which keeps the four-sweep SVD's residual (strains of 0.3 to 1: 2.4e-5, 2.1e-5
+// and 2.3e-5 of the 2-norm against 2.5e-5, 3.9e-5 and 5.7e-5).
+__device__ __forceinline__ void kirchhoff(const float (&U)[3][3], const float (&tau)[3], float* PF) {
 #pragma unroll
   for (int i = 0; i < 3; ++i)
 #pragma unroll
-    for (int j = 0; j < 3; ++j) P[i][j] = Ph[0] * U[i][0] * V[j][0] + Ph[1] * U[i][1] * V[j][1] + Ph[2] * U[i][2] * V[j][2];
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j)
-      PF[i + 3 * j] = (P[i][0] * F[j] + P[i][1] * F[j + 3] + P[i][2] * F[j + 6]) * vol;
+    for (int j = i; j < 3; ++j) {
+      const float e = U[i][0] * tau[0] * U[j][0] + U[i][1] * tau[1] * U[j][1] + U[i][2] * tau[2] * U[j][2];
+      PF[i + 3 * j] = e;
+      PF[j + 3 * i] = e;
+    }
 }
 
 // Fixed-corotated near the identity; false: out of the series' range (nothing written).
@@ -703,13 +709,14 @@ __device__ __forceinline__ bool series_fixedcorotated(const Model& m, const floa
 
 // Fixed-corotated from the SVD: Ph_i = 2 mu (s_i - 1) + lambda (J - 1) prod_{j!=i} s_j.
 __device__ __forceinline__ void svd_fixedcorotated(const Model& m, const float (&U)[3][3], const float (&S)[3],
-                                                   const float (&V)[3][3], const float* F, float* PF) {
+                                                   float* PF) {
   const float J = S[0] * S[1] * S[2];
   const float smu = 2.f * m.mu;
   const float slam = m.lambda * (J - 1.f);
-  const float Ph[3] = {smu * (S[0] - 1.f) + slam * (S[1] * S[2]), smu * (S[1] - 1.f) + slam * (S[0] * S[2]),
-                       smu * (S[2] - 1.f) + slam * (S[0] * S[1])};
-  pft_volume(U, Ph, V, F, m.volume, PF);
+  const float tau[3] = {(smu * (S[0] - 1.f) + slam * (S[1] * S[2])) * S[0] * m.volume,
+                        (smu * (S[1] - 1.f) + slam * (S[0] * S[2])) * S[1] * m.volume,
+                        (smu * (S[2] - 1.f) + slam * (S[0] * S[1])) * S[2] * m.volume};
+  kirchhoff(U, tau, PF);
 }
 
 // Sand near the identity: the return mapping of stress_sand on the tensor E.
@@ -767,12 +774,14 @@ __device__ __forceinline__ int series_sand(const Model& m, const float* F, float
   return which;
 }
 
-// Drucker-Prager with volume correction, from the SVD; F is projected locally
-// (the stored F is left alone), logJp is updated. Returns the case: 1 inside
-// the cone, 2 cone tip, 3 projected to the cone surface, 0 otherwise.
-__device__ __forceinline__ int svd_sand(const Model& m, const float (&U)[3][3], const float (&S)[3],
-                                        const float (&V)[3][3], const float* F, float& logJp, float* PF,
-                                        float* Fproj) {
+// Drucker-Prager with volume correction, from the SVD; logJp is updated. tau_i =
+// Ph_i ns_i = 2 mu ln ns_i + lambda sum_j ln ns_j of the projected F = U diag(ns)
+// V^T: ln ns_i = H_i is the exponent the projection chose (no exp / log round
+// trip, no division). Returns the case: 1 inside the cone, 2 cone tip, 3
+// projected to the cone surface, 0 otherwise (mu = 0 under compression: zpc
+// leaves ns at 0 there, and log 0 over 0 makes every entry NaN).
+__device__ __forceinline__ int svd_sand(const Model& m, const float (&U)[3][3], const float (&S)[3], float& logJp,
+                                        float* PF) {
   const float smu = 2.f * m.mu;
   float eps[3];
 #pragma unroll
@@ -785,11 +794,11 @@ __device__ __forceinline__ int svd_sand(const Model& m, const float (&U)[3][3], 
   const float third = tr / 3.f;
   const float eh[3] = {eps[0] - third, eps[1] - third, eps[2] - third};
   const float ehn = sqrtf(eh[0] * eh[0] + eh[1] * eh[1] + eh[2] * eh[2]);
-  float ns[3] = {0.f, 0.f, 0.f};
+  const float nan = __builtin_nanf("");
+  float H[3] = {nan, nan, nan};
   int which = 0;
   if (tr >= 0.f) {
-    const float e = expf(m.cohesion);
-    ns[0] = ns[1] = ns[2] = e;
+    H[0] = H[1] = H[2] = m.cohesion;
     if (m.volume_correction) logJp = m.beta * sum_eps + logJp;
     which = 2;
   } else if (m.mu != 0.f) {
@@ -797,66 +806,19 @@ __device__ __forceinline__ int svd_sand(const Model& m, const float (&U)[3][3], 
     const float dg = ehn + (3.f * m.lambda + smu) / smu * tr * m.yield_surface;
     if (dg <= 0.f) {
 #pragma unroll
-      for (int i = 0; i < 3; ++i) ns[i] = expf(eps[i] + m.cohesion);
+      for (int i = 0; i < 3; ++i) H[i] = eps[i] + m.cohesion;
       which = 1;
     } else {
       const float r = dg / ehn;
 #pragma unroll
-      for (int i = 0; i < 3; ++i) ns[i] = expf(eps[i] - r * eh[i] + m.cohesion);
+      for (int i = 0; i < 3; ++i) H[i] = eps[i] - r * eh[i] + m.cohesion;
       which = 3;
     }
   }
-  if (which != 0 && !Fproj) {
-    // With the projected F = U diag(ns) V^T and P = U diag(Ph) V^T,
-    // P F^T = U diag(Ph) V^T V diag(ns) U^T = U diag(tau) U^T (V^T V = I to
-    // rounding), tau_i = Ph_i ns_i = 2 mu ln ns_i + lambda sum_j ln ns_j, the
-    // Kirchhoff stress: no division, and ln ns_i is the exponent the
-    // projection chose (no exp / log round trip). Symmetric: 6 entries. It
-    // agrees with the composed form to 1e-6 of the largest entry.
-    float H[3];
-    if (which == 2) {
-      H[0] = H[1] = H[2] = m.cohesion;
-    } else if (which == 1) {
-#pragma unroll
-      for (int i = 0; i < 3; ++i) H[i] = eps[i] + m.cohesion;
-    } else {
-      const float r = (ehn + (3.f * m.lambda + smu) / smu * tr * m.yield_surface) / ehn;
-#pragma unroll
-      for (int i = 0; i < 3; ++i) H[i] = eps[i] - r * eh[i] + m.cohesion;
-    }
-    const float trl = H[0] + H[1] + H[2];
-    const float tau[3] = {(smu * H[0] + m.lambda * trl) * m.volume, (smu * H[1] + m.lambda * trl) * m.volume,
-                          (smu * H[2] + m.lambda * trl) * m.volume};
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int j = i; j < 3; ++j) {
-        const float e = U[i][0] * tau[0] * U[j][0] + U[i][1] * tau[1] * U[j][1] + U[i][2] * tau[2] * U[j][2];
-        PF[i + 3 * j] = e;
-        PF[j + 3 * i] = e;
-      }
-    return which;
-  }
-  // projected F = U diag(ns) V^T (column-major)
-  float Fp[9];
-  if (which != 0) {
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int j = 0; j < 3; ++j)
-        Fp[i + 3 * j] = U[i][0] * ns[0] * V[j][0] + U[i][1] * ns[1] * V[j][1] + U[i][2] * ns[2] * V[j][2];
-  } else {
-#pragma unroll
-    for (int i = 0; i < 9; ++i) Fp[i] = F[i];
-  }
-  const float ls[3] = {logf(ns[0]), logf(ns[1]), logf(ns[2])};
-  const float trl = ls[0] + ls[1] + ls[2];
-  const float Ph[3] = {(smu * ls[0] + m.lambda * trl) / ns[0], (smu * ls[1] + m.lambda * trl) / ns[1],
-                       (smu * ls[2] + m.lambda * trl) / ns[2]};
-  pft_volume(U, Ph, V, Fp, m.volume, PF);
-  if (Fproj)
-#pragma unroll
-    for (int i = 0; i < 9; ++i) Fproj[i] = Fp[i];
+  const float trl = H[0] + H[1] + H[2];
+  const float tau[3] = {(smu * H[0] + m.lambda * trl) * m.volume, (smu * H[1] + m.lambda * trl) * m.volume,
+                        (smu * H[2] + m.lambda * trl) * m.volume};
+  kirchhoff(U, tau, PF);
   return which;
 }
 
@@ -872,30 +834,36 @@ __device__ __forceinline__ void stress_plain(const Model& m, const float* F, flo
   bool fp64;
   svd_colmajor(F, U, S, V, 0.f, fp64);
   if (m.kind == 0)
-    svd_fixedcorotated(m, U, S, V, F, PF);
+    svd_fixedcorotated(m, U, S, PF);
   else
-    (void)svd_sand(m, U, S, V, F, logJp, PF, nullptr);
+    (void)svd_sand(m, U, S, logJp, PF);
 }
 
-// The same of any model: with the FP64 SVD on, a particle with nearly repeated
-// singular values (and fp64 set) takes that, every other one what it gets
-// with it off.
-__device__ __forceinline__ void stress_any(const Model& m, const float* F, float& logJp, float* PF, bool& fp64) {
-  const float lj0 = logJp;
-  fp64 = false;
-  stress_plain(m, F, logJp, PF);
-  if (m.fp64_gap > 0.f) {
-    float U[3][3], S[3], V[3][3];
-    svd_colmajor(F, U, S, V, m.fp64_gap, fp64);
-    if (fp64) {
-      logJp = lj0;
-      if (m.kind == 0)
-        svd_fixedcorotated(m, U, S, V, F, PF);
-      else
-        (void)svd_sand(m, U, S, V, F, logJp, PF, nullptr);
-    }
+// The same of a model with the FP64 SVD on (fp64_gap > 0): a particle with nearly
+// repeated singular values takes that (and sets fp64), every other one what it
+// gets with it off. One float SVD serves the look at the singular values and
+// the particles out of the series' range.
+__device__ __forceinline__ void stress_gap(const Model& m, const float* F, float& logJp, float* PF, bool& fp64) {
+  float U[3][3], S[3], V[3][3];
+  svd_colmajor(F, U, S, V, m.fp64_gap, fp64);
+  if (m.kind == 0) {
+    if (!fp64 && series_fixedcorotated(m, F, PF)) return;
+    svd_fixedcorotated(m, U, S, PF);
+  } else {
+    if (!fp64 && series_sand(m, F, logJp, PF) >= 0) return;
+    (void)svd_sand(m, U, S, logJp, PF);
   }
 }
+
+__device__ __forceinline__ void stress_any(const Model& m, const float* F, float& logJp, float* PF, bool& fp64) {
+  fp64 = false;
+  if (m.fp64_gap > 0.f)
+    stress_gap(m, F, logJp, PF, fp64);
+  else
+    stress_plain(m, F, logJp, PF);
+}
+
+#pragma clang fp contract(fast)
 
 // ---------------------------------------------------------------------------
 // quadratic B-spline arena (simulation/Utils.hpp:51-70): X = x / dx,
