@@ -26,6 +26,7 @@ hipError_t build_place(const TableView&, Workspace&, int64_t, const SortView&, h
 size_t rank_scratch_words() { return 64; }
 hipError_t table_enlarge(const TableView&, Workspace&, const int32_t*, const int32_t*, int32_t, hipStream_t s) { return touch(s); }
 hipError_t table_query(const TableView&, const int32_t*, int64_t, int32_t*, hipStream_t s) { return touch(s); }
+hipError_t count_runs(Workspace&, int64_t, hipStream_t) { return hipSuccess; }
 hipError_t bucket_sort(const TableView&, Workspace&, const float*, int64_t, float, int, int, float, const SortView&, hipStream_t s) { return touch(s); }
 hipError_t block_neighbours(const TableView&, Workspace&, hipStream_t s) { return touch(s); }
 hipError_t check_launch_limits(int) { return hipSuccess; }

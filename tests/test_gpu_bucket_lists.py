@@ -58,3 +58,31 @@ def test_segment_lists_exact(driver, segments, run):
     assert np.array_equal(gc[:k], counts) and not gc[k:].any()
     assert np.array_equal(go[:k], np.cumsum(counts) - counts) and np.all(go[k:] == sc.n)
     assert np.array_equal(gi, want)
+
+
+@pytest.mark.parametrize("driver", ["operator", "substep", "graph"])
+@pytest.mark.parametrize("segments,run", [(2, 1), (6, 640), (130, 70), (300, 256), (9, 1024), (700, 3001)])
+def test_counters_runs_and_new_keys(driver, segments, run):
+    """The diagnostic counters: particle runs of the last bucket sort, whatever
+    tiles the sort cuts them into (both tile sizes), and the new keys of the
+    last insertion (the enlargement's)."""
+    from zpc_amd import rocm
+
+    sc, block = _scene(segments, run, tail=3)
+    sim = rocm.Simulator(sc, reorder=driver == "graph")
+    if driver == "operator":
+        sim.clear_table()
+        sim.activate()
+        sim.sync()
+        assert sim.pol.counters()[0] == 3
+        sim.enlarge()
+        sim.bucket_sort()
+    elif driver == "substep":
+        sim.substep()
+    else:  # particles in bucket order from the second substep on: a run per block
+        sim.substeps(4, graph=True)
+    sim.sync()
+    got = sim.pol.counters()
+    assert got[0] == sim.nblocks() - 3
+    assert got[2] == (3 if driver == "graph" else segments + 1)
+    assert sim.pol.counters()[2] == got[2]

@@ -982,6 +982,12 @@ int32_t zsmpm_policy_counters(zsmpm_policy pol, uint32_t* out) {
   DeviceGuard g(pol->devid);
   ZS_HIP(hipStreamSynchronize(pol->stream));
   ZS_HIP(hipMemcpy(out, pol->ws.counters, sizeof(uint32_t) * kCtrCount, hipMemcpyDeviceToHost));
+  out[kCtrRuns] = 0;
+  if (out[kCtrSorted] > 0) {
+    ZS_HIP(count_runs(pol->ws, out[kCtrSorted], pol->stream));
+    ZS_HIP(hipStreamSynchronize(pol->stream));
+    ZS_HIP(hipMemcpy(out + kCtrRuns, pol->ws.counters + kCtrRuns, sizeof(uint32_t), hipMemcpyDeviceToHost));
+  }
   out[kCtrBhtRounds] = (uint32_t)pol->bht_rounds;
   return ZSMPM_OK;
 }

@@ -610,7 +610,7 @@ __global__ __launch_bounds__(kThreads) void build_clear_kernel(ClearList c, Tabl
   if (i0 == 0) {
     *t.cnt = 0;
     counters[kCtrList] = 0u;
-    counters[kCtrListB] = 0u;
+    counters[kCtrBlocks] = 0u;
     counters[kCtrMaxVel] = 0u;
   }
 }
@@ -782,8 +782,8 @@ __global__ __launch_bounds__(kThreads) void build_finish_kernel(TableView t, uin
                                                                 SortView sv, uint32_t* segoff,
                                                                 float4* __restrict__ grid, int32_t grid_cap) {
   __shared__ uint64_t lds[2 * (kThreads / kWave)];
-  const int64_t na = min((int64_t)counters[kCtrList], (int64_t)t.T);
-  const int64_t nb = min((int64_t)counters[kCtrList] + counters[kCtrListB], (int64_t)t.T);
+  const int64_t na = min((int64_t)counters[kCtrBlocks], (int64_t)t.T);
+  const int64_t nb = min((int64_t)counters[kCtrBlocks] + counters[kCtrList], (int64_t)t.T);
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   const int64_t i0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i0 == 0) {  // nothing in this kernel reads the count
@@ -883,7 +883,6 @@ __global__ __launch_bounds__(kThreads) void counts_scan_kernel(const uint64_t* _
 __global__ __launch_bounds__(kThreads) void segment_emit_kernel(Segments sg, int64_t n, int32_t tile_size,
                                                                 const int32_t* __restrict__ slot_block, uint32_t ts,
                                                                 const uint32_t* __restrict__ segoff,
-                                                                const uint64_t* __restrict__ bcnt,
                                                                 const int32_t* nblocks, int32_t cap, SortView sv,
                                                                 uint64_t* __restrict__ list, uint32_t* counters,
                                                                 uint32_t* err) {
@@ -897,8 +896,7 @@ __global__ __launch_bounds__(kThreads) void segment_emit_kernel(Segments sg, int
       sv.counts[i] = 0;
       sv.offsets[i] = total;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0)
-      counters[kCtrRuns] = nb > 0 ? segoff[nb - 1] + (uint32_t)(bcnt[nb - 1] >> 32) : 0u;
+    if (blockIdx.x == 0 && threadIdx.x == 0) counters[kCtrSorted] = (uint32_t)n;
   }
   const int64_t nwaves = (int64_t)gridDim.x * (kThreads / kWave);
   constexpr int kAhead = 4;
@@ -935,6 +933,28 @@ __global__ __launch_bounds__(kThreads) void segment_emit_kernel(Segments sg, int
         if (at[k] != ~0u && (int64_t)at[k] < n)
           list[at[k]] = (uint64_t)(uint32_t)(base + (w[k] & 0xffffu)) | ((uint64_t)(w[k] >> 16) << 32);
     }
+  }
+}
+
+// Runs of equal bucket in the last bucket sort (a diagnostic, formed when it is
+// asked for): the segments, less those that continue the previous tile's last.
+__global__ __launch_bounds__(1024) void count_runs_kernel(Segments sg, int64_t n, int32_t tile_size, uint32_t* runs) {
+  __shared__ uint32_t wsum[1024 / kWave];
+  const int64_t ntiles = (n + tile_size - 1) / tile_size;
+  uint32_t sum = 0;
+  for (int64_t tile = threadIdx.x; tile < ntiles; tile += blockDim.x) {
+    const int64_t base = tile * tile_size;
+    sum += sg.count[tile];
+    if (tile > 0 && sg.in[base].x == sg.in[base - tile_size + sg.count[tile - 1] - 1].x) --sum;
+  }
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o, kWave);
+  if (lane_id() == 0) wsum[threadIdx.x / kWave] = sum;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint32_t total = 0;
+    for (int w = 0; w < 1024 / kWave; ++w) total += wsum[w];
+    *runs = total;
   }
 }
 
@@ -1248,7 +1268,7 @@ hipError_t place_segments(const TableView& t, Workspace& ws, int64_t n, const in
   cap = cap < t.T ? cap : t.T;
   const int ge = groups_for(tiles * kWave, kThreads), gc = groups_for((int64_t)cap + 1, kThreads * 4);
   segment_emit_kernel<<<ge > gc ? ge : gc, kThreads, 0, s>>>(segments_of(ws, nullptr), n, tile_size(n), slot_block, ws.ts_cap,
-                                                             ws.segoff, ws.bcnt, nblocks, cap, out, ws.seg_list,
+                                                             ws.segoff, nblocks, cap, out, ws.seg_list,
                                                              ws.counters, ws.err);
   if (n <= 0) return hipGetLastError();
   const int g = cap < 32768 ? cap : 32768;
@@ -1258,6 +1278,11 @@ hipError_t place_segments(const TableView& t, Workspace& ws, int64_t n, const in
 }
 
 }  // namespace
+
+hipError_t count_runs(Workspace& ws, int64_t n, hipStream_t s) {
+  count_runs_kernel<<<1, 1024, 0, s>>>(segments_of(ws, nullptr), n, tile_size(n), ws.counters + kCtrRuns);
+  return hipGetLastError();
+}
 
 hipError_t bucket_sort(const TableView& t, Workspace& ws, const float* x, int64_t n, float dx, int blockLen,
                        int offset, float disp, const SortView& out, hipStream_t s) {
@@ -1343,7 +1368,7 @@ hipError_t build_activate(const TableView& t, Workspace& ws, const float* x, int
   if (n > 0) launch_activate<true>(ws, x, n, dx, 4, -2, 0.5f, segments_of(ws, ws.scnt), s, ss);
   const uint32_t nw = (ws.ts_cap + 31u) / 32u;
   build_collect_kernel<<<(int)((nw + kWave - 1) / kWave), kThreads, 0, s>>>(
-      ws.dmask, nw, ws.sorder, ranks_a(ws, n), ws.counters + kCtrList, ws.la_key, ws.la_val);
+      ws.dmask, nw, ws.sorder, ranks_a(ws, n), ws.counters + kCtrBlocks, ws.la_key, ws.la_val);
   return hipGetLastError();
 }
 
@@ -1352,13 +1377,13 @@ hipError_t build_enlarge(const TableView& t, Workspace& ws, int64_t n, const Sor
   uint32_t* mask2 = ws.dmask + (ws.ts_cap / 32 + 1);
   const Ranks ra = ranks_a(ws, n), rb = ranks_b(ws, t);
   build_number_kernel<true><<<number_groups(ra, ws.ts_cap, 1024), kThreads, 4 * padded(ra.groups), s>>>(
-      ws.counters + kCtrList, nullptr, ws.la_key, ws.la_val, ra, t, dedup_of(ws), mask2, ws.slot_block, ws.scnt,
+      ws.counters + kCtrBlocks, nullptr, ws.la_key, ws.la_val, ra, t, dedup_of(ws), mask2, ws.slot_block, ws.scnt,
       ws.bcnt, ws.nbr);
   const uint32_t nw = (ws.ts_cap + 31u) / 32u;
   build_collect_kernel<<<(int)((nw + kWave - 1) / kWave), kThreads, 0, s>>>(
-      mask2, nw, ws.sorder, rb, ws.counters + kCtrListB, ws.lb_key, ws.lb_val);
+      mask2, nw, ws.sorder, rb, ws.counters + kCtrList, ws.lb_key, ws.lb_val);
   build_number_kernel<false><<<number_groups(rb, ws.ts_cap, 256), kThreads, 4 * padded(rb.groups), s>>>(
-      ws.counters + kCtrListB, ws.counters + kCtrList, ws.lb_key, ws.lb_val, rb, t, dedup_of(ws), mask2,
+      ws.counters + kCtrList, ws.counters + kCtrBlocks, ws.lb_key, ws.lb_val, rb, t, dedup_of(ws), mask2,
       ws.slot_block, ws.scnt, ws.bcnt, ws.nbr);
   build_finish_kernel<<<few(ws.ts_cap, 2048), kThreads, 0, s>>>(t, ws.counters, ws.err, ws.slot_block, ws.ts_cap,
                                                                 ws.nbr, ws.bcnt, sv, ws.segoff,
@@ -1367,7 +1392,7 @@ hipError_t build_enlarge(const TableView& t, Workspace& ws, int64_t n, const Sor
 }
 
 hipError_t build_place(const TableView& t, Workspace& ws, int64_t n, const SortView& out, hipStream_t s) {
-  return place_segments(t, ws, n, ws.slot_block, reinterpret_cast<const int32_t*>(ws.counters + kCtrList), out, s);
+  return place_segments(t, ws, n, ws.slot_block, reinterpret_cast<const int32_t*>(ws.counters + kCtrBlocks), out, s);
 }
 
 }  // namespace zsmpm

@@ -129,14 +129,15 @@ __device__ __forceinline__ int32_t scene_of_particle(const int64_t* first, int32
 enum : int {
   kCtrList = 0,     // unique new keys found by a dedup pass
   kCtrCnt0 = 1,     // table size before the current insertion pass
-  kCtrRuns = 2,     // segments of equal bucket in the last bucket sort
+  kCtrRuns = 2,     // particle runs of equal bucket in the last bucket sort (filled by count_runs)
   kCtrFp64 = 3,     // particles that took the FP64 SVD path
   kCtrFallback = 4, // particles that took the SVD fallback of the learned closure
   kCtrMaxVel = 5,   // max |v|^2 as float bits
   kCtrFbQueue = 7,  // length of the closure's SVD fallback queue (per pass)
   kCtrNetQueue = 8, // waves the closure's network pass took (per pass)
   kCtrNetWaves = 9, // waves that evaluated the closure's network (all passes)
-  kCtrListB = 11,   // unique keys the substep's enlargement adds
+  kCtrBlocks = 11,  // unique keys of the substep's particles (kCtrList then counts those its enlargement adds)
+  kCtrSorted = 12,  // particles of the last bucket sort
   kCtrBhtRounds = 10, // placement rounds of the last bht insertion (host-side, filled by the counters call)
   kCtrCount = 16
 };
@@ -251,6 +252,8 @@ hipError_t table_enlarge(const TableView& t, Workspace& ws, const int32_t lo[3],
 hipError_t table_query(const TableView& t, const int32_t* keys, int64_t n, int32_t* out, hipStream_t s);
 hipError_t bucket_sort(const TableView& t, Workspace& ws, const float* x, int64_t n, float dx,
                        int blockLen, int offset, float disp, const SortView& out, hipStream_t s);
+// counters[kCtrRuns] of the last bucket sort, of n particles (counters[kCtrSorted])
+hipError_t count_runs(Workspace& ws, int64_t n, hipStream_t s);
 size_t rank_scratch_words();
 // The substep's build: clear, activation (blockLen 4, offset -2, displacement
 // 0.5), enlargement by {0,1}^3 and bucket sort in one chain. The table, the
