@@ -360,9 +360,10 @@ int32_t zsmpm_policy_transfer_scheme__rocm(zsmpm_policy pol, int32_t scheme);
  * whose launches have one shape): P2G's chunk (576 particles over four waves,
  * three workgroups per CU, or 256 over two waves, six per CU) and G2P's
  * threads per bucket (128 or 256). ZSMPM_SUBSTEPS_AUTOTUNE picks them with the
- * workgroup counts; set 0 for the default (576, 128, in more waves for small
- * scenes). Results do not depend
- * on them beyond float summation order. Other values: ZSMPM_INVALID_ARGUMENT. */
+ * workgroup counts. 0 is the default rule: 576 and 128, in more waves for small
+ * scenes; a value given holds at every size. The query reports 576 and 128 for
+ * the default rule too. Results do not depend on them beyond float summation
+ * order. Other values: ZSMPM_INVALID_ARGUMENT. */
 int32_t zsmpm_policy_launch_tiles__rocm(zsmpm_policy pol, int32_t* p2g_chunk, int32_t* g2p_threads);
 int32_t zsmpm_policy_set_launch_tiles__rocm(zsmpm_policy pol, int32_t p2g_chunk, int32_t g2p_threads);
 

@@ -6,6 +6,7 @@
 #include <cstdlib>
 #include <vector>
 #include "zsmpm.h"
+extern "C" int mock_p2g_chunk, mock_g2p_threads;
 template <typename D> D mk() { D d{}; d.hdr = {sizeof(D), ZSMPM_ABI_MAJOR, ZSMPM_ABI_MINOR}; return d; }
 struct Sc {
   zsmpm_model model; zsmpm_particles a, b; zsmpm_table t; zsmpm_buckets bk; zsmpm_grid g; zsmpm_plane_collider cols[6];
@@ -74,6 +75,16 @@ int main(int argc, char** argv) {
   expect("cell + fuse unsupported", zsmpm_substeps_sorted__rocm(pol, &s0.model, &s0.a, &s0.b, &s0.t, &s0.bk, &s0.g, 1e-4f, g3, s0.cols, 6, 2, ZSMPM_SUBSTEPS_FUSE_STRESS, &inb), ZSMPM_UNSUPPORTED_OPERATION);
   expect("apic transfer", zsmpm_policy_transfer_scheme__rocm(pol, ZSMPM_TRANSFER_APIC), 0);
   expect("default tiles", zsmpm_policy_set_launch_tiles__rocm(pol, 0, 0) == 0 && zsmpm_policy_launch_tiles__rocm(pol, &tc, &tt) == 0 && tc == 576 && tt == 128, 1);
+  // 0 leaves the tile to the particle count; a value given reaches the launch
+  for (int k = 0; k < 3; ++k) {
+    const int32_t chunk[3] = {0, 576, 256}, threads[3] = {0, 128, 256}, widths[3] = {768, 768, 1536};
+    expect("tiles for the launch", zsmpm_policy_set_launch_tiles__rocm(pol, chunk[k], threads[k]), 0);
+    expect("default widths", zsmpm_policy_set_launch_widths__rocm(pol, 0, 0), 0);
+    expect("width of the tile", zsmpm_policy_launch_widths__rocm(pol, &wp, &wg) == 0 && wp == widths[k], 1);
+    expect("substep with the tiles", zsmpm_substeps_sorted__rocm(pol, &s0.model, &s0.a, &s0.b, &s0.t, &s0.bk, &s0.g, 1e-4f, g3, s0.cols, 6, 1, 0, &inb), 0);
+    expect("tiles reach the launch", mock_p2g_chunk == chunk[k] && mock_g2p_threads == threads[k], 1);
+  }
+  expect("tiles by the particle count", zsmpm_policy_set_launch_tiles__rocm(pol, 0, 0), 0);
   expect("set widths", zsmpm_policy_set_launch_widths__rocm(pol, 300, 5000), 0);
   expect("widths read back", zsmpm_policy_launch_widths__rocm(pol, &wp, &wg) == 0 && wp == 300 && wg == 5000, 1);
   expect("negative width rejected", zsmpm_policy_set_launch_widths__rocm(pol, -1, 5000), ZSMPM_INVALID_ARGUMENT);

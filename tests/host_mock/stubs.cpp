@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include "zsmpm_internal.hpp"
 extern "C" hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t, hipStream_t s);
+// the launch tiles the last substep asked its transfers for
+extern "C" { int mock_p2g_chunk = -1, mock_g2p_threads = -1; }
 namespace zsmpm {
 static hipError_t touch(hipStream_t s) { return hipLaunchKernel(nullptr, dim3(1), dim3(1), nullptr, 0, s); }
 // a batch's scene table reaches the kernels whole: device arrays set, the
@@ -38,9 +40,9 @@ hipError_t mlp_grad(const float*, const float*, const float*, int64_t, float*, f
 hipError_t mlp_reduce(float*, float*, float*, const float*, const float*, int, float, float, float, float*, float*, hipStream_t s) { return touch(s); }
 hipError_t mlp_harvest(const Model&, const float*, const float*, int64_t, float*, float*, hipStream_t s) { return touch(s); }
 hipError_t closure_launch_limits() { return hipSuccess; }
-hipError_t p2g_scatter(const ParticlesView&, const TableView&, const SortView&, float*, int32_t, float, float, bool, Workspace&, hipStream_t s, const SceneSet* ss, const StressFrom&) { return scenes_ok(ss, s); }
+hipError_t p2g_scatter(const ParticlesView&, const TableView&, const SortView&, float*, int32_t, float, float, bool, Workspace& w, hipStream_t s, const SceneSet* ss, const StressFrom&) { mock_p2g_chunk = w.p2g_chunk; return scenes_ok(ss, s); }
 hipError_t grid_update(float*, int32_t, const TableView&, float, const float*, const Colliders&, float, int, Workspace&, hipStream_t s, const SceneSet* ss, const GeneralColliders* gen) { return gen && gen->n > kMaxColliders ? hipErrorInvalidValue : scenes_ok(ss, s); }
-hipError_t g2p(const ParticlesView&, const ParticlesView*, const TableView&, const SortView&, const float*, int32_t, float, float, Workspace&, hipStream_t s, const NextStress*, const SceneSet* ss) { return scenes_ok(ss, s); }
+hipError_t g2p(const ParticlesView&, const ParticlesView*, const TableView&, const SortView&, const float*, int32_t, float, float, Workspace& w, hipStream_t s, const NextStress*, const SceneSet* ss) { mock_g2p_threads = w.g2p_threads; return scenes_ok(ss, s); }
 hipError_t grid_angular_momentum(const float*, int32_t, const TableView&, float, int, int, double*, Workspace&, hipStream_t s) { return touch(s); }
 hipError_t p2c2g_scatter(const ParticlesView&, const TableView&, const SortView&, float*, int32_t, float, float, Workspace&, hipStream_t s, const StressFrom&) { return touch(s); }
 hipError_t p2g_force_scatter(const ParticlesView&, const TableView&, const SortView&, float*, int32_t, float, float, Workspace&, hipStream_t s, const StressFrom&) { return touch(s); }

@@ -56,7 +56,7 @@ struct zsmpm_policy_s {
   int32_t bht_rounds = 0;
   // P2G / G2P workgroup counts picked by ZSMPM_SUBSTEPS_AUTOTUNE (0: default)
   int32_t tuned_p2g = 0, tuned_g2p = 0;
-  int32_t tuned_p2g_tile = 0, tuned_g2p_threads = 0;  // launch tiles (0: defaults)
+  int32_t tuned_p2g_chunk = 0, tuned_g2p_threads = 0;  // launch tiles (0: by the particle count)
   int32_t transfer = 0;  // the substep drivers' transfers: ZSMPM_TRANSFER_APIC or ZSMPM_TRANSFER_CELL
   Workspace ws{};
   std::vector<void*> allocs;
@@ -554,7 +554,7 @@ int32_t run_substep(zsmpm_policy_s* pol, const zsmpm_model* model, const zsmpm_p
   Workspace& ws = pol->ws;
   ws.grid_p2g = pol->tuned_p2g;
   ws.grid_g2p = pol->tuned_g2p;
-  ws.p2g_tile = pol->tuned_p2g_tile;
+  ws.p2g_chunk = pol->tuned_p2g_chunk;
   ws.g2p_threads = pol->tuned_g2p_threads;
   // the transfer scheme holds for this substep's launches only (the
   // stage-wise entry points keep their own transfers)
@@ -667,7 +667,7 @@ int32_t capture_pair(zsmpm_policy_s* pol, const zsmpm_model* model, const zsmpm_
   key_put(key, &pol->closure);
   key_put(key, &pol->tuned_p2g);
   key_put(key, &pol->tuned_g2p);
-  key_put(key, &pol->tuned_p2g_tile);
+  key_put(key, &pol->tuned_p2g_chunk);
   key_put(key, &pol->tuned_g2p_threads);
   key_put(key, &pol->transfer);
   key_put(key, &pol->gcols);
@@ -826,14 +826,16 @@ int32_t substeps_driver(zsmpm_policy_s* pol, const zsmpm_model* model, const zsm
   // Autotuning: the first 8 substeps (real ones, in pairs a -> b -> a) run
   // with four P2G and four G2P launch configurations (tile and workgroup
   // count), timed per kernel with the stage events; each kernel keeps its
-  // fastest. P2G: four waves with 576-particle chunks at 1,024 and 768 (resident)
-  // workgroups, two waves with 256-particle chunks at 2,048 and 4,096; G2P:
-  // 128 and 256 threads per bucket at 32,768 and 65,536 workgroups.
+  // fastest. P2G: the default rule's tile (four waves with 576-particle chunks,
+  // nine waves for small scenes) at 1,024 and 768 (resident) workgroups, two
+  // waves with 256-particle chunks at 2,048 and 4,096; G2P: the default rule's
+  // threads per bucket (128, 512 for small scenes) and 256, each at 32,768 and
+  // 65,536 workgroups.
   int32_t done = 0;
   if ((flags & ZSMPM_SUBSTEPS_AUTOTUNE) && nsteps >= 8 && !fuse) {
     DeviceGuard g(pol->devid);
     const int32_t cand_p2g[4] = {1024, 768, 2048, 4096}, cand_g2p[4] = {32768, 65536, 32768, 65536};
-    const int32_t cand_p2g_tile[4] = {0, 0, 1, 1}, cand_g2p_threads[4] = {0, 0, 256, 256};
+    const int32_t cand_p2g_chunk[4] = {0, 0, 256, 256}, cand_g2p_threads[4] = {0, 0, 256, 256};
     const bool prof = pol->profile;
     ZS_HIP(hipStreamSynchronize(pol->stream));
     harvest_events(pol);
@@ -844,7 +846,7 @@ int32_t substeps_driver(zsmpm_policy_s* pol, const zsmpm_model* model, const zsm
     for (int c = 0; c < 4 && r == ZSMPM_OK; ++c) {
       pol->tuned_p2g = cand_p2g[c];
       pol->tuned_g2p = cand_g2p[c];
-      pol->tuned_p2g_tile = cand_p2g_tile[c];
+      pol->tuned_p2g_chunk = cand_p2g_chunk[c];
       pol->tuned_g2p_threads = cand_g2p_threads[c];
       const double p0 = pol->stage_ms[ZSMPM_STAGE_P2G], g0 = pol->stage_ms[ZSMPM_STAGE_G2P];
       for (int k = 0; k < 2 && r == ZSMPM_OK; ++k, ++done)
@@ -856,7 +858,7 @@ int32_t substeps_driver(zsmpm_policy_s* pol, const zsmpm_model* model, const zsm
       if (c == 0 || dp < best_p) {
         best_p = dp;
         pick_p = cand_p2g[c];
-        pick_pt = cand_p2g_tile[c];
+        pick_pt = cand_p2g_chunk[c];
       }
       if (c == 0 || dg < best_g) {
         best_g = dg;
@@ -868,7 +870,7 @@ int32_t substeps_driver(zsmpm_policy_s* pol, const zsmpm_model* model, const zsm
     if (r != ZSMPM_OK) return r;
     pol->tuned_p2g = pick_p;
     pol->tuned_g2p = pick_g;
-    pol->tuned_p2g_tile = pick_pt;
+    pol->tuned_p2g_chunk = pick_pt;
     pol->tuned_g2p_threads = pick_gt;
   }
   nsteps -= done;  // an even count: the particles are back in a
@@ -1830,7 +1832,7 @@ constexpr int32_t kMaxLaunchGroups = 1 << 20;
 
 int32_t zsmpm_policy_launch_widths__rocm(zsmpm_policy pol, int32_t* p2g_groups, int32_t* g2p_groups) {
   if (!pol || !p2g_groups || !g2p_groups) return ZSMPM_INVALID_ARGUMENT;
-  *p2g_groups = pol->tuned_p2g > 0 ? pol->tuned_p2g : default_p2g_groups();
+  *p2g_groups = pol->tuned_p2g > 0 ? pol->tuned_p2g : default_p2g_groups(pol->tuned_p2g_chunk);
   *g2p_groups = pol->tuned_g2p > 0 ? pol->tuned_g2p : default_g2p_groups();
   return ZSMPM_OK;
 }
@@ -1851,7 +1853,7 @@ int32_t zsmpm_policy_transfer_scheme__rocm(zsmpm_policy pol, int32_t scheme) {
 
 int32_t zsmpm_policy_launch_tiles__rocm(zsmpm_policy pol, int32_t* p2g_chunk, int32_t* g2p_threads) {
   if (!pol || !p2g_chunk || !g2p_threads) return ZSMPM_INVALID_ARGUMENT;
-  *p2g_chunk = pol->tuned_p2g_tile == 1 ? 256 : 576;
+  *p2g_chunk = pol->tuned_p2g_chunk == 256 ? 256 : 576;
   *g2p_threads = pol->tuned_g2p_threads == 256 ? 256 : 128;
   return ZSMPM_OK;
 }
@@ -1860,7 +1862,7 @@ int32_t zsmpm_policy_set_launch_tiles__rocm(zsmpm_policy pol, int32_t p2g_chunk,
   if (!pol || (p2g_chunk != 0 && p2g_chunk != 576 && p2g_chunk != 256) ||
       (g2p_threads != 0 && g2p_threads != 128 && g2p_threads != 256))
     return ZSMPM_INVALID_ARGUMENT;
-  pol->tuned_p2g_tile = p2g_chunk == 256 ? 1 : 0;
+  pol->tuned_p2g_chunk = p2g_chunk;
   pol->tuned_g2p_threads = g2p_threads;
   return ZSMPM_OK;
 }

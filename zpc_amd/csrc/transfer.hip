@@ -1532,15 +1532,14 @@ hipError_t stress(const Model& m, const ParticlesView& ps, Workspace& ws, hipStr
 namespace {
 
 // Workgroups of the per-bucket kernels: the policy's counts, else P2G as many
-// as are resident (three of four waves per CU, or six of two) -- more only
-// queue behind each other -- and G2P one per bucket up to 32,768; no more than
-// there can be buckets.
+// as are resident and G2P one per bucket up to 32,768; no more than there can
+// be buckets.
 int bucket_bound(const SortView& sv, int32_t grid_cap) {
   const int32_t cap = grid_cap < sv.cap_blocks ? grid_cap : sv.cap_blocks;
   return cap > 1 ? cap : 1;
 }
 int p2g_groups(const Workspace& ws, const SortView& sv, int32_t grid_cap) {
-  const int g = ws.grid_p2g > 0 ? ws.grid_p2g : (ws.p2g_tile == 1 ? 2 : 1) * default_p2g_groups();
+  const int g = ws.grid_p2g > 0 ? ws.grid_p2g : default_p2g_groups(ws.p2g_chunk);
   const int cap = bucket_bound(sv, grid_cap);
   return g < cap ? g : cap;
 }
@@ -1558,7 +1557,7 @@ hipError_t p2g_scatter(const ParticlesView& ps, const TableView& t, const SortVi
   const int g = p2g_groups(ws, sv, grid_cap);
   const bool multi = ss && ss->n > 0;
   const SceneSet sset = multi ? *ss : SceneSet{};
-  const bool tile1 = ws.p2g_tile == 1;  // the folded launches take the tuned tile
+  const bool tile1 = ws.p2g_chunk == 256;  // the folded launches take the tuned tile
   if (fold && ws.cell && !multi)  // the substep's P2C2G (one tile)
     p2g_kernel<0, false, true><<<g, kP2GThreads, 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt, dx,
                                                          ws.err, sset, 1);
@@ -1570,7 +1569,7 @@ hipError_t p2g_scatter(const ParticlesView& ps, const TableView& t, const SortVi
   else if (fold && tile1)
     p2g_kernel<0, false, false, 1><<<g, p2g_threads(1), 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt,
                                                                 dx, ws.err, sset, 1);
-  else if (fold && ps.n <= kP2GWideParticles)
+  else if (fold && ws.p2g_chunk == 0 && ps.n <= kP2GWideParticles)
     p2g_kernel<0, false, false, kWideTile><<<g, p2g_threads(kWideTile), 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid,
                                                                                grid_cap, dt, dx, ws.err, sset, 1);
   else if (fold)

@@ -188,7 +188,7 @@ struct Workspace {
   uint32_t* wq = nullptr;        // [n_cap / 64 + 2] per wave: 1 where the closure's network must run
   int32_t grid_p2g = 0;          // P2G / G2P workgroups (0: the defaults below), set by the policy
   int32_t grid_g2p = 0;
-  int32_t p2g_tile = 0;     // folded P2G launch tile: 0 four waves / 576-particle chunks, 1 two waves / 256
+  int32_t p2g_chunk = 0;    // folded P2G launch tile: 576 (four waves) or 256 (two waves); 0: by the particle count
   int32_t g2p_threads = 0;  // sorted G2P threads per bucket: 256 or 128; 0: by the particle count
   bool cell = false;        // the substep's transfers are P2C2G / G2C2P (set by the substep driver only)
   float* lj_next[2] = {nullptr, nullptr};  // [n_cap] each: logJp caches of the fused multi-substep driver
@@ -330,8 +330,10 @@ hipError_t reorder_particles(const ParticlesView& in, const ParticlesView& out, 
 
 // grid-stride launch width for kernels that loop over a device-resident count
 inline int persistent_groups() { return 4096; }
-// P2G / G2P workgroups where the policy sets none
-inline int default_p2g_groups() { return 768; }
+// P2G / G2P workgroups where the policy sets none: P2G as many as are resident,
+// three of four waves per CU or six of two (chunks of 256) -- more only queue
+// behind each other
+inline int default_p2g_groups(int32_t chunk) { return chunk == 256 ? 1536 : 768; }
 inline int default_g2p_groups() { return 32768; }
 
 // ---- implicit step (implicit.hip; the projection in transfer.hip) ----
