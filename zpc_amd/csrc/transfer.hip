@@ -58,25 +58,31 @@ __device__ __forceinline__ int vel_at(int r0, int r1, int r2) { return r0 * kVel
 constexpr int kG2PThreads = 128;
 // G2P of a small scene: as many waves as a full bucket has rounds of rows. With
 // two, a bucket's rounds ran one after another while most CUs idled: substep
-// 84 -> 74 us at 64K particles, 95 -> 91 at 256K, equal at 512K (1,000 buckets
-// of two waves fill the card).
+// 77.2 -> 68.8 us at 64K particles of 8 per cell, 91.0 -> 87.0 at 262K (729
+// buckets). Sparse buckets leave the extra waves idle and many buckets fill the
+// card with two: 115 -> 124 at 250K of 2 per cell (2,200 buckets), 81.5 -> 89.8
+// at 64K of 1 (1,331). The line is on the buckets' capacity (wide_buckets); below
+// it bodies of 1 particle per cell lose most, 69.8 -> 72.9 at 27K, and dense ones
+// gain most, 241 -> 176 at 512K of 64.
 constexpr int kG2PWide = 512;
-constexpr int64_t kG2PWideParticles = 262144;
+constexpr int kG2PWideBuckets = 2048;
 constexpr int kP2GThreads = 256;  // one workgroup per bucket
 constexpr int kP2GWaves = kP2GThreads / kWave;
 // Launch tiles the autotuner chooses between. P2G tile 0: four waves and
 // chunks of Rec::kChunk particles (a whole bucket of up to 576, three
 // workgroups per CU); tile 1: two waves and chunks of 256 (six workgroups per
 // CU, for sparser buckets). G2P: 128 or 256 threads per bucket.
-// kWideTile, P2G of a small scene: a wave per round of a full bucket's rows
-// (records and scatter in one round each, no serial chain of three). One such
-// workgroup fits a CU, so it pays while a CU has no second bucket: up to 256
-// buckets of some 300 particles, counting the partly filled ones at a body's
-// surface. Substep 70.3 -> 65.4 us at 4K particles, 74.1 -> 70.8 at 64K; past
-// the line 76.7 -> 80.9 at 96K (343 buckets). Splitting a bucket over four
-// workgroups instead gained 3 us at 4K and lost 15 at 64K.
-constexpr int64_t kP2GWideParticles = 256 * 300;
-constexpr int kWideTile = 2, kWideP2GThreads = 576;
+//
+// kWideTile, P2G of a small scene: eight waves per bucket (records and scatter
+// in about one round each, no serial chain of three). At 128 registers two such
+// workgroups fit a CU, so it pays while every bucket is resident at once, up to
+// 512: substep 67.1 -> 64.7 us at 4K particles, 70.9 -> 68.9 at 64K, 88.3 -> 82.3
+// at 128K of 16 per cell, 224 -> 170 at 262K of 64; past the line 89.4 -> 101 at
+// 64K of 1 per cell (1,331 buckets). Nine waves at 144 registers, one workgroup
+// per CU, cost more from 256 buckets on (72.5 -> 76.2 at 72K). Splitting a bucket
+// over four workgroups instead gained 3 us at 4K and lost 15 at 64K.
+constexpr int kP2GWideBuckets = 1024;
+constexpr int kWideTile = 2, kWideP2GThreads = 512;
 constexpr int p2g_threads(int tile) { return tile == kWideTile ? kWideP2GThreads : tile == 1 ? 128 : kP2GThreads; }
 constexpr int p2g_chunk(int tile, int fold_chunk) { return tile == 1 ? 256 : fold_chunk; }
 
@@ -289,7 +295,7 @@ __global__ __launch_bounds__(kThreads) void stress_kernel(Model m, ParticlesView
 // (cell_w) in place of the quadratic B-spline, with C and the stress scaled
 // per column by the cell kernel's Dinv.
 template <int kMode, bool kMulti, bool kCell = false, int kTile = 0>
-__global__ __launch_bounds__(p2g_threads(kTile), 3) void p2g_kernel(ParticlesView ps, const float* __restrict__ contrib,
+__global__ __launch_bounds__(p2g_threads(kTile), kTile == kWideTile ? 4 : 3) void p2g_kernel(ParticlesView ps, const float* __restrict__ contrib,
                                                        StressFrom st,
                                                        TableView t, SortView sv, const int32_t* __restrict__ nbr_tab,
                                                        float* __restrict__ grid, int32_t grid_cap, float dt,
@@ -1538,6 +1544,10 @@ int bucket_bound(const SortView& sv, int32_t grid_cap) {
   const int32_t cap = grid_cap < sv.cap_blocks ? grid_cap : sv.cap_blocks;
   return cap > 1 ? cap : 1;
 }
+// The caller's capacity for blocks is at most `line`. The launch cannot know how
+// many buckets there will be, but grids are sized for a table of at least twice
+// the blocks with their enlargement, so at most half the capacity is in use.
+bool wide_buckets(const SortView& sv, int32_t grid_cap, int line) { return bucket_bound(sv, grid_cap) <= line; }
 int p2g_groups(const Workspace& ws, const SortView& sv, int32_t grid_cap) {
   const int g = ws.grid_p2g > 0 ? ws.grid_p2g : default_p2g_groups(ws.p2g_chunk);
   const int cap = bucket_bound(sv, grid_cap);
@@ -1569,7 +1579,7 @@ hipError_t p2g_scatter(const ParticlesView& ps, const TableView& t, const SortVi
   else if (fold && tile1)
     p2g_kernel<0, false, false, 1><<<g, p2g_threads(1), 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid, grid_cap, dt,
                                                                 dx, ws.err, sset, 1);
-  else if (fold && ws.p2g_chunk == 0 && ps.n <= kP2GWideParticles)
+  else if (fold && ws.p2g_chunk == 0 && wide_buckets(sv, grid_cap, kP2GWideBuckets))
     p2g_kernel<0, false, false, kWideTile><<<g, p2g_threads(kWideTile), 0, s>>>(ps, ws.contrib, st, t, sv, ws.nbr, grid,
                                                                                grid_cap, dt, dx, ws.err, sset, 1);
   else if (fold)
@@ -1677,7 +1687,7 @@ hipError_t g2p(const ParticlesView& ps, const ParticlesView* out, const TableVie
   } else if (out && ws.g2p_threads == 256) {
     g2p_kernel<true, -1, false, false, 256><<<g, 256, 0, s>>>(ps, *out, t, sv, ws.nbr, grid, grid_cap, dt, dx, ns,
                                                               ws.err, ws.counters, sset);
-  } else if (sset.n == 0 && ws.g2p_threads == 0 && ps.n <= kG2PWideParticles) {
+  } else if (sset.n == 0 && ws.g2p_threads == 0 && wide_buckets(sv, grid_cap, kG2PWideBuckets)) {
     if (out)
       g2p_kernel<true, -1, false, false, kG2PWide><<<g, kG2PWide, 0, s>>>(ps, *out, t, sv, ws.nbr, grid, grid_cap, dt,
                                                                           dx, ns, ws.err, ws.counters, sset);
