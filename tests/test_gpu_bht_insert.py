@@ -1,5 +1,6 @@
-"""Insertion at the edges of its steps: words of 64 keys, tiles of 1,024, runs
-of equal keys across both, and more distinct keys than twice the table's slots
+"""Insertion at the edges of its steps: words of 64 keys, tiles of 1,024, the
+line of 2^20 keys, runs of equal keys across them, mostly distinct keys, and more
+distinct keys than twice the table's slots
 (the deduplication starts again with a larger hash); sampling on positions that
 share blocks and on positions that do not. Whole numbers: exact against the
 sequential insertion; samples are the same operations in the same order, equal
@@ -14,7 +15,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("run", [1, 7, 64])
 @pytest.mark.parametrize("T,n", [(4096, 1), (4096, 63), (4096, 64), (4096, 65), (4096, 1023), (4096, 1025),
-                                 (4096, 4097), (64, 1500), (64, 40000)])
+                                 (4096, 4097), (64, 1500), (64, 40000), (32768, (1 << 20) - 1),
+                                 (32768, 1 << 20), (32768, (1 << 20) + 65)])
 def test_insert_edges(T, n, run):
     import torch
     from zpc_amd import rocm
@@ -45,6 +47,26 @@ def test_insert_edges(T, n, run):
     assert np.array_equal(got[~first], np.full(int((~first).sum()), -1))
     assert np.all((got[first] == rank[first]) | (got[first] == O.BHT_FAILURE))
     assert np.all(got[first & (rank >= T - 20)] == O.BHT_FAILURE)
+
+
+@pytest.mark.parametrize("n", [1000, 32768, (1 << 20) + 77])
+def test_insert_distinct_into_a_used_table(n):
+    """Nearly all keys are first occurrences, and half of them are in the table."""
+    import torch
+    from zpc_amd import rocm
+
+    rng = np.random.default_rng(n)
+    keys = rng.integers(-4000, 4000, size=(n, 3)).astype(np.int32)
+    h = O.HostBht(1 << 22)
+    t = rocm.DeviceBht(1 << 22)
+    for part in (keys[::2], keys):
+        part = np.ascontiguousarray(part)
+        ref = h.insert(part)
+        got = t.insert(torch.as_tensor(part).cuda()).cpu().numpy()
+        assert int(h.success[0])
+        assert np.array_equal(got, ref)
+    t.pol.sync()
+    assert np.array_equal(t.keys.cpu().numpy().reshape(-1), h.keys)
 
 
 def test_insert_far_over_the_table_on_used_scratch():

@@ -30,6 +30,8 @@ constexpr uint64_t kEmpty64 = ~0ull;
 constexpr uint32_t kNone = 0xffffffffu;    // an input key out of range
 constexpr uint32_t kRepeat = 0xfffffffeu;  // an input equal to the one before it
 constexpr int kMaxRounds = 64;
+// From here on a key per thread fills the card (524,288 threads) with threads to spare.
+constexpr int64_t kManyKeys = 1 << 20;
 
 int groups_n(int64_t n, int per = kBT) {
   const int64_t g = (n + per - 1) / per;
@@ -114,26 +116,25 @@ __global__ __launch_bounds__(kBT) void dedup_clear_kernel(uint64_t* skey, uint32
 // A key that finds no slot in kProbes steps raises *full; the tiles not yet
 // begun are then skipped (their head and slot_of stay as they were, and nothing
 // reads them) and the caller starts again with the hash sized for n distinct
-// keys. What bounds it is the latency
-// of the probe, so a thread takes four keys in a row (a run that a wave
-// boundary cuts goes to the hash once per 256 keys) and an index that cannot
-// lower a slot's minimum (a few blocks collect all runs) does no atomic. With
-// the keys formed here instead of in a pass of their own, 112 -> 62 us at 4.2M
-// positions in 1,500 blocks.
-constexpr int kDedupItems = 4;
+// keys. What bounds it is the latency of the probe, so a thread takes kItems
+// keys in a row (four: a run that a wave boundary cuts goes to the hash once per
+// 256 keys; one below kManyKeys, where four probes in a row are the longer
+// chain, 23 us against 10 at 1,000 keys) and an index that cannot lower a slot's
+// minimum (a few blocks collect all runs) does no atomic. With the keys formed here instead of in a pass of their own, 112 ->
+// 62 us at 4.2M positions in 1,500 blocks.
 constexpr int kProbes = 256;
-template <bool kAll, typename Keys>
-__global__ __launch_bounds__(kBT) void dedup_insert_kernel(Keys keys, int64_t n, uint64_t* skey, uint32_t* smin,
-                                                           int64_t S, bool bounded, uint32_t* slot_of,
-                                                           uint8_t* __restrict__ head, uint32_t* full,
-                                                           uint32_t* err) {
-  constexpr int kTile = kBT * kDedupItems;
+template <bool kAll, int kItems, typename Keys>
+__global__ __launch_bounds__(kBT) void dedup_insert_kernel(Keys keys, int64_t n, int64_t words, uint64_t* skey,
+                                                           uint32_t* smin, int64_t S, bool bounded,
+                                                           uint32_t* slot_of, uint64_t* __restrict__ head,
+                                                           uint32_t* full, uint32_t* err) {
+  constexpr int kTile = kBT * kItems;
   for (int64_t base = blockIdx.x * (int64_t)kTile; base < n; base += (int64_t)gridDim.x * kTile) {
     if (bounded && uniform((int32_t)__hip_atomic_load(full, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) return;
-    const int64_t i0 = base + (int64_t)threadIdx.x * kDedupItems;
-    uint64_t p[kDedupItems];
+    const int64_t i0 = base + (int64_t)threadIdx.x * kItems;
+    uint64_t p[kItems];
 #pragma unroll
-    for (int r = 0; r < kDedupItems; ++r) {
+    for (int r = 0; r < kItems; ++r) {
       const bool live = i0 + r < n;
       int32_t k0 = 0, k1 = 0, k2 = 0;
       if (live) keys.get(i0 + r, k0, k1, k2);
@@ -144,25 +145,30 @@ __global__ __launch_bounds__(kBT) void dedup_insert_kernel(Keys keys, int64_t n,
         if (kAll) slot_of[i0 + r] = kNone;
       }
     }
-    uint64_t left = __shfl_up(p[kDedupItems - 1], 1, kWave);
+    uint64_t left = __shfl_up(p[kItems - 1], 1, kWave);
     if (lane_id() == 0) left = kEmpty64;
     uint32_t probe = 0;
 #pragma unroll
-    for (int r = 0; r < kDedupItems; ++r) {
+    for (int r = 0; r < kItems; ++r) {
       const bool valid = p[r] != kEmpty64, repeat = left == p[r];
       if (kAll && valid && repeat) slot_of[i0 + r] = kRepeat;
       probe |= valid && !repeat ? 1u << r : 0u;
       left = p[r];
     }
-    static_assert(kDedupItems == 4, "two lanes write one byte");
-    const uint32_t byte = probe | (uint32_t)__shfl_down((int)probe, 1, kWave) << 4;
-    if ((threadIdx.x & 1) == 0 && i0 < n) head[i0 / 8] = (uint8_t)byte;
+    static_assert(kItems == 1 || kItems == 4, "a wave writes one word of head, or two lanes a byte");
+    if constexpr (kItems == 1) {
+      const uint64_t word = ballot(probe != 0u);
+      if (lane_id() == 0 && i0 < n) head[i0 / kWave] = word;
+    } else {
+      const uint32_t byte = probe | (uint32_t)__shfl_down((int)probe, 1, kWave) << 4;
+      if ((threadIdx.x & 1) == 0 && i0 < words * kWave) reinterpret_cast<uint8_t*>(head)[i0 / 8] = (uint8_t)byte;
+    }
     while (probe) {
       const int r = __ffs(probe) - 1;
       probe &= probe - 1u;
       uint64_t key = p[0];
 #pragma unroll
-      for (int q = 1; q < kDedupItems; ++q) key = r == q ? p[q] : key;
+      for (int q = 1; q < kItems; ++q) key = r == q ? p[q] : key;
       const int64_t i = i0 + r;
       uint64_t h = mix64(key) & (uint64_t)(S - 1);
       uint32_t slot = kNone;
@@ -189,50 +195,74 @@ __global__ __launch_bounds__(kBT) void dedup_insert_kernel(Keys keys, int64_t n,
   }
 }
 
-// a bit per key: the first occurrence of a key the table does not hold yet; none
+// A bit per key: the first occurrence of a key the table does not hold yet; none
 // after a hash that was too small (*full), whose skipped tiles left head and
-// slot_of unwritten. A thread per byte of head: few bits are set where
-// neighbours share a block, and eight in a row are the most it follows.
-template <typename Keys>
-__global__ __launch_bounds__(kBT) void first_kernel(Keys keys, int64_t n, int64_t bytes,
-                                                    const uint8_t* __restrict__ head, const uint32_t* slot_of,
-                                                    const uint32_t* smin, const uint32_t* full, BhtView t,
-                                                    uint8_t* __restrict__ flag) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+// slot_of unwritten. A wave takes kWords words of 64 keys, a lane a key of each,
+// with the words' loads in flight together: few heads are first occurrences where
+// neighbours share a block, and where every key is one the queries of a word run
+// side by side (a thread that followed a byte of heads made eight in a row, 34
+// us instead of 13 for 32K distinct keys).
+template <int kWords, typename Keys>
+__global__ __launch_bounds__(kBT) void first_kernel(Keys keys, int64_t words, const uint64_t* __restrict__ head,
+                                                    const uint32_t* slot_of, const uint32_t* smin,
+                                                    const uint32_t* full, BhtView t, uint64_t* __restrict__ flag) {
+  const int lane = lane_id();
   const bool complete = *full == 0u;
-  for (int64_t w = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; w < bytes; w += stride) {
-    uint32_t out = 0;
-    for (uint32_t bits = complete && 8 * w < n ? head[w] : 0u; bits; bits &= bits - 1u) {
-      const int b = __ffs(bits) - 1;
-      const int64_t i = 8 * w + b;
-      const uint32_t s = slot_of[i];
-      if (s >= kRepeat || smin[s] != (uint32_t)i) continue;
-      int32_t k0, k1, k2;
-      keys.get(i, k0, k1, k2);
-      if (bht_query(t, k0, k1, k2) < 0) out |= 1u << b;
+  const int64_t nwaves = (int64_t)gridDim.x * (kBT / kWave);
+  for (int64_t w0 = (blockIdx.x * (int64_t)(kBT / kWave) + uniform((int32_t)(threadIdx.x / kWave))) * kWords; w0 < words;
+       w0 += nwaves * kWords) {
+    const int64_t i0 = w0 * kWave + lane;
+    uint32_t s[kWords];
+    uint64_t cand[kWords];
+#pragma unroll
+    for (int r = 0; r < kWords; ++r) {
+      const uint64_t bits = complete && w0 + r < words ? head[w0 + r] : 0ull;  // no bit past the last key
+      s[r] = (bits >> lane) & 1ull ? slot_of[i0 + r * kWave] : kNone;
     }
-    flag[w] = (uint8_t)out;
+#pragma unroll
+    for (int r = 0; r < kWords; ++r)
+      cand[r] = ballot(s[r] < kRepeat && smin[s[r] < kRepeat ? s[r] : 0u] == (uint32_t)(i0 + r * kWave));
+    for (int r = 0; r < kWords && w0 + r < words; ++r) {
+      uint64_t bits = cand[0];
+#pragma unroll
+      for (int q = 1; q < kWords; ++q) bits = r == q ? cand[q] : bits;
+      bool is_new = false;
+      if ((bits >> lane) & 1ull) {
+        int32_t k0, k1, k2;
+        keys.get(i0 + (int64_t)r * kWave, k0, k1, k2);
+        is_new = bht_query(t, k0, k1, k2) < 0;
+      }
+      bits = ballot(is_new);
+      if (lane == 0) flag[w0 + r] = bits;
+    }
   }
 }
 
-// the new keys in order of first occurrence: rank[w] of them before word w
-template <typename Keys>
-__global__ __launch_bounds__(kBT) void compact_kernel(Keys keys, int64_t words, const uint32_t* __restrict__ flag,
+// the new keys in order of first occurrence: rank[w] of them before 32-bit word
+// w. A wave takes kWords words of 64 keys, a lane a key of each.
+template <int kWords, typename Keys>
+__global__ __launch_bounds__(kBT) void compact_kernel(Keys keys, int64_t words, const uint64_t* __restrict__ flag,
                                                       const uint32_t* __restrict__ rank, int32_t* nk,
                                                       uint32_t* level) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t w = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; w < words; w += stride) {
-    uint32_t bits = flag[w];
-    if (!bits) continue;
-    int64_t r = rank[w];
-    for (; bits; bits &= bits - 1u, ++r) {
-      const int64_t i = 32 * w + __ffs(bits) - 1;
+  const int lane = lane_id();
+  const int64_t nwaves = (int64_t)gridDim.x * (kBT / kWave);
+  for (int64_t w0 = (blockIdx.x * (int64_t)(kBT / kWave) + uniform((int32_t)(threadIdx.x / kWave))) * kWords; w0 < words;
+       w0 += nwaves * kWords) {
+    uint64_t bits[kWords];
+#pragma unroll
+    for (int r = 0; r < kWords; ++r) bits[r] = w0 + r < words ? flag[w0 + r] : 0ull;
+#pragma unroll
+    for (int r = 0; r < kWords; ++r) {
+      if (!((bits[r] >> lane) & 1ull)) continue;
+      const uint32_t half = lane < 32 ? (uint32_t)bits[r] : (uint32_t)(bits[r] >> 32);
+      const int64_t at =
+          (int64_t)rank[2 * (w0 + r) + lane / 32] + __popc(half & ((1u << (lane & 31)) - 1u));
       int32_t k0, k1, k2;
-      keys.get(i, k0, k1, k2);
-      nk[3 * r] = k0;
-      nk[3 * r + 1] = k1;
-      nk[3 * r + 2] = k2;
-      level[r] = 0;
+      keys.get((w0 + r) * kWave + lane, k0, k1, k2);
+      nk[3 * at] = k0;
+      nk[3 * at + 1] = k1;
+      nk[3 * at + 2] = k2;
+      level[at] = 0;
     }
   }
 }
@@ -472,7 +502,7 @@ struct Carve {
   uint32_t *smin, *slot_of, *flag, *rank, *total, *c0, *changed, *level, *bkey, *bval, *bkey2, *bval2, *L0, *seg_start,
       *seg_end, *scan, *radix;
   int32_t* nk;
-  uint8_t* head;
+  uint64_t* head;
   int64_t S;
 };
 
@@ -507,7 +537,7 @@ size_t carve(void* base, int64_t n, int64_t nb, Carve* c) {
   k.scan = (uint32_t*)take(4 * scan_scratch_words());
   k.radix = (uint32_t*)take(4 * radix_sort_scratch_words((uint32_t)nn));
   k.nk = (int32_t*)take(12 * (size_t)nn);
-  k.head = (uint8_t*)take(8 * (size_t)((nn + kWave - 1) / kWave));
+  k.head = (uint64_t*)take(8 * (size_t)((nn + kWave - 1) / kWave));
   if (c) *c = k;
   return off + 256;
 }
@@ -543,13 +573,24 @@ int32_t insert_keys(const BhtView& t, const Keys& keys, int64_t n, int32_t* out,
   for (int64_t S = std::min(c.S, pow2_at_least(2 * (int64_t)t.T));; S = c.S) {
     const bool bounded = S < c.S;
     dedup_clear_kernel<<<groups_n(S), kBT, 0, s>>>(c.skey, c.smin, S, c.total);
-    dedup_insert_kernel<kAll><<<groups_n(n, kBT * kDedupItems), kBT, 0, s>>>(keys, n, c.skey, c.smin, S, bounded,
-                                                                            c.slot_of, c.head, c.total + 1, err);
-    first_kernel<<<groups_n(8 * words), kBT, 0, s>>>(keys, n, 8 * words, c.head, c.slot_of, c.smin,
-                                                    c.total + 1, t, (uint8_t*)c.flag);
+    if (n >= kManyKeys) {
+      dedup_insert_kernel<kAll, 4><<<groups_n(n, kBT * 4), kBT, 0, s>>>(keys, n, words, c.skey, c.smin, S, bounded,
+                                                                        c.slot_of, c.head, c.total + 1, err);
+      first_kernel<8><<<groups_n(n, kBT * 8), kBT, 0, s>>>(keys, words, c.head, c.slot_of, c.smin, c.total + 1, t,
+                                                           (uint64_t*)c.flag);
+    } else {
+      dedup_insert_kernel<kAll, 1><<<groups_n(n), kBT, 0, s>>>(keys, n, words, c.skey, c.smin, S, bounded, c.slot_of,
+                                                               c.head, c.total + 1, err);
+      first_kernel<1><<<groups_n(n), kBT, 0, s>>>(keys, words, c.head, c.slot_of, c.smin, c.total + 1, t,
+                                                  (uint64_t*)c.flag);
+    }
     e = exclusive_scan_popc_u32(c.flag, c.rank, (uint32_t)(2 * words), c.scan, s, c.total);
     if (e != hipSuccess) return ZSMPM_DEVICE_ERROR;
-    compact_kernel<<<groups_n(2 * words), kBT, 0, s>>>(keys, 2 * words, c.flag, c.rank, c.nk, c.level);
+    if (n >= kManyKeys)
+      compact_kernel<8><<<groups_n(n, kBT * 8), kBT, 0, s>>>(keys, words, (const uint64_t*)c.flag, c.rank, c.nk,
+                                                             c.level);
+    else
+      compact_kernel<1><<<groups_n(n), kBT, 0, s>>>(keys, words, (const uint64_t*)c.flag, c.rank, c.nk, c.level);
     loads_kernel<<<groups_n(t.nb), kBT, 0, s>>>(t, c.L0, c.c0);
     if ((e = hipMemcpyAsync(found, c.total, 8, hipMemcpyDeviceToHost, s)) != hipSuccess) return ZSMPM_DEVICE_ERROR;
     if ((e = hipStreamSynchronize(s)) != hipSuccess) return ZSMPM_DEVICE_ERROR;
