@@ -468,25 +468,17 @@ __global__ __launch_bounds__(kBT) void query_kernel(BhtView t, const int32_t* __
   }
 }
 
-// Whole waves, for the shared block queries. What bounded it were those
-// queries, 16 slots of 16 bytes per lane and corner: 99 -> 81 us at 4.2M
-// positions.
+// bound by the block queries (bht_query)
 __global__ __launch_bounds__(kBT) void spg_sample_kernel(SpgView g, int chn, int width, const float* __restrict__ x,
                                                          int64_t n, float* out) {
 #pragma clang fp contract(off)
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t base = blockIdx.x * (int64_t)blockDim.x; base < n; base += stride) {
-    const int64_t i = base + threadIdx.x;
-    const bool live = i < n;
-    float X[3] = {0.f, 0.f, 0.f};
-    if (live) {
-      float p[3];
-      load_row(x, i, p);
-      spg_apply(g.w2i, p[0], p[1], p[2], X);
-    }
-    spg_isample_each<true>(g, chn, width, X, live, [&](int w, float v) {
-      if (live) out[width * i + w] = v;
-    });
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += stride) {
+    float p[3], X[3], v[3];
+    load_row(x, i, p);
+    spg_apply(g.w2i, p[0], p[1], p[2], X);
+    spg_isample_n(g, chn, width, X, v);
+    for (int w = 0; w < width; ++w) out[width * i + w] = v[w];
   }
 }
 

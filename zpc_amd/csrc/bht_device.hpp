@@ -48,15 +48,21 @@ __device__ __forceinline__ int32_t bht_query(const BhtView& t, int32_t k0, int32
   if (t.nb == 0) return -1;
   for (int l = 0; l < 3; ++l) {
     const int32_t off = bht_bucket(t, l, k0, k1, k2) * kBhtBucket;
-    // one bit per match, no branch between the slots: the sixteen loads are in
-    // flight together
-    uint32_t m = 0;
+    // Four slots' first components are in flight together, the others are read
+    // where the first agrees. A bucket fills from its first slot, so most keys
+    // are found in the first four or eight: sampling 525K shuffled positions takes
+    // 25 us, 39 with all sixteen components at once and 48 with all 256 bytes.
+    constexpr int kBatch = 4;
+#pragma clang loop unroll(disable)
+    for (int j0 = 0; j0 < kBhtBucket; j0 += kBatch) {
+      uint32_t m = 0;
 #pragma unroll
-    for (int j = 0; j < kBhtBucket; ++j) {
-      const int4 s = t.keys[off + j];
-      m |= (uint32_t)((s.x == k0) & (s.y == k1) & (s.z == k2)) << j;
+      for (int j = 0; j < kBatch; ++j) m |= (uint32_t)(t.keys[off + j0 + j].x == k0) << j;
+      for (; m; m &= m - 1u) {
+        const int j = off + j0 + __ffs((int)m) - 1;
+        if (t.keys[j].y == k1 && t.keys[j].z == k2) return t.indices[j];
+      }
     }
-    if (m) return t.indices[off + __ffs((int)m) - 1];
   }
   return -1;
 }
@@ -88,74 +94,33 @@ __device__ __forceinline__ float spg_value_or(const SpgView& g, int chn, int32_t
   return g.data[((int64_t)b * g.nch + chn) * 512 + k];
 }
 
-// bht_query of every lane with `need`, the whole wave active: the lanes that
-// share a key take one probe, the wave's first 48 lanes reading the key's
-// three buckets at once. Neighbouring positions share a few blocks; lanes left
-// after kShared distinct keys probe by themselves.
-__device__ __forceinline__ int32_t bht_query_wave(const BhtView& t, int32_t k0, int32_t k1, int32_t k2, bool need) {
-  constexpr int kShared = 4;
-  static_assert(3 * kBhtBucket <= 64, "three buckets per wave");
-  int32_t res = -1;
-  if (t.nb == 0) return res;
-  const int lane = (int)__lane_id();
-  const int level = lane / kBhtBucket, at = lane % kBhtBucket;
-  uint64_t todo = __ballot(need);
-  for (int r = 0; r < kShared && todo != 0; ++r) {
-    const int src = __ffsll((unsigned long long)todo) - 1;
-    const int32_t u0 = __builtin_amdgcn_readlane(k0, src), u1 = __builtin_amdgcn_readlane(k1, src),
-                  u2 = __builtin_amdgcn_readlane(k2, src);
-    const int32_t b0 = bht_bucket(t, 0, u0, u1, u2), b1 = bht_bucket(t, 1, u0, u1, u2),
-                  b2 = bht_bucket(t, 2, u0, u1, u2);
-    const int32_t slot = (level == 0 ? b0 : level == 1 ? b1 : b2) * kBhtBucket + at;
-    bool hit = false;
-    int32_t idx = -1;
-    if (level < 3) {
-      const int4 s = t.keys[slot];
-      idx = t.indices[slot];
-      hit = s.x == u0 && s.y == u1 && s.z == u2;
-    }
-    const uint64_t hits = __ballot(hit);
-    const int32_t found = __builtin_amdgcn_readlane(idx, hits ? __ffsll((unsigned long long)hits) - 1 : 63);
-    const bool same = need && k0 == u0 && k1 == u1 && k2 == u2;
-    res = same ? found : res;
-    todo &= ~__ballot(same);
-  }
-  if ((todo >> lane) & 1ull) res = bht_query(t, k0, k1, k2);
-  return res;
-}
-
 // iSample, kernel_e::linear (GridArena + xlerp): corner = floor(X), the 2^3
 // cell values (background where a block is inactive), lerp a + (b - a) t with
 // x outermost. The eight values share at most eight block queries: a corner
-// takes its neighbour's block along an axis that does not leave it. kShare: the
-// whole wave is active and shares queries (`live`: the lane samples). Channel
-// w's value goes to put(w, value).
-template <bool kShare, typename Put>
-__device__ __forceinline__ void spg_isample_each(const SpgView& g, int chn, int width, const float X[3], bool live,
-                                                 Put put) {
+// takes its neighbour's block along an axis that does not leave it.
+__device__ __forceinline__ void spg_isample_n(const SpgView& g, int chn, int width, const float X[3], float* out) {
 #pragma clang fp contract(off)
   int32_t c[3];
   float t[3];
-  bool cross[3];
+  int cross = 0;  // the axes along which the corners leave the first one's block
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
     c[d] = (int32_t)floorf(X[d]);
     t[d] = X[d] - (float)c[d];
-    cross[d] = (c[d] & 7) == 7;
+    cross |= (c[d] & 7) == 7 ? 4 >> d : 0;
   }
+  // corner i lies in the block of corner i & cross; a loop keeps the query in the
+  // code once
   int32_t blk[8];
 #pragma unroll
+  for (int i = 0; i < 8; ++i) blk[i] = -1;
+#pragma clang loop unroll(disable)
   for (int i = 0; i < 8; ++i) {
-    const bool keep0 = (i & 4) && !cross[0], keep1 = (i & 2) && !cross[1], keep2 = (i & 1) && !cross[2];
-    const bool need = live && !keep0 && !keep1 && !keep2;
-    const int32_t a0 = c[0] + (i >> 2), a1 = c[1] + ((i >> 1) & 1), a2 = c[2] + (i & 1);
+    const int32_t k0 = (c[0] + (i >> 2)) & ~7, k1 = (c[1] + ((i >> 1) & 1)) & ~7, k2 = (c[2] + (i & 1)) & ~7;
     int32_t q = -1;
-    if constexpr (kShare) {
-      if (__ballot(need) != 0) q = bht_query_wave(g.t, a0 & ~7, a1 & ~7, a2 & ~7, need);
-    } else {
-      if (need) q = bht_query(g.t, a0 & ~7, a1 & ~7, a2 & ~7);
-    }
-    blk[i] = keep0 ? blk[i & 3] : keep1 ? blk[i & 5] : keep2 ? blk[i & 6] : q;
+    if ((i & ~cross) == 0) q = bht_query(g.t, k0, k1, k2);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) blk[j] = (j & cross) == i ? q : blk[j];
   }
   for (int w = 0; w < width; ++w) {
     float a[2][2][2];
@@ -174,12 +139,8 @@ __device__ __forceinline__ void spg_isample_each(const SpgView& g, int chn, int 
       const float q = a[i][1][0] + (a[i][1][1] - a[i][1][0]) * t[2];
       yz[i] = p + (q - p) * t[1];
     }
-    put(w, yz[0] + (yz[1] - yz[0]) * t[0]);
+    out[w] = yz[0] + (yz[1] - yz[0]) * t[0];
   }
-}
-
-__device__ __forceinline__ void spg_isample_n(const SpgView& g, int chn, int width, const float X[3], float* out) {
-  spg_isample_each<false>(g, chn, width, X, true, [&](int w, float v) { out[w] = v; });
 }
 
 __device__ __forceinline__ float spg_wsample(const SpgView& g, int chn, float x0, float x1, float x2) {
