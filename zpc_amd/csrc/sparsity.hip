@@ -22,7 +22,7 @@
 // list by first particle and writes the bucket's indices. No sort over the
 // whole set: the counts give the buckets, and a list has ~2 entries when the
 // particles are in bucket order (a few hundred when they are shuffled).
-// The substep's own build (build_begin .. build_place) numbers, places and
+// The substep's own build (build_clear .. build_place) numbers, places and
 // enlarges from one dedup hash and one clear, with no device-wide scan: 9
 // launches where the stage-by-stage operators take about 35.
 #include <hip/hip_runtime.h>
@@ -1188,7 +1188,7 @@ int tile_groups(int64_t n) {
   return wide_tiles(n) && g > 2048 ? 2048 : g;
 }
 
-// the activation's insertion pass
+// the activation's insertion pass (a batch, ss, only in the substep's build, which records the segments)
 template <bool kSegs>
 void launch_activate(Workspace& ws, const float* x, int64_t n, float dx, int blockLen, int offset, float disp,
                      const Segments& sg, hipStream_t s, const SceneSet* ss) {
@@ -1199,11 +1199,16 @@ void launch_activate(Workspace& ws, const float* x, int64_t n, float dx, int blo
   auto launch = [&](auto kernel) {
     kernel<<<g, kThreads, 0, s>>>(x, n, dxinv, blockLen, offset, disp, dedup_of(ws), sg, sset);
   };
-  if (multi && wide_tiles(n))
-    launch(activate_kernel<true, kSegs, kWideTile>);
-  else if (multi)
-    launch(activate_kernel<true, kSegs, kTightTile>);
-  else if (wide_tiles(n))
+  if constexpr (kSegs) {
+    if (multi) {
+      if (wide_tiles(n))
+        launch(activate_kernel<true, true, kWideTile>);
+      else
+        launch(activate_kernel<true, true, kTightTile>);
+      return;
+    }
+  }
+  if (wide_tiles(n))
     launch(activate_kernel<false, kSegs, kWideTile>);
   else
     launch(activate_kernel<false, kSegs, kTightTile>);

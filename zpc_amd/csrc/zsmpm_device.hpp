@@ -584,7 +584,7 @@ struct Model {
 // has no cancellation, so small strains keep their relative accuracy (the SVD
 // forms log sigma from sigma ~ 1: an absolute 1e-7). About 170 operations
 // against 1,240 with the four-sweep SVD; the range is ||Z||_F <= 0.3 (sigma
-// in [0.734, 1.363]), where the first omitted term is below 1e-8.
+// in [0.734, 1.363]), where the first omitted terms are 1e-8.
 struct NearB {
   float A[6], Z[6], Y[6];  // b - I, Z, Z^2 as (xx, yy, zz, xy, xz, yz)
   float i1, i2, i3;        // invariants of Z
