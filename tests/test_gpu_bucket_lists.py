@@ -1,6 +1,6 @@
 """Bucket sort at the edges of its segment lists: particles of two blocks
 interleaved so that each bucket's list has a given number of segments (one
-wave, the LDS sort's powers of two and its limit of 4,096, the radix sort
+wave, the LDS sort's powers of two and its limit of 2,048, the radix sort
 beyond), as short and as long runs, through the stand-alone operator and
 through a substep. Integer results: exact against a stable argsort."""
 import dataclasses
@@ -31,7 +31,9 @@ def _scene(segments, run, tail):
 
 @pytest.mark.parametrize("driver", ["operator", "substep"])
 @pytest.mark.parametrize("segments,run", [(2, 1), (2, 640), (126, 3), (128, 1), (130, 1), (130, 70), (512, 1),
-                                          (8190, 1), (8192, 1), (8194, 1), (8194, 5), (20002, 1)])
+                                          (514, 1), (1026, 8), (2046, 1), (2050, 1), (2050, 8), (4094, 1), (4096, 1),
+                                          (4096, 8), (4098, 1), (4098, 8), (8190, 1), (8192, 1), (8194, 1),
+                                          (8194, 5), (20002, 1)])
 def test_segment_lists_exact(driver, segments, run):
     from zpc_amd import rocm
 

@@ -208,9 +208,9 @@ def test_bucket_sort_shuffled_exact(cube):
 
 @pytest.mark.parametrize("cap_log2", [17, 18])
 def test_bucket_sort_wide_buckets_exact(cube, cap_log2):
-    """Bucket capacities of 2^17 and 2^18 blocks: the runs are radix-sorted
-    in two 9-bit passes (three 8-bit passes below 2^16 keys and above 2^18).
-    Shuffled particles make nearly every particle its own run."""
+    """Bucket capacities of 2^17 and 2^18 blocks, far more than there are blocks:
+    the counts and offsets past them are filled. Shuffled particles make nearly
+    every particle its own run."""
     import torch
 
     rng = np.random.default_rng(23 + cap_log2)
