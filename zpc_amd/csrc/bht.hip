@@ -230,7 +230,7 @@ __global__ __launch_bounds__(kBT) void first_kernel(Keys keys, int64_t words, co
       if ((bits >> lane) & 1ull) {
         int32_t k0, k1, k2;
         keys.get(i0 + (int64_t)r * kWave, k0, k1, k2);
-        is_new = bht_query(t, k0, k1, k2) < 0;
+        is_new = bht_query<kBhtBucket>(t, k0, k1, k2) < 0;
       }
       bits = ballot(is_new);
       if (lane == 0) flag[w0 + r] = bits;

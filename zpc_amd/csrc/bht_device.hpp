@@ -43,26 +43,37 @@ __device__ __forceinline__ int32_t bht_bucket(const BhtView& t, int level, int32
   return (int32_t)(bht_hash(t.h[2 * level], t.h[2 * level + 1], k0, k1, k2) % (uint32_t)t.nb);
 }
 
-// BHTView::query (Bht.hpp:551-580) by one thread: the key's index, or -1
+// The slot of a key among kCount slots of a bucket, or -1: the slots' first
+// components are in flight together, the others are read where the first agrees.
+template <int kCount>
+__device__ __forceinline__ int32_t bht_slots(const BhtView& t, int32_t off, int32_t k0, int32_t k1, int32_t k2) {
+  uint32_t m = 0;
+#pragma unroll
+  for (int j = 0; j < kCount; ++j) m |= (uint32_t)(t.keys[off + j].x == k0) << j;
+  for (; m; m &= m - 1u) {
+    const int j = off + __ffs((int)m) - 1;
+    if (t.keys[j].y == k1 && t.keys[j].z == k2) return j;
+  }
+  return -1;
+}
+
+// BHTView::query (Bht.hpp:551-580) by one thread: the key's index, or -1. A bucket
+// fills from its first slot, so a key that is there is mostly found in the first
+// kFirst = 4: sampling 525K shuffled positions takes 24 us, 39 with all sixteen
+// first components at once and 48 with all 256 bytes. Four at a time to the end
+// made keys that are not there twelve round trips (4.2M positions off the grid
+// 135 -> 110 us with the other twelve at once); the insertion's look-up, whose
+// keys are mostly absent, takes all sixteen in three.
+template <int kFirst = 4>
 __device__ __forceinline__ int32_t bht_query(const BhtView& t, int32_t k0, int32_t k1, int32_t k2) {
   if (t.nb == 0) return -1;
+#pragma clang loop unroll(disable)
   for (int l = 0; l < 3; ++l) {
     const int32_t off = bht_bucket(t, l, k0, k1, k2) * kBhtBucket;
-    // Four slots' first components are in flight together, the others are read
-    // where the first agrees. A bucket fills from its first slot, so most keys
-    // are found in the first four or eight: sampling 525K shuffled positions takes
-    // 25 us, 39 with all sixteen components at once and 48 with all 256 bytes.
-    constexpr int kBatch = 4;
-#pragma clang loop unroll(disable)
-    for (int j0 = 0; j0 < kBhtBucket; j0 += kBatch) {
-      uint32_t m = 0;
-#pragma unroll
-      for (int j = 0; j < kBatch; ++j) m |= (uint32_t)(t.keys[off + j0 + j].x == k0) << j;
-      for (; m; m &= m - 1u) {
-        const int j = off + j0 + __ffs((int)m) - 1;
-        if (t.keys[j].y == k1 && t.keys[j].z == k2) return t.indices[j];
-      }
-    }
+    int32_t s = bht_slots<kFirst>(t, off, k0, k1, k2);
+    if constexpr (kFirst < kBhtBucket)
+      if (s < 0) s = bht_slots<kBhtBucket - kFirst>(t, off + kFirst, k0, k1, k2);
+    if (s >= 0) return t.indices[s];
   }
   return -1;
 }
