@@ -176,11 +176,12 @@ enum zsmpm_stage {
   ZSMPM_STAGE_ACTIVATE = 1,
   ZSMPM_STAGE_ENLARGE = 2,
   ZSMPM_STAGE_BUCKET_SORT = 3,
-  ZSMPM_STAGE_GRID_CLEAR = 4,
+  ZSMPM_STAGE_GRID_CLEAR = 4, /* a substep clears its grid in ENLARGE */
   ZSMPM_STAGE_P2G = 5,
   ZSMPM_STAGE_GRID_UPDATE = 6,
   ZSMPM_STAGE_G2P = 7,
-  ZSMPM_STAGE_STRESS = 8, /* the per-particle constitutive part of P2G */
+  ZSMPM_STAGE_STRESS = 8, /* the per-particle constitutive part of P2G as a pass of its own
+                             (the closure, the FP64 SVD); otherwise in P2G */
   ZSMPM_STAGE_COUNT = 9
 };
 /* policy.profile(bool) (execution/ExecutionPolicy.hpp:105-122; per-launch stream
@@ -307,8 +308,8 @@ int32_t zsmpm_substep_sorted__rocm(zsmpm_policy pol, const zsmpm_model* model, c
  * the result is in b when nsteps is odd (*final_in_b = nsteps & 1); the
  * particle state after every substep is what the single-substep calls
  * produce. With ZSMPM_SUBSTEPS_FUSE_STRESS, G2P also computes the next
- * substep's stress from the F it stores (P2G.hpp:57-100), so the separate
- * per-particle constitutive pass runs once per call. a and b must not overlap.
+ * substep's stress from the F it stores (P2G.hpp:57-100), so P2G forms it only
+ * in the call's first. a and b must not overlap.
  * With ZSMPM_SUBSTEPS_GRAPH (not combinable with FUSE_STRESS), the pair of
  * substeps a -> b -> a is captured once into a hipGraph (zpc launches every
  * kernel separately; graph replay has no counterpart there) and replayed
