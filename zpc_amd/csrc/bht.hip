@@ -209,8 +209,8 @@ __global__ __launch_bounds__(kBT) void first_kernel(Keys keys, int64_t words, co
   const int lane = lane_id();
   const bool complete = *full == 0u;
   const int64_t nwaves = (int64_t)gridDim.x * (kBT / kWave);
-  for (int64_t w0 = (blockIdx.x * (int64_t)(kBT / kWave) + uniform((int32_t)(threadIdx.x / kWave))) * kWords; w0 < words;
-       w0 += nwaves * kWords) {
+  const int64_t wave = blockIdx.x * (int64_t)(kBT / kWave) + uniform((int32_t)(threadIdx.x / kWave));
+  for (int64_t w0 = wave * kWords; w0 < words; w0 += nwaves * kWords) {
     const int64_t i0 = w0 * kWave + lane;
     uint32_t s[kWords];
     uint64_t cand[kWords];
@@ -246,8 +246,8 @@ __global__ __launch_bounds__(kBT) void compact_kernel(Keys keys, int64_t words, 
                                                       uint32_t* level) {
   const int lane = lane_id();
   const int64_t nwaves = (int64_t)gridDim.x * (kBT / kWave);
-  for (int64_t w0 = (blockIdx.x * (int64_t)(kBT / kWave) + uniform((int32_t)(threadIdx.x / kWave))) * kWords; w0 < words;
-       w0 += nwaves * kWords) {
+  const int64_t wave = blockIdx.x * (int64_t)(kBT / kWave) + uniform((int32_t)(threadIdx.x / kWave));
+  for (int64_t w0 = wave * kWords; w0 < words; w0 += nwaves * kWords) {
     uint64_t bits[kWords];
 #pragma unroll
     for (int r = 0; r < kWords; ++r) bits[r] = w0 + r < words ? flag[w0 + r] : 0ull;

@@ -77,8 +77,9 @@ constexpr int kP2GWaves = kP2GThreads / kWave;
 // in about one round each, no serial chain of three). At 128 registers two such
 // workgroups fit a CU, so it pays while every bucket is resident at once, up to
 // 512: substep 67.1 -> 64.7 us at 4K particles, 70.9 -> 68.9 at 64K, 88.3 -> 82.3
-// at 128K of 16 per cell, 224 -> 170 at 262K of 64; past the line 89.4 -> 101 at
-// 64K of 1 per cell (1,331 buckets). Nine waves at 144 registers, one workgroup
+// at 128K of 16 per cell, 224 -> 170 at 262K of 64 (73.8 -> 74.0 at 97K and 74.2 ->
+// 75.0 at 120K of 8, some 350 buckets); past the line 89.4 -> 101 at 64K of 1 per
+// cell (1,331 buckets). Nine waves at 144 registers, one workgroup
 // per CU, cost more from 256 buckets on (72.5 -> 76.2 at 72K). Splitting a bucket
 // over four workgroups instead gained 3 us at 4K and lost 15 at 64K.
 constexpr int kP2GWideBuckets = 1024;
@@ -295,8 +296,9 @@ __global__ __launch_bounds__(kThreads) void stress_kernel(Model m, ParticlesView
 // (cell_w) in place of the quadratic B-spline, with C and the stress scaled
 // per column by the cell kernel's Dinv.
 template <int kMode, bool kMulti, bool kCell = false, int kTile = 0>
-__global__ __launch_bounds__(p2g_threads(kTile), kTile == kWideTile ? 4 : 3) void p2g_kernel(ParticlesView ps, const float* __restrict__ contrib,
-                                                       StressFrom st,
+__global__ __launch_bounds__(p2g_threads(kTile),
+                             kTile == kWideTile ? 4 : 3) void p2g_kernel(ParticlesView ps,
+                                                       const float* __restrict__ contrib, StressFrom st,
                                                        TableView t, SortView sv, const int32_t* __restrict__ nbr_tab,
                                                        float* __restrict__ grid, int32_t grid_cap, float dt,
                                                        float dx, uint32_t* err, SceneSet ss, int32_t fch) {
